@@ -447,8 +447,8 @@ wt_status wt_fit_synthesize(wt_ctx* ctx, const wt_fit_problem* problem, float si
                             void* stream);
 /* Phase-storage policy of the adjoint: the bytes a stored (cos, sin) tensor of
  * S x n^2 x W would take, and whether the kernels recompute the phases instead
- * (always 1 in this build: recomputing by rotation is cheaper than the HBM round
- * trip at every size). */
+ * (always 1 in this build: the kernels contract separable factors of the
+ * phases, which is cheaper than an HBM round trip at every size). */
 wt_status wt_fit_phase_plan(const wt_fit_problem* problem, uint64_t budget_bytes, uint64_t* phase_tensor_bytes,
                             int* recompute);
 

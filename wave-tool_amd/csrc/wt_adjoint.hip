@@ -6,27 +6,49 @@
 // d = (Q A Dx cos theta, A sin theta, Q A Dz cos theta) (water-grid.vert:79-81).
 // Loss = 1 / (2 S V) * sum over snapshots and grid points of |d - target|^2.
 //
-// adjoint_kernel<SMAX, KP>: KP grid points per thread (256 KP per block), all S <= SMAX
-//   snapshots of each in registers; one instantiation per snapshot class (SMAX = 4, 8,
-//   ..., 32), so a batch of mixed problems runs one launch per class present.
-//   forward: per wave, seed (cos, sin) from the FP64-reduced phase at t0 and step the
-//     snapshots with the three-term recurrence (or, for |sin(omega dt)| < 0.25, a
-//     rotation by omega dt); accumulate d per snapshot.
-//   residual r = d - target, loss contribution 1/2 |r|^2.
-//   backward: per wave, re-seed and step again (recomputing the phases is cheaper than
-//     storing them: 4 VALU ops per snapshot against an 8-byte HBM round trip), with six
-//     running sums over snapshots plus three running sums of those sums (the
-//     time-weighted sums follow by summation by parts: sum_s s f_s = S U - V), from
-//     which the five parameter derivatives of each grid point follow; the thread's KP
-//     points are added, then a fixed-order wavefront reduction (DPP row sums, lane
-//     swaps across rows), a fixed-order sum over the 4 wavefronts, and one partial per
-//     (parameter, block) in global memory.
+// On a regular grid exp(i theta) splits into a column factor and a (row, snapshot) factor
+// P = exp(i (kx x_mid + kz z_j + omega t_s + phi0)), x_mid the centre of a strip of 64
+// columns. The columns pair up about the centre at the offsets +-delta, so the column
+// factors are the real cos(kx delta) and sin(kx delta) of 32 offsets, and both passes are
+// contractions for the matrix cores over the even and the odd part of what they act on:
+//   forward   (d+ + d-) / 2 [delta, (j,s)] = sum over waves of cos(kx delta) x B, and
+//             (d+ - d-) / 2 the same with sin and B', B and B' the coefficients times P;
+//   backward  G[wave, (j,s)] = sum over offsets of cos(kx delta) x (r+ + r-) and of
+//             sin(kx delta) x (r+ - r-), and the same weighted with the offset, from which
+//             P gives every wave's sums of r cos theta and r sin theta.
+// Folding halves the products of the plain split into 64 columns (fit_batch of 256 uneven
+// problems on one MI355X: 1.3 ms an iteration against 1.5 ms).
+// adjoint_kernel: a workgroup takes one strip and a run of (row, snapshot) pairs q = j S + s,
+//   16 consecutive pairs (a tile) per wavefront at a time, so any snapshot count packs the
+//   tiles without padding. The column factors sit in LDS as matrix fragments, built once
+//   per workgroup; per tile a wavefront forms P and B in registers, contracts the forward
+//   pass onto the negated targets, and contracts the backward pass with the residuals still
+//   in the registers the forward pass left them in (the offset order of the backward
+//   fragments is the accumulators' order). Chunks of 16 waves are looped over, not
+//   unrolled: one body serves every wave count and stays in the instruction cache.
+// Operands are FP32 values split into two FP16 halves, v = hi + lo with hi = fp16(v)
+//   and lo = fp16(v - hi), multiplied as hi hi + hi lo + lo hi with FP32 accumulation
+//   (about 2^-22 per product). Powers of two keep both halves in FP16's range: the column
+//   factors are scaled by 2^4, the coefficients by their largest magnitude in the problem,
+//   and the residuals by the largest of the wavefront's tile where that leaves the range.
+//   Against the FP64 adjoint the gradients of 2- to 32-snapshot problems are as close or
+//   closer than with FP32 recurrences over the snapshots (rms of the relative error over 16
+//   problems: 200^2 x 2 x 64 1.1e-7 against 1.1e-7, 128^2 x 16 x 32 1.0e-7 against 8.6e-7).
+// What bounds it: VALU issue and the matrix cores together, which do not overlap on one
+//   SIMD (two wavefronts of one SIMD, one issuing only matrix instructions and one only
+//   FMAs, take the sum of their times): per tile of 64 waves about 1300 VALU instructions
+//   and 216 matrix instructions of 16 cycles. 512^2 x 16 x 32: 18 us (62 us with FP32
+//   recurrences over the snapshots on the VALU); the 256-problem batch 1.25 ms (3.6 ms).
+//   Two wavefronts per SIMD at up to 256 VGPRs: a 32-column strip at three or four
+//   wavefronts repeats P, B and the sums per point (1.7 ms), and a spilled register is a
+//   round trip to cold scratch memory (5 us per workgroup).
 // reduce_adam_kernel: one workgroup per (problem, parameter row): fixed-order sum of
 //   the block partials, scaling to the mean misfit, and either an Adam step on the
 //   parameter or a plain gradient / loss write-out.
 // Both kernels find their problem through a block (row) -> problem map built at
-// creation, so one launch per snapshot class covers a whole batch; a single problem is a
-// table of one.
+// creation, so one launch per wave-count class covers a whole batch; a single problem is
+// a table of one. A problem's blocks and the order of every sum depend on the problem
+// alone, so a batch repeats the bits of its problems run one by one.
 #include <hip/hip_runtime.h>
 
 #include <utility>
@@ -35,24 +57,18 @@
 
 namespace wt {
 
-struct FitWaveLds {
-  double kx, kz, c0;   // revolutions per metre along x / z, phase at t0 (fract)
-  double om_rev;       // omega / 2 pi, revolutions per second
-  float qadx, qadz, A, Q, Dx, Dz;
-  float rc, rs;        // rotation by omega dt
-  float tc;            // 2 cos(omega dt), the three-term recurrence's coefficient
-  int orig;            // the wave's index in the problem (its gradient rows)
-  float w, wL, om2L;   // w, w / L, omega / (2 L)
-  float qdx, qdz;      // Q Dx, Q Dz
-  float od, op;        // D . (x0, z0) and D-perp . (x0, z0), the grid origin's terms
-};
+typedef _Float16 Half2 __attribute__((ext_vector_type(2)));
+typedef _Float16 Half8 __attribute__((ext_vector_type(8)));
+typedef float Float4 __attribute__((ext_vector_type(4)));
 
-// The three-term recurrence x[s+1] = 2 cos(d) x[s] - x[s-1] steps (cos, sin) with one FMA
-// per value instead of the rotation's two. Its FP32 errors grow by at most 1 / |sin d|
-// per step and the rounding of 2 cos d shifts the step by at most 1.2e-7 / (2 |sin d|),
-// so with |sin d| >= 0.25 and at most 32 snapshots the phases stay within 1e-5 rad;
-// waves with a smaller |sin d| keep the rotation.
-constexpr double kFitChebMinSin = 0.25;
+// A wave's constants in the tile loop (zero for the padding up to a multiple of 16).
+struct FitWaveLds {
+  double kx, kz, c0, om;  // revolutions per metre along x and z, phase at t0 (fract), revolutions per second
+};
+// And those that turn its sums into parameter derivatives.
+struct FitWaveGrad {
+  float A, Q, Dx, Dz, w, wL, om2L;  // wL = w / L, om2L = omega / (2 L)
+};
 
 // Sum over the 64 lanes of a wavefront with DPP moves (VALU only, fixed order); the
 // total lands in lane 63. quad_perm [1,0,3,2] and [2,3,0,1] give quad sums,
@@ -61,18 +77,7 @@ template <int CTRL, int ROW_MASK>
 __device__ __forceinline__ float dpp_term(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROW_MASK, 0xf, false));
 }
-__device__ __forceinline__ float wave_sum63(float v) {
-  v += dpp_term<0xB1, 0xf>(v);
-  v += dpp_term<0x4E, 0xf>(v);
-  v += dpp_term<0x141, 0xf>(v);
-  v += dpp_term<0x140, 0xf>(v);
-  v += dpp_term<0x142, 0xa>(v);
-  v += dpp_term<0x143, 0xc>(v);
-  return v;
-}
-
-// The sum over each row of 16 lanes, in every lane of the row (the first four steps of
-// wave_sum63).
+// The sum over each row of 16 lanes, in every lane of the row.
 __device__ __forceinline__ float row_sum(float v) {
   v += dpp_term<0xB1, 0xf>(v);
   v += dpp_term<0x4E, 0xf>(v);
@@ -80,14 +85,17 @@ __device__ __forceinline__ float row_sum(float v) {
   v += dpp_term<0x140, 0xf>(v);
   return v;
 }
-
+__device__ __forceinline__ float wave_sum63(float v) {
+  v = row_sum(v);
+  v += dpp_term<0x142, 0xa>(v);
+  v += dpp_term<0x143, 0xc>(v);
+  return v;
+}
 // gfx950's lane swaps between two registers, summed lane by lane. With rows r0..r3 of
 // 16 lanes,
 //   swap32_sum(x, y) = [x.r0 + x.r2, x.r1 + x.r3, y.r0 + y.r2, y.r1 + y.r3],
-//   swap16_sum(x, y) = [x.r0 + x.r1, y.r0 + y.r1, x.r2 + x.r3, y.r2 + y.r3].
-// Each step sums two values over half their lanes at once, so four values reduce over
-// the wavefront in two swap32 sums, one swap16 sum and one row sum of the packed result
-// (10 instructions, against 22 with a row sum per value first).
+//   swap16_sum(x, y) = [x.r0 + x.r1, y.r0 + y.r1, x.r2 + x.r3, y.r2 + y.r3],
+// so four values are summed over the rows in two swap32 sums and one swap16 sum.
 __device__ __forceinline__ float swap32_sum(float x, float y) {
   const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
   return __uint_as_float(p[0]) + __uint_as_float(p[1]);
@@ -96,345 +104,646 @@ __device__ __forceinline__ float swap16_sum(float x, float y) {
   const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
   return __uint_as_float(p[0]) + __uint_as_float(p[1]);
 }
-
-// The snapshot step omega dt of wave i in radians, reduced to [0, 2 pi).
-__device__ __forceinline__ double fit_wave_step(const FitDesc& P, int i) {
-  const float* pr = P.params + 5 * i;
-  const double L = pr[1] > 1e-3f ? pr[1] : 1e-3f;
-  const double om = sqrt(P.g * (kTwoPi / L));
-  const double step = om * P.dt * kInvTwoPi;
-  return (step - floor(step)) * kTwoPi;
+// The maximum of a non-negative value over the wavefront, wave-uniform.
+__device__ __forceinline__ float wave_max(float v) {
+  v = fmaxf(v, dpp_term<0xB1, 0xf>(v));
+  v = fmaxf(v, dpp_term<0x4E, 0xf>(v));
+  v = fmaxf(v, dpp_term<0x141, 0xf>(v));
+  v = fmaxf(v, dpp_term<0x140, 0xf>(v));
+  v = fmaxf(v, dpp_term<0x142, 0xa>(v));
+  v = fmaxf(v, dpp_term<0x143, 0xc>(v));
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
-// One wave's constants as the kernels stage them, and whether it takes the three-term
-// recurrence (|sin omega dt| >= kFitChebMinSin).
-__device__ __forceinline__ FitWaveLds fit_wave_constants(const FitDesc& P, int i, bool* cheb) {
-  const float* pr = P.params + 5 * i;
-  const double A = pr[0], L = pr[1] > 1e-3f ? pr[1] : 1e-3f, al = pr[2], Q = pr[3], ph0 = pr[4];
-  const double w = kTwoPi / L, om = sqrt(P.g * w);
-  double sa, ca;
-  sincos(al, &sa, &ca);
-  FitWaveLds o;
-  o.kx = w * ca * kInvTwoPi;
-  o.kz = w * sa * kInvTwoPi;
-  const double ph = (om * P.t0 + ph0) * kInvTwoPi;
-  o.c0 = ph - floor(ph);
-  o.om_rev = om * kInvTwoPi;
-  double sn, cs;
-  sincos(fit_wave_step(P, i), &sn, &cs);
-  *cheb = fabs(sn) >= kFitChebMinSin;
-  o.rc = (float)cs;
-  o.rs = (float)sn;
-  o.tc = (float)(2.0 * cs);
-  o.orig = i;
-  o.A = (float)A;
-  o.Q = (float)Q;
-  o.Dx = (float)ca;
-  o.Dz = (float)sa;
-  o.qadx = (float)(Q * A * ca);
-  o.qadz = (float)(Q * A * sa);
-  o.w = (float)w;
-  o.wL = (float)(w / L);
-  o.om2L = (float)(om / (2.0 * L));
-  o.qdx = (float)(Q * ca);
-  o.qdz = (float)(Q * sa);
-  o.od = (float)(ca * P.x0 + sa * P.z0);
-  o.op = (float)(ca * P.z0 - sa * P.x0);
-  return o;
+// The power of two that takes magnitude m (>= 0) to [2^3, 2^4), as an exponent; clamped
+// for m zero, denormal, infinite or NaN so that it, its inverse and (up to 2^60) what is
+// multiplied by it stay floats.
+__device__ __forceinline__ int scale_exponent(float m) {
+  const int e = (int)((__float_as_uint(m) >> 23) & 0xffu) - 127;
+  return min(max(3 - e, -110), 60);
+}
+__device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t)(127 + e) << 23); }
+
+// (a, b) as packed halves: hi = fp16, lo = fp16 of the rest (exact in FP32). The empty
+// asm statements keep the remainder a fused a - hi from the packed word, which converts on
+// the way in and out (v_fma_mixlo_f16 / v_fma_mixhi_f16: three instructions per pair).
+__device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
+  const Half2 h = {(_Float16)a, (_Float16)b};
+  hi = __builtin_bit_cast(uint32_t, h);
+  asm("" : "+v"(hi));
+  float minus = -1.0f;
+  asm("" : "+s"(minus));
+  const Half2 g = __builtin_bit_cast(Half2, hi);
+  const Half2 l = {(_Float16)fmaf((float)g.x, minus, a), (_Float16)fmaf((float)g.y, minus, b)};
+  lo = __builtin_bit_cast(uint32_t, l);
 }
 
-__device__ __forceinline__ void stage_fit_wave(const FitDesc& P, int i, FitWaveLds* o) {
-  bool cheb;
-  *o = fit_wave_constants(P, i, &cheb);
+union Frag {  // one lane's 8 halves of a 16x16x32 operand
+  uint32_t w[4];
+  Half8 h;
+};
+
+__device__ __forceinline__ Float4 mma(const Half8& a, const Half8& b, const Float4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
-// (c, sn) <- the next snapshot's (cos, sin). Rotation form: by omega dt. Three-term form:
-// a rotation from snapshot 0, which also sets the previous values (cp, sp), then
-// x[s+1] = 2 cos(omega dt) x[s] - x[s-1].
-template <bool kCheb>
-__device__ __forceinline__ void step_snapshot(int s, float& c, float& sn, float& cp, float& sp, const FitWaveLds& wv) {
-  float cn, snn;
-  if (!kCheb || s == 0) {
-    cn = fmaf(sn, -wv.rs, c * wv.rc);
-    snn = fmaf(c, wv.rs, sn * wv.rc);
+// One column factor (hi, lo) contracted with the three components of a residual part.
+__device__ __forceinline__ void column_sums(const Half8& eh, const Half8& el, const Frag (&rh)[3], const Frag (&rl)[3],
+                                            Float4 (&o)[3]) {
+#pragma unroll
+  for (int c = 0; c < 3; ++c) o[c] = mma(rh[c].h, eh, o[c]);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) o[c] = mma(rl[c].h, eh, o[c]);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) o[c] = mma(rh[c].h, el, o[c]);
+}
+
+// Consecutive floats at 4-byte alignment.
+struct __attribute__((packed, aligned(4))) Target4 {
+  float v[4];
+};
+struct __attribute__((packed, aligned(4))) Target3 {
+  float v[3];
+};
+
+// cos and sin of 2 pi f for an FP64 phase f in revolutions: reduced in FP64 to r in
+// [-1/8, 1/8] of a quarter turn's centre, then interpolating polynomials in r^2 through
+// the Chebyshev nodes of [0, 1/64] (truncation below 1e-8), signs and order by quadrant.
+// Worst error 9e-8, rms 2e-8, against 2e-7 and about 1e-7 for v_sin_f32 / v_cos_f32 with
+// the argument's rounding corrected: one factor serves a whole row or column of products
+// here, so its error does not average out, and with the hardware functions the gradients
+// of few-snapshot problems were up to 1.6 times further from the FP64 adjoint.
+__device__ __forceinline__ void sincos_turn(double f, float* c, float* s) {
+  f = __builtin_amdgcn_fract(f);
+  const double k = rint(4.0 * f);
+  const float r = (float)fma(-0.25, k, f), u = r * r;
+  const int quad = (int)k;
+  const float sp = r * fmaf(fmaf(fmaf(-75.4016127f, u, 81.5925429f), u, -41.3416626f), u, 6.28318529f);
+  const float cp = fmaf(fmaf(fmaf(fmaf(59.2201690f, u, -85.4428447f), u, 64.9393161f), u, -19.7392087f), u, 1.0f);
+  const bool odd = quad & 1;
+  const float sv = odd ? cp : sp, cv = odd ? sp : cp;
+  *s = __uint_as_float(__float_as_uint(sv) ^ ((uint32_t)(quad & 2) << 30));
+  *c = __uint_as_float(__float_as_uint(cv) ^ ((uint32_t)((quad + 1) & 2) << 30));
+}
+
+// Orders this wavefront's LDS accesses around it: its lanes read what other lanes of it
+// wrote (LDS operations of one wavefront complete in order, so no wait is needed).
+__device__ __forceinline__ void wavefront_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+constexpr float kFitTrigScale = 16.0f;  // scale of E in its fragments
+// The largest scaled residual a tile is split at without rescaling: the halves stay finite
+// (2^15 below FP16's largest) and the low halves' FP16 spacing, 2^-24, stays below 2^-24 of
+// the largest.
+constexpr float kFitResLow = 1.0f, kFitResHigh = 32768.0f;
+
+constexpr int kRunFloats = 52;  // a run of 48 target floats, padded: rows of eight pairs on different banks
+
+// The workgroup's LDS for up to KMAX chunks of 16 waves (`chunks` of them in use).
+//  fwd, bwd: the column factors cos(kx delta), sin(kx delta) of the 32 column offsets
+//    delta = (t + 1/2) spacing as matrix operands. Two chunks make the forward pass's inner
+//    dimension of 32 (hi, then lo); a last odd chunk takes it as [hi | lo] of its 16 waves.
+//    fwd [16 offsets][cos / sin][chunk][lane], bwd [chunk][cos / sin][plain / times
+//    t + 1/2][hi / lo][lane].
+//  sums: per wavefront, chunk and lane two of the part's running sums of wave lane mod 16.
+//  time: exp(i omega s dt), [snapshot][wave] (cos, sin), then a row of zeros for the pairs
+//    past the last; rows padded by 16 bytes to keep the 16-byte reads of eight neighbouring
+//    rows on different banks.
+//  row: per wavefront the factors exp(i (kx x + kz z_j + phase at t0)) at the strip's centre
+//    of a tile's four rows, [row][wave] (cos, sin).
+//  run: per wavefront one run of 16 columns' targets of 16 pairs, on the way to its lanes.
+template <int KMAX, int NW, bool kTable>
+struct FitShared {
+  float4 coef[16 * KMAX];  // Q A Dx, A, Q A Dz, scaled by the problem's power of two
+  float2 dir[16 * KMAX];   // Q Dx, Q Dz
+  FitWaveLds wave[16 * KMAX];
+  FitWaveGrad grad[16 * KMAX];
+  uint32_t max;  // bits of the largest coefficient magnitude
+  float loss[NW];
+  alignas(16) float row[NW][kTable ? 4 * 32 * KMAX : 4];
+  alignas(16) float time[kTable ? (kFitMaxSnapshots + 1) * (32 * KMAX + 4) : 4];
+  float2 sums[NW][KMAX][64];
+  alignas(16) float run[NW][kTable ? 16 * kRunFloats : 4];
+  Half8 fwd[2 * 2 * KMAX * 64];
+  Half8 bwd[KMAX * 2 * 2 * 2 * 64];
+  __device__ __forceinline__ Half8* fwd_at(int chunks, int mt, int o, int k) { return fwd + ((mt * 2 + o) * chunks + k) * 64; }
+  __device__ __forceinline__ Half8* bwd_at(int kc, int o, int m, int h) { return bwd + (((kc * 2 + o) * 2 + m) * 2 + h) * 64; }
+};
+
+constexpr int kStrip = 64, kHalf = 32;  // a strip's columns, and the offsets they pair up at
+
+// The targets of one (row, snapshot) pair, twelve floats each of the columns 32 + t .. and
+// 31 - t .. of the strip, t = 16 mt + 4 g + 0 .. 3 (up, dn). Columns past the grid and
+// pairs past the last give zero. `whole` (the strip and the tile lie inside,
+// wave-uniform): the four lanes of a pair together read each 192-byte run of 16 columns,
+// 64 consecutive bytes per instruction, and unshuffle() hands every lane its own columns
+// (a lane's 48 bytes read directly made every load instruction 64 cache accesses, 60% of
+// the time of a tile of 32 waves).
+__device__ __forceinline__ void load_targets(const FitDesc& P, bool whole, bool valid, uint32_t j, uint32_t sn,
+                                             int col0, int g, float (&up)[2][12], float (&dn)[2][12]) {
+  const float* tp = P.target + (size_t)sn * (3 * (size_t)P.n * (size_t)P.n) +
+                    3 * ((size_t)j * (size_t)P.n + (size_t)(col0 + kHalf));
+  if (whole) {
+    const float* tl = tp + 4 * g;
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const Target4 a = *reinterpret_cast<const Target4*>(tl + 48 * mt + 16 * k);
+        const Target4 b = *reinterpret_cast<const Target4*>(tl - 48 * (mt + 1) + 16 * k);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          up[mt][4 * k + i] = a.v[i];
+          dn[mt][4 * k + i] = b.v[i];
+        }
+      }
   } else {
-    cn = fmaf(wv.tc, c, -cp);
-    snn = fmaf(wv.tc, sn, -sp);
-  }
-  if (kCheb) {
-    cp = c;
-    sp = sn;
-  }
-  c = cn;
-  sn = snn;
-}
-
-// (cos, sin) of a wave's phase at the thread's points at t0: FP64 reduction to
-// revolutions, then the hardware sine and cosine (which take revolutions).
-template <int KP>
-__device__ __forceinline__ void wave_seeds(const FitWaveLds& wv, const double (&x)[KP], const double (&z)[KP],
-                                           float (&c)[KP], float (&sn)[KP]) {
+    // columns clamped to the row, and what lies outside taken times zero (a select on a
+    // loaded value would become a branch around every load)
+    int last = P.n - 1 - (col0 + kHalf);  // the row's last column, from the strip's centre
+    asm volatile("" : "+s"(last));  // keeps the clamped addresses out of the tile loop's live registers
 #pragma unroll
-  for (int k = 0; k < KP; ++k) {
-    const float ph = (float)__builtin_amdgcn_fract(fma(wv.kx, x[k], fma(wv.kz, z[k], wv.c0)));
-    c[k] = __builtin_amdgcn_cosf(ph);
-    sn[k] = __builtin_amdgcn_sinf(ph);
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int iu = 16 * mt + 4 * g + r, id = -(16 * mt + 4 * g + 4) + r;
+        const float mu = valid && iu <= last ? 1.0f : 0.0f, md = valid && id <= last ? 1.0f : 0.0f;
+        const Target3 a = *reinterpret_cast<const Target3*>(tp + 3 * min(iu, last));
+        const Target3 b = *reinterpret_cast<const Target3*>(tp + 3 * min(id, last));
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          up[mt][3 * r + c] = mu * a.v[c];
+          dn[mt][3 * r + c] = md * b.v[c];
+        }
+      }
   }
 }
 
-// Forward of one wave at the thread's points, from its seeds: add its displacement to
-// every snapshot.
-template <int SMAX, int KP, bool kCheb>
-__device__ __forceinline__ void forward_wave(const FitWaveLds& wv, const float (&c0)[KP], const float (&s0)[KP],
-                                             float (&r)[KP][SMAX][3]) {
+// One run through the wavefront's LDS buffer: from 64-byte pieces of every pair to lane
+// g's twelve floats at 12 * column group `at`.
+__device__ __forceinline__ void unshuffle(float* run, int n16, int g, int at, float (&v)[12]) {
+  float4* w = reinterpret_cast<float4*>(run + n16 * kRunFloats);
 #pragma unroll
-  for (int k = 0; k < KP; ++k) {
-    float c = c0[k], sn = s0[k], cp = 0.0f, sp = 0.0f;
+  for (int k = 0; k < 3; ++k) w[4 * k + g] = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+  wavefront_lds_sync();
 #pragma unroll
-    for (int s = 0; s < SMAX; ++s) {
-      r[k][s][0] = fmaf(wv.qadx, c, r[k][s][0]);
-      r[k][s][1] = fmaf(wv.A, sn, r[k][s][1]);
-      r[k][s][2] = fmaf(wv.qadz, c, r[k][s][2]);
-      step_snapshot<kCheb>(s, c, sn, cp, sp, wv);
+  for (int k = 0; k < 3; ++k) {
+    const float4 t = w[3 * at + k];
+    v[4 * k] = t.x;
+    v[4 * k + 1] = t.y;
+    v[4 * k + 2] = t.z;
+    v[4 * k + 3] = t.w;
+  }
+  wavefront_lds_sync();
+}
+
+// A unit's tiles and the sums of its parts. Lane (n16, g) works in the forward pass on
+// pair n16, the column offsets t = 16 mt + 4 g + r and the waves 4 g + u of a chunk; after the
+// backward contraction on wave n16 of a chunk and the pairs 4 g + r. kTable: P from the
+// time table and the tile's row factors, else a sine and cosine per pair and wave.
+template <bool kByTable, int KMAX, int NW, bool kTable>
+__device__ __forceinline__ void fit_tiles(const FitDesc& P, const FitUnit& unit, FitShared<KMAX, NW, kTable>& sh,
+                                          int chunks, int coef_exp) {
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n16 = lane & 15, g = lane >> 4;
+  const int time_row = 32 * chunks + 4;
+  float* const s_row = sh.row[wid];
+  // the last strip ends with the row (from 64 columns on), its columns that belong to the
+  // strip before it left out
+  const int lo_col = unit.strip * kStrip, col0 = max(0, min(lo_col, P.n - kStrip));
+  const uint32_t pairs = (uint32_t)P.n * (uint32_t)P.S;  // n <= 8192, S <= 32
+  // q / S by a multiply-high: exact for q < 2^18, S <= 32
+  const uint32_t magic = 0xffffffffu / (uint32_t)P.S + 1u;
+  const bool one = P.S == 1;
+  auto row_of = [&](uint32_t q) { return one ? q : __umulhi(q, magic); };
+  const int tiles = (int)((pairs + 15) >> 4);
+  const int first = unit.part * P.tiles_per_block;
+  const int end = min(tiles, first + unit.parts * P.tiles_per_block);
+  const bool inside = P.n >= kStrip, full_strip = lo_col + kStrip <= P.n;
+  const float fwd_scale = pow2f(coef_exp) * kFitTrigScale;
+  const float inv_fwd = pow2f(-coef_exp) * (1.0f / kFitTrigScale), neg_half = -0.5f * fwd_scale;
+  const double x_mid = P.x0 + ((double)col0 + 31.5) * P.spacing;  // the strip's centre
+
+  for (int kc = 0; kc < chunks; ++kc) sh.sums[wid][kc][lane] = make_float2(0.0f, 0.0f);
+  float sq = 0.0f;
+
+
+  int part = unit.part, part_end = first + P.tiles_per_block;
+#pragma unroll 1
+  for (int base = first; base < end; base += NW) {
+    const int tile = base + wid;
+    if (tile < end) {
+      const uint32_t q = (uint32_t)tile * 16u + (uint32_t)n16;
+      const bool valid = q < pairs;
+      const uint32_t qc = valid ? q : pairs - 1u;
+      const uint32_t j = row_of(qc), sn = qc - j * (uint32_t)P.S;
+      const uint32_t j0 = row_of((uint32_t)tile * 16u);  // the tile's first row
+      const bool whole = kTable && inside && (uint32_t)tile * 16u + 16u <= pairs;
+      float up[2][12], dn[2][12];
+      load_targets(P, whole, valid, j, sn, col0, g, up, dn);
+      if constexpr (kByTable) {
+#pragma unroll 1
+        for (int kc = 0; kc < chunks; ++kc) {
+          const FitWaveLds& w = sh.wave[16 * kc + n16];
+          float cv, sv;
+          sincos_turn(fma(w.kz, P.z0 + (double)(j0 + (uint32_t)g) * P.spacing, fma(w.kx, x_mid, w.c0)), &cv, &sv);
+          *reinterpret_cast<float2*>(&s_row[(g * chunks + kc) * 32 + 2 * n16]) = make_float2(cv, sv);
+        }
+        wavefront_lds_sync();
+      }
+
+      if (whole) {
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+          unshuffle(sh.run[wid], n16, g, g, up[mt]);
+          unshuffle(sh.run[wid], n16, g, 3 - g, dn[mt]);
+        }
+      }
+      // forward, onto the negated folded targets in the contraction's units
+      Float4 d[2][2][3];  // [16 offsets][even / odd][x, y, z]
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float a = up[mt][3 * r + c] * neg_half, b = dn[mt][3 * (3 - r) + c];
+            d[mt][0][c][r] = fmaf(b, neg_half, a);
+            d[mt][1][c][r] = fmaf(b, -neg_half, a);
+          }
+      // the pairs past the last take the table's zero row (or zeros) for P
+      const float* trow = sh.time + (valid ? sn : (uint32_t)P.S) * (uint32_t)time_row + 8 * g;
+      const float* rrow = s_row + (j - j0) * (uint32_t)(32 * chunks) + 8 * g;
+      const double zj = P.z0 + (double)j * P.spacing, ts = (double)sn * P.dt;
+      const float live = valid ? 1.0f : 0.0f;
+      // P of a chunk times the coefficients, split: words [at, at + 2) of the operands
+      auto coefficients = [&](int kc, int at, Frag(&bh)[2][3], Frag(&bl)[2][3]) {
+        float pc[4], ps[4];
+        if constexpr (kByTable) {
+          const float4* rp = reinterpret_cast<const float4*>(rrow + 32 * kc);
+          const float4* qp = reinterpret_cast<const float4*>(trow + 32 * kc);
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const float4 a = rp[h], t = qp[h];
+            pc[2 * h] = fmaf(a.x, t.x, -(a.y * t.y));
+            ps[2 * h] = fmaf(a.x, t.y, a.y * t.x);
+            pc[2 * h + 1] = fmaf(a.z, t.z, -(a.w * t.w));
+            ps[2 * h + 1] = fmaf(a.z, t.w, a.w * t.z);
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const FitWaveLds& w = sh.wave[16 * kc + 4 * g + u];
+            sincos_turn(fma(w.om, ts, fma(w.kz, zj, fma(w.kx, x_mid, w.c0))), &pc[u], &ps[u]);
+            pc[u] *= live;
+            ps[u] *= live;
+          }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const float4 w0 = sh.coef[16 * kc + 4 * g + 2 * h], w1 = sh.coef[16 * kc + 4 * g + 2 * h + 1];
+          const float c0 = pc[2 * h], s0 = ps[2 * h], c1 = pc[2 * h + 1], s1 = ps[2 * h + 1];
+          split2(w0.x * c0, w1.x * c1, bh[0][0].w[at + h], bl[0][0].w[at + h]);
+          split2(w0.y * s0, w1.y * s1, bh[0][1].w[at + h], bl[0][1].w[at + h]);
+          split2(w0.z * c0, w1.z * c1, bh[0][2].w[at + h], bl[0][2].w[at + h]);
+          split2(-w0.x * s0, -w1.x * s1, bh[1][0].w[at + h], bl[1][0].w[at + h]);
+          split2(w0.y * c0, w1.y * c1, bh[1][1].w[at + h], bl[1][1].w[at + h]);
+          split2(-w0.z * s0, -w1.z * s1, bh[1][2].w[at + h], bl[1][2].w[at + h]);
+        }
+      };
+#pragma unroll 1
+      for (int kp = 0; kp < chunks; kp += 2) {
+        Frag bh[2][3], bl[2][3];  // [even / odd]
+        const bool two = kp + 1 < chunks;
+        coefficients(kp, 0, bh, bl);
+        if (two) {
+          coefficients(kp + 1, 2, bh, bl);
+        } else {  // [hi | lo] x ([hi | hi] + [lo | 0])
+#pragma unroll
+          for (int o = 0; o < 2; ++o)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+              bh[o][c].w[2] = bh[o][c].w[0];
+              bh[o][c].w[3] = bh[o][c].w[1];
+              bl[o][c].w[2] = bl[o][c].w[3] = 0u;
+            }
+        }
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+          for (int o = 0; o < 2; ++o) {
+            const Half8 a = sh.fwd_at(chunks, mt, o, kp)[lane];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) d[mt][o][c] = mma(a, bh[o][c].h, d[mt][o][c]);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) d[mt][o][c] = mma(a, bl[o][c].h, d[mt][o][c]);
+          }
+        if (two) {
+#pragma unroll
+          for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int o = 0; o < 2; ++o) {
+              const Half8 a = sh.fwd_at(chunks, mt, o, kp + 1)[lane];
+#pragma unroll
+              for (int c = 0; c < 3; ++c) d[mt][o][c] = mma(a, bh[o][c].h, d[mt][o][c]);
+            }
+        }
+      }
+
+      __builtin_amdgcn_sched_barrier(0);
+      // d holds the folded residuals: r+ = even + odd, r- = even - odd. Columns outside the
+      // strip's share are taken out of both (the last strip only).
+      if (!full_strip) {
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int t = 16 * mt + 4 * g + r, cu = col0 + kHalf + t, cd = col0 + kHalf - 1 - t;
+            const float mu = cu >= lo_col && cu < P.n ? 0.5f : 0.0f, md = cd >= lo_col && cd < P.n ? 0.5f : 0.0f;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+              const float u = mu * (d[mt][0][c][r] + d[mt][1][c][r]), v = md * (d[mt][0][c][r] - d[mt][1][c][r]);
+              d[mt][0][c][r] = u + v;
+              d[mt][1][c][r] = u - v;
+            }
+          }
+      }
+      float big = 0.0f;
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+        for (int o = 0; o < 2; ++o)
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; r += 2)
+              big = fmaxf(fmaxf(fabsf(d[mt][o][c][r]), fabsf(d[mt][o][c][r + 1])), big);
+      big = wave_max(big);
+      // in these units a residual of the size of the largest coefficient is about 2^7: in
+      // range as it is, unless the tile's largest is far from that
+      int res_exp = 0;
+      if (!(big >= kFitResLow && big <= kFitResHigh)) {
+        res_exp = scale_exponent(big);
+        const float res_scale = pow2f(res_exp);
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+          for (int o = 0; o < 2; ++o)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) d[mt][o][c] *= res_scale;
+      }
+      const float inv_r = pow2f(-res_exp) * inv_fwd;  // a residual from its scaled value
+      const float inv_g = 2.0f * inv_r * (1.0f / kFitTrigScale);  // r+ + r- is twice the even part
+      Frag rh[2][3], rl[2][3];  // [even / odd]
+      float sq_t = 0.0f;
+#pragma unroll
+      for (int o = 0; o < 2; ++o)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const Float4& v = d[k >> 1][o][c];
+            const float v0 = v[2 * (k & 1)], v1 = v[2 * (k & 1) + 1];
+            sq_t = fmaf(v0, v0, sq_t);
+            sq_t = fmaf(v1, v1, sq_t);
+            split2(v0, v1, rh[o][c].w[k], rl[o][c].w[k]);
+          }
+      sq = fmaf(sq_t * inv_r, inv_r, sq);  // half the squares: r+^2 + r-^2 = 2 (even^2 + odd^2)
+
+      // backward: per chunk the sums over the strip's columns of r cos and r sin of the
+      // column factor, for 16 waves and 16 pairs; then P turns them into sums over theta
+      float jf[4], sf[4];
+      uint32_t r4[4], t4[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const uint32_t q4 = (uint32_t)tile * 16u + (uint32_t)(4 * g + r);
+        const uint32_t j4 = row_of(q4), s4 = q4 - j4 * (uint32_t)P.S;
+        jf[r] = (float)j4;
+        sf[r] = (float)s4;
+        r4[r] = (j4 - j0) * (uint32_t)(32 * chunks);
+        t4[r] = s4 * (uint32_t)time_row;
+      }
+#pragma unroll 1
+      for (int kc = 0; kc < chunks; ++kc) {
+        const float2 dir = sh.dir[16 * kc + n16];
+        const float qdx = dir.x, qdz = dir.y;
+        float cp[4], sp[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if constexpr (kByTable) {
+            const float2 a = *reinterpret_cast<const float2*>(&s_row[r4[r] + 32 * kc + 2 * n16]);
+            const float2 b = *reinterpret_cast<const float2*>(&sh.time[t4[r] + 32 * kc + 2 * n16]);
+            cp[r] = fmaf(a.x, b.x, -(a.y * b.y));
+            sp[r] = fmaf(a.x, b.y, a.y * b.x);
+          } else {
+            const FitWaveLds& w = sh.wave[16 * kc + n16];
+            sincos_turn(fma(w.om, (double)sf[r] * P.dt, fma(w.kz, P.z0 + (double)jf[r] * P.spacing, fma(w.kx, x_mid, w.c0))),
+                        &cp[r], &sp[r]);
+          }
+        }
+        // per wave of the lane, over its four pairs: sums of r_x cos, r_z cos, r_y sin, and
+        // of h = the misfit's derivative by theta over A = sum r_y cos theta - Q (D . r) sin
+        // theta (plain, times s, times j, times the column's offset). cos of the offset goes
+        // with the even part and sin with the odd one; weighted the other way round.
+        float t[7] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        {
+          Float4 gc[3], gn[3];  // [x, y, z] of the cos and the sin sums
+#pragma unroll
+          for (int c = 0; c < 3; ++c) gc[c] = gn[c] = Float4{0.0f, 0.0f, 0.0f, 0.0f};
+          column_sums(sh.bwd_at(kc, 0, 0, 0)[lane], sh.bwd_at(kc, 0, 0, 1)[lane], rh[0], rl[0], gc);
+          column_sums(sh.bwd_at(kc, 1, 0, 0)[lane], sh.bwd_at(kc, 1, 0, 1)[lane], rh[1], rl[1], gn);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            t[0] = fmaf(cp[r], gc[0][r], fmaf(-sp[r], gn[0][r], t[0]));
+            t[1] = fmaf(cp[r], gc[2][r], fmaf(-sp[r], gn[2][r], t[1]));
+            t[2] = fmaf(cp[r], gn[1][r], fmaf(sp[r], gc[1][r], t[2]));
+            const float hc = fmaf(qdx, gc[0][r], qdz * gc[2][r]), hs = fmaf(qdx, gn[0][r], qdz * gn[2][r]);
+            const float h = fmaf(cp[r], gc[1][r] - hs, -(sp[r] * (gn[1][r] + hc)));
+            t[3] += h;
+            t[4] = fmaf(sf[r], h, t[4]);
+            t[5] = fmaf(jf[r], h, t[5]);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        {
+          Float4 gc[3], gn[3];
+#pragma unroll
+          for (int c = 0; c < 3; ++c) gc[c] = gn[c] = Float4{0.0f, 0.0f, 0.0f, 0.0f};
+          column_sums(sh.bwd_at(kc, 0, 1, 0)[lane], sh.bwd_at(kc, 0, 1, 1)[lane], rh[1], rl[1], gc);
+          column_sums(sh.bwd_at(kc, 1, 1, 0)[lane], sh.bwd_at(kc, 1, 1, 1)[lane], rh[0], rl[0], gn);
+          float wx = 0.0f, wy = 0.0f, wz = 0.0f;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            wy = fmaf(cp[r], gc[1][r], fmaf(-sp[r], gn[1][r], wy));
+            wx = fmaf(cp[r], gn[0][r], fmaf(sp[r], gc[0][r], wx));
+            wz = fmaf(cp[r], gn[2][r], fmaf(sp[r], gc[2][r], wz));
+          }
+          t[6] = fmaf(-qdx, wx, fmaf(-qdz, wz, wy));
+        }
+        // summed over the four groups of pairs by lane swaps: lane rows 0..3 then hold sums
+        // 0, 2, 1, 3 and 4, 6, 5 and a zero
+        const float lo = swap16_sum(swap32_sum(t[0], t[1]), swap32_sum(t[2], t[3]));
+        const float hi = swap16_sum(swap32_sum(t[4], t[5]), swap32_sum(t[6], 0.0f));
+        float2* o = &sh.sums[wid][kc][lane];
+        const float2 old = *o;
+        *o = make_float2(fmaf(lo, inv_g, old.x), fmaf(hi, inv_g, old.y));
+      }
+      if constexpr (kByTable) wavefront_lds_sync();  // the next tile rewrites the row factors
     }
+    if (base + NW < part_end && base + NW < end) continue;
+
+    // ---- the end of a part: the wavefronts' sums in index order, then the parameter
+    // derivatives of the part
+    const float lsum = wave_sum63(sq);
+    if (lane == 63) sh.loss[wid] = lsum;
+    sq = 0.0f;
+    __syncthreads();
+    const int part_index = unit.strip * P.blocks_per_strip + part;
+    if (tid < P.W) {
+      double v[8];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float2 t = sh.sums[0][tid >> 4][16 * r + (tid & 15)];
+        for (int i = 1; i < NW; ++i) {
+          const float2 u = sh.sums[i][tid >> 4][16 * r + (tid & 15)];
+          t.x += u.x;
+          t.y += u.y;
+        }
+        const int k = ((r & 1) << 1) | (r >> 1);
+        v[k] = (double)t.x;
+        v[4 + k] = (double)t.y;
+      }
+      const FitWaveGrad w = sh.grad[tid];
+      // sums of r . dd/dtheta: plain, times t, times the world x and z
+      const double A = w.A, Dx = w.Dx, Dz = w.Dz;
+      const double g0 = A * v[3], gt = A * (P.t0 * v[3] + P.dt * v[4]);
+      const double gx = A * (x_mid * v[3] + P.spacing * v[6]);
+      const double gz = A * (P.z0 * v[3] + P.spacing * v[5]);
+      const double sec = Dx * v[0] + Dz * v[1], sepc = Dx * v[1] - Dz * v[0];
+      const float out[5] = {(float)(w.Q * sec + v[2]), (float)-(w.wL * (Dx * gx + Dz * gz) + w.om2L * gt),
+                            (float)(w.w * (Dx * gz - Dz * gx) + w.Q * A * sepc), (float)(A * sec), (float)g0};
+      float* o = P.partials + (size_t)(5 * tid) * P.nblocks + part_index;
+#pragma unroll
+      for (int k = 0; k < 5; ++k) o[(size_t)k * P.nblocks] = out[k];
+    }
+    if (tid == 0) {
+      float t = sh.loss[0];
+      for (int i = 1; i < NW; ++i) t += sh.loss[i];
+      P.partials[(size_t)(5 * P.W) * P.nblocks + part_index] = t;
+    }
+    __syncthreads();  // the sums have been read
+    for (int kc = 0; kc < chunks; ++kc) sh.sums[wid][kc][lane] = make_float2(0.0f, 0.0f);
+    ++part;
+    part_end += P.tiles_per_block;
   }
 }
 
-// Backward of one wave: six sums over snapshots and three sums of their running values
-// per point, then the five derivatives, added over the thread's points and reduced over
-// the wavefront: lane swaps first (each step sums two registers), then one row sum of
-// the packed register, which leaves dA, dalpha, dL, dQ in rows 0..3 and dphi0 in every
-// row; written to the wave's rows of s_red.
-template <int SMAX, int KP, bool kCheb>
-__device__ __forceinline__ void backward_wave(const FitDesc& P, const FitWaveLds& wv, const float (&c0)[KP],
-                                              const float (&s0)[KP], const double (&x)[KP], const double (&z)[KP],
-                                              const float (&r)[KP][SMAX][3], float* s_red, int lane, int wid) {
-  const float dtf = (float)P.dt;
-  // t0 + SMAX dt: the time weight of the snapshot sums (below)
-  const float tS = (float)(P.t0 + P.dt * SMAX);
-  const float A = wv.A, Q = wv.Q, Dx = wv.Dx, Dz = wv.Dz;
-  float gA = 0.0f, gL = 0.0f, gAl = 0.0f, gQ = 0.0f, gP = 0.0f;
-#pragma unroll
-  for (int k = 0; k < KP; ++k) {
-    float c = c0[k], sn = s0[k], cp = 0.0f, sp = 0.0f;
-    float sxc = 0, szc = 0, syc = 0, sxs = 0, szs = 0, sys = 0, vyc = 0, vxs = 0, vzs = 0;
-#pragma unroll
-    for (int s = 0; s < SMAX; ++s) {
-      const float rx = r[k][s][0], ry = r[k][s][1], rz = r[k][s][2];
-      sxc = fmaf(rx, c, sxc);
-      szc = fmaf(rz, c, szc);
-      syc = fmaf(ry, c, syc);
-      sxs = fmaf(rx, sn, sxs);
-      szs = fmaf(rz, sn, szs);
-      sys = fmaf(ry, sn, sys);
-      vyc += syc;
-      vxs += sxs;
-      vzs += szs;
-      step_snapshot<kCheb>(s, c, sn, cp, sp, wv);
-    }
-    // r . dd/dtheta = A (ry cos - Q (D . r) sin): m0 is its sum over snapshots / A, m1
-    // the same of the running sums. With t_s = t0 + s dt and sum_s s f_s = SMAX U - V
-    // (U a sum, V the sum of its running values; the residuals past S are zero),
-    // sum_s t_s f_s = (t0 + SMAX dt) U - dt V.
-    const float m0 = syc - fmaf(wv.qdx, sxs, wv.qdz * szs);
-    const float m1 = vyc - fmaf(wv.qdx, vxs, wv.qdz * vzs);
-    const float g0 = A * m0;                        // sum of r . dd/dtheta
-    const float g0t = A * fmaf(tS, m0, -dtf * m1);  // sum of t r . dd/dtheta
-    const float sec = fmaf(Dx, sxc, Dz * szc);      // sum of (r . D) cos
-    const float sepc = fmaf(Dx, szc, -Dz * sxc);    // sum of (r . D-perp) cos
-    // D . x and D-perp . x: the local offset from the grid origin plus the origin's term
-    const float xf = (float)(x[k] - P.x0), zf = (float)(z[k] - P.z0);
-    const float dotx = fmaf(Dx, xf, fmaf(Dz, zf, wv.od));
-    const float perpx = fmaf(Dx, zf, fmaf(-Dz, xf, wv.op));
-    // inactive points have zero residuals, so every sum above is zero for them
-    gA += fmaf(Q, sec, sys);
-    gL -= fmaf(wv.wL * dotx, g0, wv.om2L * g0t);
-    gAl += fmaf(wv.w * perpx, g0, Q * A * sepc);
-    gQ += A * sec;
-    gP += g0;
-  }
-  const float t = row_sum(swap16_sum(swap32_sum(gA, gL), swap32_sum(gAl, gQ)));
-  const float pp = swap32_sum(gP, gP);
-  const float tp = row_sum(swap16_sum(pp, pp));
-  if ((lane & 15) == 15) {
-    const int row = lane >> 4;
-    float* o = s_red + (wv.orig * 5) * 4 + wid;
-    o[(((row & 1) << 1) | (row >> 1)) * 4] = t;  // rows 0..3 hold dA, dalpha, dL, dQ
-    if (row == 0) o[4 * 4] = tp;
-  }
-}
-
-// Forward passes of waves [i0, i1). Each iteration seeds the next wave first: its FP64
-// phase reduction, sine and cosine (long-latency, and independent of the current wave)
-// then overlap the current wave's snapshot steps instead of stalling at the top of the
-// next iteration.
-template <int SMAX, int KP, bool kCheb>
-__device__ __forceinline__ void forward_waves(const FitWaveLds* s_wave, int i0, int i1, const double (&x)[KP],
-                                              const double (&z)[KP], float (&r)[KP][SMAX][3]) {
-  if (i0 >= i1) return;
-  float c[KP], sn[KP];
-  wave_seeds<KP>(s_wave[i0], x, z, c, sn);
-  for (int i = i0; i < i1; ++i) {
-    float cn[KP], snn[KP];
-    wave_seeds<KP>(s_wave[i + 1 < i1 ? i + 1 : i], x, z, cn, snn);
-    forward_wave<SMAX, KP, kCheb>(s_wave[i], c, sn, r);
-#pragma unroll
-    for (int k = 0; k < KP; ++k) {
-      c[k] = cn[k];
-      sn[k] = snn[k];
-    }
-  }
-}
-
-// Backward passes of waves [i0, i1), seeded one wave ahead as in forward_waves.
-template <int SMAX, int KP, bool kCheb>
-__device__ __forceinline__ void backward_waves(const FitDesc& P, const FitWaveLds* s_wave, int i0, int i1,
-                                               const double (&x)[KP], const double (&z)[KP],
-                                               const float (&r)[KP][SMAX][3], float* s_red, int lane, int wid) {
-  if (i0 >= i1) return;
-  float c[KP], sn[KP];
-  wave_seeds<KP>(s_wave[i0], x, z, c, sn);
-  for (int i = i0; i < i1; ++i) {
-    float cn[KP], snn[KP];
-    wave_seeds<KP>(s_wave[i + 1 < i1 ? i + 1 : i], x, z, cn, snn);
-    backward_wave<SMAX, KP, kCheb>(P, s_wave[i], c, sn, x, z, r, s_red, lane, wid);
-#pragma unroll
-    for (int k = 0; k < KP; ++k) {
-      c[k] = cn[k];
-      sn[k] = snn[k];
-    }
-  }
-}
-
-// s_wave holds the problem's waves with the ncheb three-term-recurrence waves first, so
-// each loop over waves is branch-free.
-template <int SMAX, int KP>
-__device__ __forceinline__ void adjoint_body(const FitDesc& P, int local_block, const FitWaveLds* s_wave, int ncheb,
-                                             float* s_red) {
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int V = P.n * P.n;
-  const int S = P.S;
-  // a wave64 VALU instruction runs as four passes of 16 lanes: lanes l, l + 16, l + 32,
-  // l + 48 take four consecutive points, so consecutive passes see close operand values
-  // and toggle less of the datapath (the kernel runs at the board's power limit); the
-  // wavefront still covers 64 consecutive points
-  const int pt = (wid << 6) + ((lane & 15) << 2) + (lane >> 4);
-  bool active[KP];
-  int vv[KP];
-  double x[KP], z[KP];
-#pragma unroll
-  for (int k = 0; k < KP; ++k) {
-    const int v = (local_block * KP + k) * kFitThreads + pt;
-    active[k] = v < V;
-    vv[k] = active[k] ? v : 0;
-    x[k] = P.x0 + (double)(vv[k] % P.n) * P.spacing;
-    z[k] = P.z0 + (double)(vv[k] / P.n) * P.spacing;
-  }
-
-  float r[KP][SMAX][3];
-#pragma unroll
-  for (int k = 0; k < KP; ++k)
-#pragma unroll
-    for (int s = 0; s < SMAX; ++s) r[k][s][0] = r[k][s][1] = r[k][s][2] = 0.0f;
-
-  // forward: d per snapshot
-  forward_waves<SMAX, KP, true>(s_wave, 0, ncheb, x, z, r);
-  forward_waves<SMAX, KP, false>(s_wave, ncheb, P.W, x, z, r);
-  // residuals and loss
-  float sq = 0.0f;  // sum of squared residuals; the loss is half of it
-#pragma unroll
-  for (int k = 0; k < KP; ++k) {
-    // the point's target record in snapshot 0; snapshot s is s V records further (a
-    // wave-uniform offset)
-    const float* tgp = P.target + (size_t)vv[k] * 3;
-#pragma unroll
-    for (int s = 0; s < SMAX; ++s) {
-      // snapshots past S (and points past the grid) get zero residuals; their loads
-      // read the last snapshot so every address stays inside the target. The mask is a
-      // factor rather than a select: a select on a loaded value is turned into a branch
-      // around the load, which then waits for memory once per snapshot.
-      const float use = active[k] && s < S ? 1.0f : 0.0f;
-      const float* tg = tgp + (size_t)(s < S ? s : S - 1) * (size_t)(3 * V);
-      const float t0 = tg[0], t1 = tg[1], t2 = tg[2];
-      r[k][s][0] = (r[k][s][0] - t0) * use;
-      r[k][s][1] = (r[k][s][1] - t1) * use;
-      r[k][s][2] = (r[k][s][2] - t2) * use;
-      sq = fmaf(r[k][s][0], r[k][s][0], sq);
-      sq = fmaf(r[k][s][1], r[k][s][1], sq);
-      sq = fmaf(r[k][s][2], r[k][s][2], sq);
-    }
-  }
-  const float lsum = 0.5f * wave_sum63(sq);
-  if (lane == 63) s_red[(P.W * 5) * 4 + wid] = lsum;
-
-  // backward
-  backward_waves<SMAX, KP, true>(P, s_wave, 0, ncheb, x, z, r, s_red, lane, wid);
-  backward_waves<SMAX, KP, false>(P, s_wave, ncheb, P.W, x, z, r, s_red, lane, wid);
-}
-
-// Stage the problem's waves into LDS, three-term-recurrence waves first (each group in
-// wave order); returns their number. Wavefront 0 does it, lane l taking waves l and
-// l + 64 (kFitMaxWaves = 128): the recurrence flags of both halves are balloted, so each
-// wave's position comes from two population counts, with no pass over the flags.
-__device__ __forceinline__ int stage_fit_waves(const FitDesc& P, FitWaveLds* s_wave, int* s_ncheb) {
-  static_assert(kFitMaxWaves <= 128, "two waves per lane of one wavefront");
-  if (threadIdx.x < 64) {
-    const int lane = threadIdx.x;
-    const int i0 = lane, i1 = lane + 64;
-    bool c0 = false, c1 = false;
-    FitWaveLds w0, w1;
-    if (i0 < P.W) w0 = fit_wave_constants(P, i0, &c0);
-    if (i1 < P.W) w1 = fit_wave_constants(P, i1, &c1);
-    const uint64_t b0 = __ballot(c0), b1 = __ballot(c1);
-    const uint64_t below = (1ull << lane) - 1ull;  // lanes under this one
-    const int n0 = __popcll(b0), ncheb = n0 + __popcll(b1);
-    if (i0 < P.W) {
-      const int before = __popcll(b0 & below);  // recurrence waves ahead of i0
-      s_wave[c0 ? before : ncheb + (i0 - before)] = w0;
-    }
-    if (i1 < P.W) {
-      const int before = n0 + __popcll(b1 & below);
-      s_wave[c1 ? before : ncheb + (i1 - before)] = w1;
-    }
-    if (lane == 0) *s_ncheb = ncheb;
-  }
-  __syncthreads();
-  return *s_ncheb;
-}
-
-// One launch covers the blocks [base, base + gridDim.x) of the batch's block -> problem
-// map, all of one snapshot class.
-template <int SMAX, int KP>
-__global__ __launch_bounds__(kFitThreads) __attribute__((amdgpu_waves_per_eu(kFitWavesPerSimd[(SMAX - 1) / 4])))
-void adjoint_kernel(const FitDesc* __restrict__ probs,
-                                                              const int* __restrict__ block_prob, long long base,
-                                                              int bump_step) {
-  __shared__ FitWaveLds s_wave[kFitMaxWaves];
-  __shared__ float s_red[(kFitMaxWaves * 5 + 1) * 4];
-  __shared__ int s_ncheb;
-  const long long gb = base + blockIdx.x;
-  // the problem and block tables do not change during the launch: scalar loads, so the
+// One workgroup: a unit's strip and parts. KMAX bounds the problem's chunks of 16 waves.
+template <int KMAX, int NW, bool kTable>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4)))
+void adjoint_kernel(const FitDesc* __restrict__ probs, const FitUnit* __restrict__ units, int bump_step) {
+  __shared__ FitShared<KMAX, NW, kTable> sh;
+  const int tid = threadIdx.x;
+  // the problem and unit tables do not change during the launch: scalar loads, so the
   // descriptor sits in SGPRs rather than VGPRs
-  const FitDesc P = load_uniform(probs, load_uniform(block_prob, gb));
-  const int local_block = (int)(gb - P.block_offset);
-  if (bump_step && local_block == 0 && threadIdx.x == 0) P.step[0] += 1;  // Adam step of this iteration
-  const int ncheb = stage_fit_waves(P, s_wave, &s_ncheb);
-  adjoint_body<SMAX, KP>(P, local_block, s_wave, ncheb, s_red);
+  const FitUnit unit = load_uniform(units, (long long)blockIdx.x);
+  const FitDesc P = load_uniform(probs, unit.problem);
+  if (bump_step && unit.strip == 0 && unit.part == 0 && tid == 0) P.step[0] += 1;  // Adam step of this iteration
+  const int chunks = (P.W + 15) >> 4, padded = 16 * chunks;
+
+  // ---- the waves' constants, one thread per wave
+  if (tid == 0) sh.max = 0;
   __syncthreads();
-  // fixed-order sum over the 4 wavefronts, one partial per (row, block)
-  const int rows = P.W * 5 + 1;
-  for (int j = threadIdx.x; j < rows; j += blockDim.x) {
-    const float* q = s_red + j * 4;
-    P.partials[(size_t)j * P.nblocks + local_block] = ((q[0] + q[1]) + q[2]) + q[3];
+  FitWaveLds wv{};
+  float bx = 0.0f, by = 0.0f, bz = 0.0f;
+  if (tid < P.W) {
+    const float* pr = P.params + 5 * tid;
+    const double A = pr[0], L = pr[1] > 1e-3f ? pr[1] : 1e-3f, al = pr[2], Q = pr[3], ph0 = pr[4];
+    const double w = kTwoPi / L, om = sqrt(P.g * w);
+    double sa, ca;
+    sincos(al, &sa, &ca);
+    wv.kx = w * ca * kInvTwoPi;
+    wv.kz = w * sa * kInvTwoPi;
+    wv.c0 = __builtin_amdgcn_fract((om * P.t0 + ph0) * kInvTwoPi);
+    wv.om = om * kInvTwoPi;
+    bx = (float)(Q * A * ca);
+    by = (float)A;
+    bz = (float)(Q * A * sa);
+    sh.dir[tid] = make_float2((float)(Q * ca), (float)(Q * sa));
+    sh.grad[tid] = FitWaveGrad{(float)A, (float)Q, (float)ca, (float)sa, (float)w, (float)(w / L), (float)(om / (2.0 * L))};
+    atomicMax(&sh.max, __float_as_uint(fmaxf(fmaxf(fabsf(bx), fabsf(bz)), fabsf(by))));
+  }
+  __syncthreads();
+  const int coef_exp = scale_exponent(__uint_as_float(__builtin_amdgcn_readfirstlane((int)sh.max)));
+  if (tid < padded) {
+    const float sc = pow2f(coef_exp);
+    sh.coef[tid] = make_float4(bx * sc, by * sc, bz * sc, 0.0f);
+    sh.wave[tid] = wv;
+    if (tid >= P.W) sh.dir[tid] = make_float2(0.0f, 0.0f);
+  }
+  __syncthreads();
+
+  // ---- the column factors, per thread and step one wave at two neighbouring offsets t,
+  // t + 1: a word of a backward operand's lane slot (wave `slot mod 16` of a chunk, offsets
+  // 16 (e / 4) + 4 (slot / 16) + e mod 4, the order in which the forward pass leaves them
+  // in a lane), and the same values in the forward operand, whose lane (t mod 16, g) holds
+  // waves 4 g .. 4 g + 3 of each chunk
+  for (int it = tid; it < chunks * 256; it += 64 * NW) {
+    const int slot = it & 63, k = (it >> 6) & 3, kc = it >> 8;
+    const int wl = slot & 15;
+    const int t = 16 * (k >> 1) + 4 * (slot >> 4) + 2 * (k & 1);
+    const bool odd = (chunks & 1) && kc == chunks - 1;
+    const double step = sh.wave[16 * kc + wl].kx * P.spacing;  // zero for the padding, whose coefficients are zero
+#pragma unroll
+    for (int o = 0; o < 2; ++o) {
+      float c[2], s2[2];
+      sincos_turn(step * ((double)t + 0.5), &c[0], &s2[0]);
+      sincos_turn(step * ((double)t + 1.5), &c[1], &s2[1]);
+      const float v0 = (o ? s2[0] : c[0]) * kFitTrigScale, v1 = (o ? s2[1] : c[1]) * kFitTrigScale;
+      uint32_t hi, lo;
+      split2(v0, v1, hi, lo);
+      reinterpret_cast<uint32_t*>(&sh.bwd_at(kc, o, 0, 0)[slot])[k] = hi;
+      reinterpret_cast<uint32_t*>(&sh.bwd_at(kc, o, 0, 1)[slot])[k] = lo;
+      const int fs = (wl >> 2) * 16 + (t & 15);
+      _Float16* fh = reinterpret_cast<_Float16*>(&sh.fwd_at(chunks, t >> 4, o, odd ? kc : kc & ~1)[fs]);
+      _Float16* fl = reinterpret_cast<_Float16*>(&sh.fwd_at(chunks, t >> 4, o, odd ? kc : kc | 1)[fs]);
+      const int eh = 4 * (kc & 1) + (wl & 3), el = odd ? 4 + (wl & 3) : eh;
+      fh[eh] = __builtin_bit_cast(Half2, hi).x;
+      fh[8 + eh] = __builtin_bit_cast(Half2, hi).y;  // the next lane's slot
+      fl[el] = __builtin_bit_cast(Half2, lo).x;
+      fl[8 + el] = __builtin_bit_cast(Half2, lo).y;
+      split2(((float)t + 0.5f) * v0, ((float)t + 1.5f) * v1, hi, lo);
+      reinterpret_cast<uint32_t*>(&sh.bwd_at(kc, o, 1, 0)[slot])[k] = hi;
+      reinterpret_cast<uint32_t*>(&sh.bwd_at(kc, o, 1, 1)[slot])[k] = lo;
+    }
+  }
+  // a tile's 16 pairs touch at most four rows from five snapshots on: P is then a row
+  // factor times a time factor (4 FMAs per wave and pair, and one sine and cosine per wave
+  // and row); below, each pair takes its own sine and cosine. The two ways are two copies
+  // of the loop.
+  if (kTable && P.S >= 5) {
+    for (int it = tid; it < (P.S + 1) * padded; it += 64 * NW) {
+      const int sn = it / padded, wi = it - sn * padded;
+      float cv = 0.0f, sv = 0.0f;
+      if (sn < P.S) sincos_turn(sh.wave[wi].om * ((double)sn * P.dt), &cv, &sv);
+      *reinterpret_cast<float2*>(&sh.time[sn * (2 * padded + 4) + 2 * wi]) = make_float2(cv, sv);
+    }
+    __syncthreads();
+    fit_tiles<true>(P, unit, sh, chunks, coef_exp);
+  } else {
+    __syncthreads();
+    fit_tiles<false>(P, unit, sh, chunks, coef_exp);
   }
 }
 
-__global__ __launch_bounds__(kFitThreads) void reduce_adam_kernel(const FitDesc* __restrict__ probs,
+__global__ __launch_bounds__(kReduceThreads) void reduce_adam_kernel(const FitDesc* __restrict__ probs,
                                                                   const int* __restrict__ row_prob, FitAdam adam,
                                                                   int mode, float* __restrict__ grad_out,
                                                                   float* __restrict__ loss_out) {
-  static_assert(kFitThreads == 256, "the final sum reads four wavefront partials");
-  __shared__ float s[kFitThreads / 64];
+  static_assert(kReduceThreads == 256, "the final sum reads four wavefront partials");
+  __shared__ float s[kReduceThreads / 64];
   const int s_prob = load_uniform(row_prob, (long long)blockIdx.x);
   const FitDesc P = load_uniform(probs, s_prob);
   const int row = (int)(blockIdx.x - P.row_offset);
@@ -494,20 +803,42 @@ __device__ __forceinline__ unsigned long long splitmix64(unsigned long long z) {
 
 __device__ __forceinline__ double unit_double(unsigned long long z) { return (double)(z >> 11) * (1.0 / 9007199254740992.0); }
 
-__global__ __launch_bounds__(kFitThreads) void synthesize_kernel(FitDesc P, float* __restrict__ out, float sigma,
+struct SynthWaveLds {
+  double kx, kz, c0, om_rev;  // revolutions per metre along x / z, phase at t0 (fract), revolutions per second
+  float qadx, qadz, A;
+};
+
+__device__ __forceinline__ void stage_synth_wave(const FitDesc& P, int i, SynthWaveLds* o) {
+  const float* pr = P.params + 5 * i;
+  const double A = pr[0], L = pr[1] > 1e-3f ? pr[1] : 1e-3f, al = pr[2], Q = pr[3], ph0 = pr[4];
+  const double w = kTwoPi / L, om = sqrt(P.g * w);
+  double sa, ca;
+  sincos(al, &sa, &ca);
+  o->kx = w * ca * kInvTwoPi;
+  o->kz = w * sa * kInvTwoPi;
+  const double ph = (om * P.t0 + ph0) * kInvTwoPi;
+  o->c0 = ph - floor(ph);
+  o->om_rev = om * kInvTwoPi;
+  o->A = (float)A;
+  o->qadx = (float)(Q * A * ca);
+  o->qadz = (float)(Q * A * sa);
+}
+
+constexpr int kSynthThreads = 256;
+__global__ __launch_bounds__(kSynthThreads) void synthesize_kernel(FitDesc P, float* __restrict__ out, float sigma,
                                                                  unsigned long long seed) {
-  __shared__ FitWaveLds s_wave[kFitMaxWaves];
-  for (int i = threadIdx.x; i < P.W; i += blockDim.x) stage_fit_wave(P, i, &s_wave[i]);
+  __shared__ SynthWaveLds s_wave[kFitMaxWaves];
+  for (int i = threadIdx.x; i < P.W; i += blockDim.x) stage_synth_wave(P, i, &s_wave[i]);
   __syncthreads();
   const long long V = (long long)P.n * P.n;
-  const long long v = (long long)blockIdx.x * kFitThreads + threadIdx.x;
+  const long long v = (long long)blockIdx.x * kSynthThreads + threadIdx.x;
   if (v >= V) return;
   const double x = P.x0 + (double)(v % P.n) * P.spacing;
   const double z = P.z0 + (double)(v / P.n) * P.spacing;
   for (int s = 0; s < P.S; ++s) {
     float d0 = 0.0f, d1 = 0.0f, d2 = 0.0f;
     for (int i = 0; i < P.W; ++i) {
-      const FitWaveLds& wv = s_wave[i];
+      const SynthWaveLds& wv = s_wave[i];
       // phase at snapshot s in FP64: phase at t0 plus omega s dt, reduced to one revolution
       const double ph = fma(wv.kx, x, fma(wv.kz, z, wv.c0)) + wv.om_rev * (P.dt * s);
       const float f = (float)__builtin_amdgcn_fract(ph);
@@ -533,8 +864,8 @@ __global__ __launch_bounds__(kFitThreads) void synthesize_kernel(FitDesc P, floa
 
 hipError_t launch_synthesize(const FitDesc& P, float* out, float sigma, unsigned long long seed, hipStream_t st) {
   const long long V = (long long)P.n * P.n;
-  const long long blocks = (V + kFitThreads - 1) / kFitThreads;
-  hipLaunchKernelGGL(synthesize_kernel, dim3((unsigned)blocks), dim3(kFitThreads), 0, st, P, out, sigma, seed);
+  const long long blocks = (V + kSynthThreads - 1) / kSynthThreads;
+  hipLaunchKernelGGL(synthesize_kernel, dim3((unsigned)blocks), dim3(kSynthThreads), 0, st, P, out, sigma, seed);
   return hipGetLastError();
 }
 
@@ -550,32 +881,35 @@ hipError_t launch_zero_words(uint32_t* p, size_t n, hipStream_t st) {
   return hipGetLastError();
 }
 
-__global__ void fit_setup_single_kernel(FitDesc d, FitDesc* __restrict__ d_desc, int* __restrict__ d_maps,
-                                        size_t map_words, uint32_t* __restrict__ zero_begin, size_t zero_words) {
+__global__ void fit_setup_single_kernel(FitDesc d, FitDesc* __restrict__ d_desc, FitUnit* __restrict__ d_units,
+                                        size_t units, uint32_t* __restrict__ zero_begin, size_t zero_words) {
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i0 == 0) *d_desc = d;
-  for (size_t i = i0; i < map_words; i += stride) d_maps[i] = 0;
+  for (size_t i = i0; i < units; i += stride) {
+    const int strip = (int)i / d.blocks_per_strip;
+    d_units[i] = FitUnit{0, strip, (int)i - strip * d.blocks_per_strip, 1};
+  }
   for (size_t i = i0; i < zero_words; i += stride) zero_begin[i] = 0u;
 }
 
-hipError_t launch_fit_setup_single(const FitDesc& d, FitDesc* d_desc, int* d_maps, size_t map_words,
+hipError_t launch_fit_setup_single(const FitDesc& d, FitDesc* d_desc, FitUnit* d_units, size_t units,
                                    uint32_t* zero_begin, size_t zero_words, hipStream_t st) {
-  size_t n = map_words > zero_words ? map_words : zero_words;
+  size_t n = units > zero_words ? units : zero_words;
   size_t blocks = (n + 255) / 256;
   if (blocks < 1) blocks = 1;
   if (blocks > 1024) blocks = 1024;
-  hipLaunchKernelGGL(fit_setup_single_kernel, dim3((unsigned)blocks), dim3(256), 0, st, d, d_desc, d_maps, map_words,
+  hipLaunchKernelGGL(fit_setup_single_kernel, dim3((unsigned)blocks), dim3(256), 0, st, d, d_desc, d_units, units,
                      zero_begin, zero_words);
   return hipGetLastError();
 }
 
-// The adjoint launch of snapshot class c on stream st.
+// The adjoint launch of wave-count class c on stream st.
 template <int C>
 hipError_t launch_adjoint_class(const FitLaunch& L, int c, int bump, hipStream_t st) {
   if (c == C) {
-    hipLaunchKernelGGL((adjoint_kernel<kFitClassMaxS[C], kFitPointsPerThread[C]>), dim3((unsigned)L.class_blocks[C]),
-                       dim3(kFitThreads), 0, st, L.probs, L.block_prob, L.class_begin[C], bump);
+    hipLaunchKernelGGL((adjoint_kernel<kFitClassChunks[C], kFitWavefronts, C == 0>), dim3((unsigned)L.class_blocks[C]),
+                       dim3(64 * kFitWavefronts), 0, st, L.probs, L.units + L.class_begin[C], bump);
     return hipGetLastError();
   }
   if constexpr (C + 1 < kFitClasses) return launch_adjoint_class<C + 1>(L, c, bump, st);
@@ -585,11 +919,11 @@ hipError_t launch_adjoint_class(const FitLaunch& L, int c, int bump, hipStream_t
 hipError_t launch_fit_iteration(const FitLaunch& L, const FitAdam& adam, int mode, float* grad_out, float* loss_out,
                                 hipStream_t st) {
   const int bump = mode == 1 ? 1 : 0;
-  // classes present, the most work (blocks x snapshots) first
+  // classes present, the most work (blocks x waves) first
   int order[kFitClasses], n = 0;
   for (int c = 0; c < kFitClasses; ++c)
     if (L.class_blocks[c] > 0) order[n++] = c;
-  auto work = [&](int c) { return (double)L.class_blocks[c] * kFitClassMaxS[c]; };
+  auto work = [&](int c) { return (double)L.class_blocks[c] * kFitClassChunks[c]; };
   for (int i = 1; i < n; ++i)
     for (int j = i; j > 0 && work(order[j]) > work(order[j - 1]); --j) std::swap(order[j], order[j - 1]);
   if (n <= 1 || !L.side[0]) {
@@ -614,7 +948,7 @@ hipError_t launch_fit_iteration(const FitLaunch& L, const FitAdam& adam, int mod
       if ((e = hipStreamWaitEvent(st, L.join[j], 0)) != hipSuccess) return e;
     }
   }
-  hipLaunchKernelGGL(reduce_adam_kernel, dim3((unsigned)L.total_rows), dim3(kFitThreads), 0, st, L.probs, L.row_prob,
+  hipLaunchKernelGGL(reduce_adam_kernel, dim3((unsigned)L.total_rows), dim3(kReduceThreads), 0, st, L.probs, L.row_prob,
                      adam, mode, grad_out, loss_out);
   return hipGetLastError();
 }

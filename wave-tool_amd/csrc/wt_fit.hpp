@@ -12,20 +12,37 @@ namespace wt {
 
 constexpr int kFitMaxWaves = 128;
 constexpr int kFitMaxSnapshots = 32;
-constexpr int kFitThreads = 256;
-// Snapshot classes S <= 4, 8, ..., 32 and the grid points each thread of their adjoint
-// kernel carries (its residuals, KP x SMAX x 3 floats, stay in registers). The kernel
-// of a class steps all SMAX snapshots without branches (residuals past S are zero), so
-// classes 4 snapshots wide waste at most 3 per point.
-constexpr int kFitClasses = 8;
-constexpr int kFitClassMaxS[kFitClasses] = {4, 8, 12, 16, 20, 24, 28, 32};
-constexpr int kFitPointsPerThread[kFitClasses] = {2, 2, 1, 1, 1, 1, 1, 1};
-// Wavefronts per SIMD each class's adjoint kernel is compiled for (1: no request). The
-// classes listed fit one more wavefront per SIMD than the register allocator's own
-// choice gives, with no spills and the same instructions (4: 84 -> 80 VGPRs, 12: 83 ->
-// 80, 20: 101 -> 96); for the others the next step spills.
-constexpr int kFitWavesPerSimd[kFitClasses] = {6, 1, 6, 1, 5, 1, 1, 1};
-inline int fit_class(int S) { return (S - 1) / 4; }
+constexpr int kReduceThreads = 256;
+// Wave-count classes W <= 64 and W <= 128: the chunks of 16 waves the adjoint kernel's LDS
+// has room for. From 65 waves on the time table does not fit beside the rest.
+constexpr int kFitClasses = 2;
+constexpr int kFitClassChunks[kFitClasses] = {4, 8};
+constexpr int kFitWavefronts = 8;  // of an adjoint workgroup: two per SIMD, sharing the tables
+inline int fit_class(int W) { return W <= 64 ? 0 : 1; }
+// How a problem's work is cut into adjoint blocks: strips of columns, and per strip runs
+// of tiles of 16 (row, snapshot) pairs. It depends on the problem alone.
+struct FitBlocks {
+  int tiles_per_block, blocks_per_strip, nblocks;
+};
+inline FitBlocks fit_blocks(int n, int S) {
+  const long long strips = (n + 63) / 64, tiles = ((long long)n * S + 15) / 16;
+  // enough tiles per wavefront to pay for a block's set-up, unless the problem is too
+  // small to fill the GPU's wavefronts that way
+  long long per_wave = (strips * tiles + 2047) / 2048;
+  if (per_wave > 8) per_wave = 8;
+  FitBlocks b;
+  b.tiles_per_block = (int)(per_wave * kFitWavefronts);
+  b.blocks_per_strip = (int)((tiles + b.tiles_per_block - 1) / b.tiles_per_block);
+  b.nblocks = (int)(strips * b.blocks_per_strip);
+  return b;
+}
+
+// One adjoint workgroup: parts [part, part + parts) of one strip of a problem. A part's
+// sums are the same whichever workgroup takes it; a workgroup of several parts sets the
+// strip's tables up once.
+struct FitUnit {
+  int problem, strip, part, parts;
+};
 
 // One problem of a batch as the kernels see it. Device pointers are owned by the
 // wt_fit handle except params and target, which the caller owns.
@@ -38,8 +55,8 @@ struct FitDesc {
   float* partials;      // [W*5 + 1][nblocks]: per-block sums of r . dd/dp and of |r|^2 / 2
   float* loss;          // [1] loss of the last evaluation
   int* step;            // [1] Adam step counter
-  int n, S, W, nblocks;         // nblocks: adjoint blocks of kFitThreads x KP points
-  long long block_offset;      // first block of this problem in the block -> problem map
+  int n, S, W;
+  int tiles_per_block, blocks_per_strip, nblocks;  // FitBlocks
   long long row_offset;        // first row of this problem in the reduce grid
   long long param_out_offset;  // first parameter of this problem in a concatenated gradient
 };
@@ -48,16 +65,16 @@ struct FitAdam {
   float lr, beta1, beta2, eps;
 };
 
-// Device tables of a batch: problems, block -> problem (blocks grouped by snapshot
-// class, class c at [class_begin[c], + class_blocks[c])), reduce row -> problem.
-// Streams beside the caller's on which the snapshot classes' adjoint launches run
+// Device tables of a batch: problems, adjoint units (grouped by wave-count class, class c
+// at [class_begin[c], + class_blocks[c])), reduce row -> problem.
+// Streams beside the caller's on which the classes' adjoint launches run
 // concurrently (one class's tail overlaps the next class's blocks), joined by events
 // before the reduction.
 constexpr int kFitSideStreams = 3;
 
 struct FitLaunch {
   const FitDesc* probs;
-  const int* block_prob;
+  const FitUnit* units;
   const int* row_prob;
   long long class_begin[kFitClasses];
   long long class_blocks[kFitClasses];
@@ -78,11 +95,11 @@ hipError_t launch_synthesize(const FitDesc& P, float* out, float sigma, unsigned
 // Zero n 32-bit words with a kernel (graph-capture safe).
 hipError_t launch_zero_words(uint32_t* p, size_t n, hipStream_t st);
 
-// Writes one problem's descriptor (passed by value) to d_desc, fills the block and row
-// maps (map_words ints at d_maps) with problem 0, and zeroes zero_words 32-bit words at
-// zero_begin, in one kernel: the set-up of a single-problem evaluation in memory the
-// caller did not allocate per call.
-hipError_t launch_fit_setup_single(const FitDesc& d, FitDesc* d_desc, int* d_maps, size_t map_words,
+// Writes one problem's descriptor (passed by value) to d_desc, its units, one part each,
+// to d_units, and zeroes zero_words 32-bit words at zero_begin (the row map, Adam state,
+// loss and step counter), in one kernel: the set-up of a single-problem evaluation in
+// memory the caller did not allocate per call.
+hipError_t launch_fit_setup_single(const FitDesc& d, FitDesc* d_desc, FitUnit* d_units, size_t units,
                                    uint32_t* zero_begin, size_t zero_words, hipStream_t st);
 
 // The device address of this library's fixed single-problem fit scratch on `device`

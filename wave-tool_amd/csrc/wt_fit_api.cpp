@@ -21,10 +21,11 @@ wt_status ctx_fail(wt_ctx* ctx, wt_status s, const std::string& msg);
 struct wt_fit {
   wt_ctx* ctx = nullptr;
   int count = 0;
-  long long total_blocks = 0, total_rows = 0, total_params = 0;
+  long long total_rows = 0, total_params = 0;
   std::vector<wt::FitDesc> host;
   wt::FitDesc* d_desc = nullptr;
-  int* d_maps = nullptr;    // block -> problem, then row -> problem
+  wt::FitUnit* d_units = nullptr;
+  int* d_rows = nullptr;    // reduce row -> problem
   char* d_state = nullptr;  // moments, partials, loss, step for every problem
   size_t state_bytes = 0;
   wt::FitLaunch launch{};
@@ -67,20 +68,34 @@ std::vector<void*> g_scratch_ptr;          // per device, once resolved
 std::vector<std::string> g_scratch_error;  // per device, when resolving failed
 std::vector<char> g_scratch_done;
 
+constexpr size_t kStaticFitDescBytes = 144;  // of a problem's descriptor, as the limit counts it
+
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // Layout of the scratch for a problem of `np` = 5 W parameters and `nblocks` adjoint
-// blocks: descriptor | maps (nblocks + np + 1 ints) | m, v (np floats each) | loss, step
-// | partials ((np + 1) x nblocks floats). Returns the total bytes; offsets through the
+// blocks: descriptor | units | row map (np + 1 ints), m, v (np floats each), loss, step |
+// partials ((np + 1) x nblocks floats). Returns the total bytes; offsets through the
 // pointers.
-size_t static_fit_layout(int np, int nblocks, size_t* maps, size_t* state, size_t* partials) {
+size_t static_fit_layout(int np, int nblocks, size_t* units, size_t* rows, size_t* partials) {
   size_t off = align256(sizeof(wt::FitDesc));
-  *maps = off;
-  off = align256(off + sizeof(int) * ((size_t)nblocks + np + 1));
-  *state = off;
-  off = align256(off + sizeof(float) * (2 * (size_t)np + 2));
+  *units = off;
+  off = align256(off + sizeof(wt::FitUnit) * (size_t)nblocks);
+  *rows = off;
+  off = align256(off + sizeof(float) * (3 * (size_t)np + 3));
   *partials = off;
   return off + sizeof(float) * (size_t)(np + 1) * nblocks;
+}
+
+// The bytes the entry point's documented limit counts, in blocks of 256 grid points (512
+// for S <= 8): descriptor, maps, state and partials of that many blocks. The adjoint's own
+// parts need less wherever this is near the limit.
+size_t static_fit_limit(const wt_fit_problem& p) {
+  const size_t V = (size_t)p.grid_side * p.grid_side, np = 5 * (size_t)p.wave_count;
+  const size_t points = p.snapshots <= 8 ? 512 : 256, blocks = (V + points - 1) / points;
+  size_t off = align256(kStaticFitDescBytes);
+  off = align256(off + sizeof(int) * (blocks + np + 1));
+  off = align256(off + sizeof(float) * (2 * np + 2));
+  return off + sizeof(float) * (np + 1) * blocks;
 }
 
 }  // namespace
@@ -135,7 +150,7 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
   // state layout per problem: m[W*5], v[W*5], partials[(W*5+1)*nblocks], loss, step
   std::vector<size_t> off(count);
   size_t bytes = 0;
-  long long class_blocks[wt::kFitClasses] = {};
+  long long rounds = 0;  // tiles per wavefront over all blocks
   for (uint32_t i = 0; i < count; ++i) {
     std::string why;
     if (!problem_ok(problems[i], &why)) {
@@ -143,10 +158,8 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
       return wt::ctx_fail(ctx, WT_ERR_INVALID_ARG, "problem " + std::to_string(i) + ": " + why);
     }
     const wt_fit_problem& p = problems[i];
-    const long long V = (long long)p.grid_side * p.grid_side;
-    const int cls = wt::fit_class((int)p.snapshots);
-    const long long per_block = (long long)wt::kFitThreads * wt::kFitPointsPerThread[cls];
-    const int nblocks = (int)((V + per_block - 1) / per_block);
+    const wt::FitBlocks fb = wt::fit_blocks((int)p.grid_side, (int)p.snapshots);
+    const int nblocks = fb.nblocks;
     const int np = (int)p.wave_count * 5;
     wt::FitDesc& d = f->host[i];
     d.spacing = p.spacing;
@@ -160,40 +173,46 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
     d.n = (int)p.grid_side;
     d.S = (int)p.snapshots;
     d.W = (int)p.wave_count;
+    d.tiles_per_block = fb.tiles_per_block;
+    d.blocks_per_strip = fb.blocks_per_strip;
     d.nblocks = nblocks;
-    d.block_offset = 0;  // set below, once the class sizes are known
     d.row_offset = f->total_rows;
     d.param_out_offset = f->total_params;
-    class_blocks[cls] += nblocks;
-    f->total_blocks += nblocks;
+    rounds += (long long)nblocks * (fb.tiles_per_block / wt::kFitWavefronts);
     f->total_rows += np + 1;
     f->total_params += np;
     off[i] = bytes;
     bytes += sizeof(float) * ((size_t)2 * np + (size_t)(np + 1) * nblocks + 1) + sizeof(int);
     bytes = (bytes + 255) & ~(size_t)255;
   }
-  // blocks grouped by snapshot class: class c occupies [class_begin[c], + class_blocks[c])
-  long long class_begin[wt::kFitClasses];
-  long long acc = 0;
+  // adjoint units by wave-count class, the longest first (the dispatcher starts
+  // workgroups in index order). A workgroup takes several parts of a strip where the batch
+  // has many more parts than the GPU has room for workgroups (256 CUs, one or two on
+  // each), so that setting the strip's tables up is paid for by several rounds of tiles.
+  const long long unit_rounds = std::min<long long>(16, std::max<long long>(1, rounds / 2048));
+  std::vector<wt::FitUnit> units;
+  long long unit_begin = 0;
   for (int c = 0; c < wt::kFitClasses; ++c) {
-    class_begin[c] = acc;
-    acc += class_blocks[c];
-    f->launch.class_begin[c] = class_begin[c];
-    f->launch.class_blocks[c] = class_blocks[c];
+    for (uint32_t i = 0; i < count; ++i) {
+      const wt::FitDesc& d = f->host[i];
+      if (wt::fit_class(d.W) != c) continue;
+      const int part_rounds = d.tiles_per_block / wt::kFitWavefronts;
+      const int per = (int)std::max<long long>(1, unit_rounds / part_rounds);
+      const int strips = d.nblocks / d.blocks_per_strip;
+      for (int st = 0; st < strips; ++st)
+        for (int b = 0; b < d.blocks_per_strip; b += per)
+          units.push_back(wt::FitUnit{(int)i, st, b, std::min(per, d.blocks_per_strip - b)});
+      if (units.size() >= (1ull << 31)) break;
+    }
+    std::stable_sort(units.begin() + unit_begin, units.end(), [&](const wt::FitUnit& x, const wt::FitUnit& y) {
+      return (long long)x.parts * f->host[x.problem].tiles_per_block >
+             (long long)y.parts * f->host[y.problem].tiles_per_block;
+    });
+    f->launch.class_begin[c] = unit_begin;
+    f->launch.class_blocks[c] = (long long)units.size() - unit_begin;
+    unit_begin = (long long)units.size();
   }
-  // within a class, problems with more waves (more work per block) come first: the
-  // dispatcher starts blocks in index order, so the costliest blocks start earliest
-  std::vector<uint32_t> order(count);
-  for (uint32_t i = 0; i < count; ++i) order[i] = i;
-  std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return f->host[a].W > f->host[b].W; });
-  long long class_next[wt::kFitClasses] = {};
-  for (uint32_t i : order) {
-    wt::FitDesc& d = f->host[i];
-    const int cls = wt::fit_class(d.S);
-    d.block_offset = class_begin[cls] + class_next[cls];
-    class_next[cls] += d.nblocks;
-  }
-  if (f->total_blocks >= (1ll << 31) || f->total_rows >= (1ll << 31)) {
+  if (units.size() >= (1ull << 31) || f->total_rows >= (1ll << 31)) {
     delete f;
     return wt::ctx_fail(ctx, WT_ERR_UNSUPPORTED, "batch too large for one launch");
   }
@@ -213,32 +232,31 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
     d.loss = d.partials + (size_t)(np + 1) * d.nblocks;
     d.step = reinterpret_cast<int*>(d.loss + 1);
   }
-  std::vector<int> maps((size_t)f->total_blocks + (size_t)f->total_rows);
+  std::vector<int> rows((size_t)f->total_rows);
   for (uint32_t i = 0; i < count; ++i) {
     const wt::FitDesc& d = f->host[i];
-    for (int b = 0; b < d.nblocks; ++b) maps[(size_t)d.block_offset + b] = (int)i;
-    for (int r = 0; r <= d.W * 5; ++r) maps[(size_t)f->total_blocks + d.row_offset + r] = (int)i;
+    for (int r = 0; r <= d.W * 5; ++r) rows[(size_t)d.row_offset + r] = (int)i;
   }
   e = hipMalloc(&f->d_desc, sizeof(wt::FitDesc) * count);
-  if (e == hipSuccess) e = hipMalloc(&f->d_maps, sizeof(int) * maps.size());
+  if (e == hipSuccess) e = hipMalloc(&f->d_units, sizeof(wt::FitUnit) * units.size());
+  if (e == hipSuccess) e = hipMalloc(&f->d_rows, sizeof(int) * rows.size());
   if (e == hipSuccess) e = hipMemcpy(f->d_desc, f->host.data(), sizeof(wt::FitDesc) * count, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(f->d_maps, maps.data(), sizeof(int) * maps.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess)
+    e = hipMemcpy(f->d_units, units.data(), sizeof(wt::FitUnit) * units.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(f->d_rows, rows.data(), sizeof(int) * rows.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemset(f->d_state, 0, bytes);
   if (e == hipSuccess) e = hipDeviceSynchronize();
   if (e != hipSuccess) {
     wt_status s = hip_err(ctx, e, "wt_fit_create");
-    if (f->d_desc) (void)hipFree(f->d_desc);
-    if (f->d_maps) (void)hipFree(f->d_maps);
-    (void)hipFree(f->d_state);
-    delete f;
+    wt_fit_destroy(f);
     return s;
   }
   f->launch.probs = f->d_desc;
-  f->launch.block_prob = f->d_maps;
-  f->launch.row_prob = f->d_maps + f->total_blocks;
+  f->launch.units = f->d_units;
+  f->launch.row_prob = f->d_rows;
   f->launch.total_rows = f->total_rows;
   // side streams (default priority, not synchronising with the null stream) and their
-  // fork / join events, for batches spanning several snapshot classes
+  // fork / join events, for batches spanning several wave-count classes
   int classes = 0;
   for (int c = 0; c < wt::kFitClasses; ++c) classes += f->launch.class_blocks[c] > 0;
   if (classes > 1) {
@@ -265,7 +283,8 @@ void wt_fit_destroy(wt_fit* f) {
   }
   if (f->launch.fork) (void)hipEventDestroy(f->launch.fork);
   if (f->d_desc) (void)hipFree(f->d_desc);
-  if (f->d_maps) (void)hipFree(f->d_maps);
+  if (f->d_units) (void)hipFree(f->d_units);
+  if (f->d_rows) (void)hipFree(f->d_rows);
   if (f->d_state) (void)hipFree(f->d_state);
   delete f;
 }
@@ -301,15 +320,14 @@ wt_status wt_fit_loss_grad_static(wt_ctx* ctx, const wt_fit_problem* p, float* d
   if (!ctx || !p || !d_grad) return WT_ERR_INVALID_ARG;
   std::string why;
   if (!problem_ok(*p, &why)) return wt::ctx_fail(ctx, WT_ERR_INVALID_ARG, why);
-  const long long V = (long long)p->grid_side * p->grid_side;
-  const int cls = wt::fit_class((int)p->snapshots);
-  const long long per_block = (long long)wt::kFitThreads * wt::kFitPointsPerThread[cls];
-  const long long nblocks = (V + per_block - 1) / per_block;
+  const int cls = wt::fit_class((int)p->wave_count);
+  const wt::FitBlocks fb = wt::fit_blocks((int)p->grid_side, (int)p->snapshots);
+  const long long nblocks = fb.nblocks;
   const int np = (int)p->wave_count * 5;
-  size_t off_maps = 0, off_state = 0, off_partials = 0;
-  const size_t need = static_fit_layout(np, (int)std::min<long long>(nblocks, 1 << 30), &off_maps, &off_state,
-                                        &off_partials);
-  if (nblocks >= (1 << 30) || need > kStaticFitScratchBytes)
+  size_t off_units = 0, off_rows = 0, off_partials = 0;
+  const size_t need =
+      std::max(static_fit_limit(*p), static_fit_layout(np, (int)nblocks, &off_units, &off_rows, &off_partials));
+  if (need > kStaticFitScratchBytes)
     return wt::ctx_fail(ctx, WT_ERR_INVALID_ARG,
                         "problem needs " + std::to_string(need) + " bytes of fixed scratch; the limit is " +
                             std::to_string(kStaticFitScratchBytes) + " (fewer grid points or waves, or wt_fit_create)");
@@ -328,7 +346,8 @@ wt_status wt_fit_loss_grad_static(wt_ctx* ctx, const wt_fit_problem* p, float* d
   d.g = p->gravity;
   d.target = p->target;
   d.params = p->params;
-  float* state = reinterpret_cast<float*>(b + off_state);
+  int* rows = reinterpret_cast<int*>(b + off_rows);
+  float* state = reinterpret_cast<float*>(rows + np + 1);
   d.adam_m = state;
   d.adam_v = state + np;
   d.loss = state + 2 * np;
@@ -337,22 +356,24 @@ wt_status wt_fit_loss_grad_static(wt_ctx* ctx, const wt_fit_problem* p, float* d
   d.n = (int)p->grid_side;
   d.S = (int)p->snapshots;
   d.W = (int)p->wave_count;
+  d.tiles_per_block = fb.tiles_per_block;
+  d.blocks_per_strip = fb.blocks_per_strip;
   d.nblocks = (int)nblocks;
-  d.block_offset = 0;
   d.row_offset = 0;
   d.param_out_offset = 0;
   const hipStream_t st = (hipStream_t)stream;
   wt::FitDesc* d_desc = reinterpret_cast<wt::FitDesc*>(b);
-  int* d_maps = reinterpret_cast<int*>(b + off_maps);
-  // the previous call's contents stay in the array: rewrite the descriptor and maps and
-  // clear the state words; every partial is overwritten by the adjoint launch
-  e = wt::launch_fit_setup_single(d, d_desc, d_maps, (size_t)nblocks + np + 1, reinterpret_cast<uint32_t*>(state),
-                                  2 * (size_t)np + 2, st);
+  wt::FitUnit* d_units = reinterpret_cast<wt::FitUnit*>(b + off_units);
+  // the previous call's contents stay in the array: rewrite the descriptor and units and
+  // clear the row map (problem 0) and the state words; every partial is overwritten by
+  // the adjoint launch
+  e = wt::launch_fit_setup_single(d, d_desc, d_units, (size_t)nblocks, reinterpret_cast<uint32_t*>(rows),
+                                  3 * (size_t)np + 3, st);
   if (e != hipSuccess) return hip_err(ctx, e, "fixed-scratch set-up launch");
   wt::FitLaunch L{};
   L.probs = d_desc;
-  L.block_prob = d_maps;
-  L.row_prob = d_maps + nblocks;
+  L.units = d_units;
+  L.row_prob = rows;
   L.class_begin[cls] = 0;
   L.class_blocks[cls] = nblocks;
   L.total_rows = np + 1;
@@ -390,10 +411,10 @@ wt_status wt_fit_phase_plan(const wt_fit_problem* p, uint64_t budget_bytes, uint
   const uint64_t V = (uint64_t)p->grid_side * p->grid_side;
   // (cos, sin) per snapshot x grid point x wave in FP32
   *phase_tensor_bytes = V * p->snapshots * p->wave_count * 8ull;
-  // Recomputing a phase costs 4 VALU ops per snapshot (one rotation) after one seed per
-  // wave; reading it back costs 8 bytes of HBM traffic, which is slower on MI355X at
-  // any size, so the kernels always recompute. The tensor size is reported so callers
-  // can see what storing would need against their budget.
+  // The kernels contract separable factors of (cos, sin), W (n + 64) values per row and
+  // column where the tensor has S n^2 W: nothing is gained by storing it at any size. The
+  // tensor size is reported so callers can see what storing would need against their
+  // budget.
   (void)budget_bytes;
   *recompute = 1;
   return WT_OK;
