@@ -232,7 +232,7 @@ def bench_batched_forward(torch, wt, scenes, frames=120, one_by_one=True):
     pos = torch.empty(V * 3, device=dev)
     nrm = torch.empty_like(pos)
     # each frame re-aims every patch from its camera on the device (the reference runs its
-    # projector every frame), then one launch per segment shape displaces all patches
+    # projector every frame), then one launch displaces all patches
     cams = torch.from_numpy(wt.camera_rows([s["camera"] for s in specs])).to(dev)
     amps = torch.full((len(specs),), 2.0, dtype=torch.float32, device=dev)
     stream = torch.cuda.Stream()
@@ -257,7 +257,7 @@ def bench_batched_forward(torch, wt, scenes, frames=120, one_by_one=True):
         batch.close()
         ctx.close()
         return dict(workload="batched forward: 512 patches, %d frames in one HIP graph (device projector and one "
-                             "launch per segment shape per frame)" % frames,
+                             "launch per frame)" % frames,
                     value=vw_frame * frames / wall, unit="vertex-waves/s", ms_per_frame=wall * 1e3 / frames)
     # the same frame as one plain launch per patch (no graph), for the batching gain
     params = [wt.water_params(wt.np_corners(p), s["camera"][4:7], s["N"], s["time"], 0.02, 0.05, 0.0, (0.3, 0.0))
@@ -278,7 +278,7 @@ def bench_batched_forward(torch, wt, scenes, frames=120, one_by_one=True):
     batched = vw_frame * frames / wall
     return dict(workload="batched forward: 512 patches (side 32-1024 log-uniform, 4-128 waves, own camera and t in "
                          "[0, 3600) s), %d frames in one HIP graph; per frame the device projector re-aims "
-                         "every patch, then one launch per segment shape displaces them" % frames,
+                         "every patch, then one launch displaces them" % frames,
                 value=batched, unit="vertex-waves/s", vertex_waves_per_frame=vw_frame,
                 vertices=V, ms_per_frame=wall * 1e3 / frames,
                 patches_per_shape={"%dx%d" % (sh[2] * sh[1], 64 // sh[2]): shapes.count(sh) for sh in set(shapes)},

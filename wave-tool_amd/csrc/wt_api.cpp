@@ -10,6 +10,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -567,8 +568,7 @@ struct wt_batch {
   std::vector<wt::PatchDesc> patches;
   wt::PatchDesc* d_patches = nullptr;
   wt::BatchUnit* d_units = nullptr;
-  long long shape_begin[wt::kBatchShapes] = {};
-  int shape_units[wt::kBatchShapes] = {};
+  long long units = 0;
   uint64_t vertices = 0;
   uint32_t max_wave_end = 0;
 };
@@ -633,29 +633,24 @@ static wt_status batch_create(wt_ctx* ctx, const wt_patch* patches, uint32_t cou
     b->max_wave_end = std::max<uint32_t>(b->max_wave_end, p.wave_offset + p.wave_count);
     max_n = std::max(max_n, p.gridLength);
   }
-  // units: one workgroup's segments of one patch, in that patch's segment shape
+  // units: one workgroup's segments of one patch, in that patch's segment shape; most
+  // expensive first, over all shapes: a unit covers 1024 vertices in each shape, so it
+  // costs about its patch's wave count
+  std::vector<uint32_t> order(count);
+  std::iota(order.begin(), order.end(), 0u);
+  std::stable_sort(order.begin(), order.end(),
+                   [&](uint32_t x, uint32_t y) { return b->patches[x].W > b->patches[y].W; });
   std::vector<wt::BatchUnit> units;
-  for (uint32_t i = 0; i < count; ++i) {
+  for (uint32_t i : order) {
     const wt::PatchDesc& d = b->patches[i];
-    const wt::LaunchShape& s = wt::kBatchShape[d.shape];
-    const long long groups = wt::forward_segment_groups(d.N, s);
+    const long long groups = wt::forward_segment_groups(d.N, wt::kBatchShape[d.shape]);
     for (long long gidx = 0; gidx < groups; ++gidx) units.push_back(wt::BatchUnit{(int)i, (int)gidx});
   }
-  // grouped by shape (one launch each), most expensive units first within a shape: a
-  // unit costs about its patch's wave count
-  auto shape_of = [&](const wt::BatchUnit& x) { return b->patches[x.patch].shape; };
-  std::stable_sort(units.begin(), units.end(), [&](const wt::BatchUnit& x, const wt::BatchUnit& y) {
-    if (shape_of(x) != shape_of(y)) return shape_of(x) < shape_of(y);
-    return b->patches[x.patch].W > b->patches[y.patch].W;
-  });
   if (units.size() >= (1ull << 31)) {
     delete b;
     return fail(ctx, WT_ERR_UNSUPPORTED, "batch too large: more than 2^31 workgroup units");
   }
-  for (size_t k = 0; k < units.size(); ++k) {
-    const int sh = shape_of(units[k]);
-    if (b->shape_units[sh]++ == 0) b->shape_begin[sh] = (long long)k;
-  }
+  b->units = (long long)units.size();
   hipError_t e = hipMalloc(&b->d_patches, sizeof(wt::PatchDesc) * count);
   if (e == hipSuccess) e = hipMalloc(&b->d_units, sizeof(wt::BatchUnit) * units.size());
   if (e == hipSuccess)
@@ -991,11 +986,11 @@ wt_status wt_water_displace_batched(wt_ctx* ctx, wt_batch* b, const wt_gerstner_
   a.nrm = out->normal;
   a.tan = out->tangent;
   a.bit = out->bitangent;
-  for (int sh = 0; sh < wt::kBatchShapes; ++sh) {
-    if (b->shape_units[sh] == 0) continue;
-    a.unit_begin = b->shape_begin[sh];
-    a.n_units = b->shape_units[sh];
-    hipError_t e = wt::launch_forward_batched(a, sh, st);
+  // one launch, unless the units pass the 2^32 threads that a launch may have
+  constexpr long long kMaxUnits = 1ll << 23;
+  for (a.unit_begin = 0; a.unit_begin < b->units; a.unit_begin += kMaxUnits) {
+    a.n_units = (int)std::min(kMaxUnits, b->units - a.unit_begin);
+    hipError_t e = wt::launch_forward_batched(a, st);
     if (e != hipSuccess) return hip_fail(ctx, e, "water_forward_batched_kernel launch");
   }
   return WT_OK;

@@ -44,20 +44,20 @@ int batch_shape_for(int N) {
   return pick;
 }
 
-hipError_t launch_forward_batched_t0(const BatchArgs& a, int shape, hipStream_t st);
-hipError_t launch_forward_batched_t1(const BatchArgs& a, int shape, hipStream_t st);
-hipError_t launch_forward_batched_t2(const BatchArgs& a, int shape, hipStream_t st);
-hipError_t launch_forward_batched_t3(const BatchArgs& a, int shape, hipStream_t st);
-hipError_t launch_forward_batched_t4(const BatchArgs& a, int shape, hipStream_t st);
+hipError_t launch_forward_batched_t0(const BatchArgs& a, hipStream_t st);
+hipError_t launch_forward_batched_t1(const BatchArgs& a, hipStream_t st);
+hipError_t launch_forward_batched_t2(const BatchArgs& a, hipStream_t st);
+hipError_t launch_forward_batched_t3(const BatchArgs& a, hipStream_t st);
+hipError_t launch_forward_batched_t4(const BatchArgs& a, hipStream_t st);
 
-hipError_t launch_forward_batched(const BatchArgs& a, int shape, hipStream_t st) {
+hipError_t launch_forward_batched(const BatchArgs& a, hipStream_t st) {
   if (a.n_units <= 0) return hipSuccess;
   switch (tex_mode(a.texels, a.tex_fmt, a.tex_wrap)) {
-    case kTexR32Repeat: return launch_forward_batched_t1(a, shape, st);
-    case kTexR32Mirror: return launch_forward_batched_t2(a, shape, st);
-    case kTexR8Repeat: return launch_forward_batched_t3(a, shape, st);
-    case kTexR8Mirror: return launch_forward_batched_t4(a, shape, st);
-    default: return launch_forward_batched_t0(a, shape, st);
+    case kTexR32Repeat: return launch_forward_batched_t1(a, st);
+    case kTexR32Mirror: return launch_forward_batched_t2(a, st);
+    case kTexR8Repeat: return launch_forward_batched_t3(a, st);
+    case kTexR8Mirror: return launch_forward_batched_t4(a, st);
+    default: return launch_forward_batched_t0(a, st);
   }
 }
 

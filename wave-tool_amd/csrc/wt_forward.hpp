@@ -527,36 +527,53 @@ __device__ __forceinline__ FwdParams patch_params(const BatchArgs& a, const Patc
   return p;
 }
 
-// Batched kernel over the patches of a batch that use segment shape kShape
-// (kBatchShape): workgroup b runs unit b (one workgroup's segments of one patch). The
-// units are sorted by cost, largest first, so the hardware dispatcher, which starts
-// workgroups in index order as slots free up, balances them like a longest-first work
-// queue, with no atomics: a device-wide unit counter serialises every fetch through one
-// address and measured twice as slow as this on a single 1024 x 1024, 64-wave patch. One
-// kernel per shape keeps each at its own register count and LDS size.
+// Batched kernel: workgroup b runs unit b (one workgroup's segments of one patch), in the
+// patch's segment shape (kBatchShape). The units are sorted by cost, largest first, so the
+// hardware dispatcher, which starts workgroups in index order as slots free up, balances
+// them like a longest-first work queue, with no atomics: a device-wide unit counter
+// serialises every fetch through one address and measured twice as slow as this on a
+// single 1024 x 1024, 64-wave patch. All shapes step K = 8 vertices per lane with the same
+// LDS size, and the branch over them costs no wavefront per SIMD (126 VGPRs, and the widest
+// shape alone takes 128), so one launch covers a batch. A launch per shape ran the shapes'
+// tails one after another: 24 patches of sides 32 to 160 (camera update and displacement)
+// took 33.3 us so and take 25.4; a batch of 512 large patches is VALU-bound and takes the
+// same time either way.
 template <int kTex, int kShape>
-__global__ __launch_bounds__(256) void water_forward_batched_kernel(BatchArgs a) {
+__device__ __forceinline__ void batched_unit(const BatchArgs& a, BatchUnit unit, void* lds) {
   constexpr int K = kBatchShape[kShape].steps, LC = kBatchShape[kShape].lanes_per_row;
   static_assert(kBatchShape[kShape].split == 2, "batched shapes pair two wavefronts per segment");
-  __shared__ SegShared<K, LC, 2> lds;
+  // the index is opaque per branch, so that no branch's part is hoisted above the switch,
+  // where it would be held in registers through the others' (138 VGPRs)
+  asm volatile("" : "+s"(unit.patch));
+  const PatchDesc pd = load_uniform(a.patches, unit.patch);
+  forward_segments<K, LC, 2, kTex>(patch_params(a, pd), (long long)unit.group, *static_cast<SegShared<K, LC, 2>*>(lds));
+}
+
+template <int kTex>
+__global__ __launch_bounds__(256, 4) void water_forward_batched_kernel(BatchArgs a) {
+  static_assert(kBatchShapes == 3, "one branch per shape below");
+  constexpr size_t kBytes =
+      cmax(cmax(sizeof(SegShared<kBatchShape[0].steps, kBatchShape[0].lanes_per_row, 2>),
+                sizeof(SegShared<kBatchShape[1].steps, kBatchShape[1].lanes_per_row, 2>)),
+           sizeof(SegShared<kBatchShape[2].steps, kBatchShape[2].lanes_per_row, 2>));
+  __shared__ alignas(16) unsigned char lds[kBytes];
   // the unit and patch tables do not change during the launch: read them through the
   // constant address space so they load with scalar loads into SGPRs (a vector load
   // would park the whole patch descriptor in VGPRs)
   const BatchUnit unit = load_uniform(a.units, a.unit_begin + (long long)blockIdx.x);
   const PatchDesc pd = load_uniform(a.patches, unit.patch);
   if (!pd.active) return;  // workgroup-uniform
-  forward_segments<K, LC, 2, kTex>(patch_params(a, pd), (long long)unit.group, lds);
+  switch (pd.shape) {
+    case 0: batched_unit<kTex, 0>(a, unit, lds); break;
+    case 1: batched_unit<kTex, 1>(a, unit, lds); break;
+    default: batched_unit<kTex, 2>(a, unit, lds); break;
+  }
 }
 
-// The batched kernel of one texture mode in segment shape `shape`, one workgroup per unit.
+// The batched kernel of one texture mode, one workgroup per unit.
 template <int kTex>
-hipError_t launch_batched_mode(const BatchArgs& a, int shape, hipStream_t st) {
-  const dim3 g((unsigned)a.n_units), b(256);
-  switch (shape) {
-    case 0: hipLaunchKernelGGL((water_forward_batched_kernel<kTex, 0>), g, b, 0, st, a); break;
-    case 1: hipLaunchKernelGGL((water_forward_batched_kernel<kTex, 1>), g, b, 0, st, a); break;
-    default: hipLaunchKernelGGL((water_forward_batched_kernel<kTex, 2>), g, b, 0, st, a); break;
-  }
+hipError_t launch_batched_mode(const BatchArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL((water_forward_batched_kernel<kTex>), dim3((unsigned)a.n_units), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 

@@ -66,7 +66,7 @@ struct BatchUnit {
 
 struct BatchArgs {
   const PatchDesc* patches;
-  const BatchUnit* units;  // every unit of the batch, grouped by segment shape
+  const BatchUnit* units;  // every unit of the batch
   long long unit_begin;    // this launch's units: [unit_begin, unit_begin + n_units)
   int n_units;
   double time_offset;  // added to every patch's time (frame clock)
@@ -127,9 +127,8 @@ hipError_t launch_projector(const ProjectorArgs& a, hipStream_t st);
 // Triangle index list of an n x n grid (n >= 2), 6 (n - 1)^2 entries, ids offset by base.
 hipError_t launch_grid_indices(uint32_t n, uint32_t base, uint32_t* out, hipStream_t st);
 
-// Launches the batched kernel of segment shape `shape` (kBatchShape), one workgroup per
-// unit of a.
-hipError_t launch_forward_batched(const BatchArgs& a, int shape, hipStream_t st);
+// Launches the batched kernel, one workgroup per unit of a.
+hipError_t launch_forward_batched(const BatchArgs& a, hipStream_t st);
 
 // Fragment stage (wt_water_shade): the water program's fragment shader over a
 // per-pixel fragment buffer. RGBA8 images are read as one 32-bit word per texel.
