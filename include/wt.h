@@ -166,7 +166,7 @@ wt_status wt_camera_matrices(const wt_camera* cam, double view[16], double proj[
 wt_status wt_projector_corners(const wt_camera* cam, float displaceable_amplitude, double corners[4][4]);
 
 /* The same projector (src/render-engine.cpp:797-1042) on the device for many
- * cameras, one thread per camera, in double. d_cameras: count wt_camera structs;
+ * cameras, in double. d_cameras: count wt_camera structs;
  * d_amplitudes: count slab half-heights. Writes d_corners[count][4][4] (NaN for a
  * camera without corners) and d_status[count] (WT_OK, WT_ERR_NO_INTERSECTION,
  * WT_ERR_DEGENERATE, or WT_ERR_INVALID_ARG for a camera wt_projector_corners would

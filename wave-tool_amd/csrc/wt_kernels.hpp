@@ -110,7 +110,7 @@ constexpr LaunchShape kBatchShape[kBatchShapes] = {{2, 8, 64, 64}, {2, 8, 32, 64
 // shape).
 int batch_shape_for(int N);
 
-// Device projector: one thread per camera runs the reference projector in FP64.
+// Device projector: the reference projector in FP64 for every camera.
 // corners (count x 16, row = corner BL, TL, BR, TR) and status (wt_status per camera)
 // may be null; with patches set, patch i takes camera i's corner algebra and camera
 // position and is switched off when its status is not WT_OK.

@@ -1,6 +1,6 @@
 // Camera and projected-grid projector of the water stage, in double precision, compiled
-// for both the host (wt_projector_corners, the host water stage) and the device (one
-// thread per camera for batched patches).
+// for both the host (wt_projector_corners, the host water stage) and the device (batched
+// patches).
 //
 // Camera restates src/camera.cpp:40-146; projector_corners restates the water block
 // of RenderEngine::render, src/render-engine.cpp:797-1042, with the reference's
@@ -229,7 +229,10 @@ struct NdcBounds {
 
   WT_HD void add_point(const Mat4& pvp, const Vec3& p) {
     const Vec4 q = mat_apply(pvp, Vec4{p.x, 0.0, p.z, 1.0});
-    const double nx = q.x / q.w, ny = q.y / q.w;
+    add_ndc(q.x / q.w, q.y / q.w);
+  }
+
+  WT_HD void add_ndc(double nx, double ny) {
     if (count++ == 0) {
       xmin = xmax = nx;
       ymin = ymax = ny;
