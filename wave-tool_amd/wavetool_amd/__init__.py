@@ -94,7 +94,8 @@ def water_params(corners, cam_pos, N, time, sample_scale=0.0, displacement_scale
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """Device address for a void* argument or field (ctypes converts the integer)."""
+    return None if t is None else t.data_ptr()
 
 
 def shade_params(uniforms):
@@ -124,36 +125,78 @@ def _check_min_array(t, dtype, numel, name):
                          (name, dtype, numel, t.dtype, tuple(t.shape)))
 
 
-def _check_waves(waves, count):
-    import torch
-    if count and (waves is None or waves.dim() != 2 or waves.shape[1] != 8 or waves.shape[0] < count):
-        raise ValueError("waves: need a (>= %d, 8) tensor, got %s" % (count, None if waves is None
-                                                                         else tuple(waves.shape)))
+def _check_waves(waves, count, f32):
     if count:
-        _check_min_array(waves, torch.float32, count * 8, "waves")
+        shape = None if waves is None else waves.shape
+        if shape is None or len(shape) != 2 or shape[1] != 8 or shape[0] < count:
+            raise ValueError("waves: need a (>= %d, 8) tensor, got %s" % (count, None if waves is None
+                                                                             else tuple(waves.shape)))
+        _check_min_array(waves, f32, count * 8, "waves")
+
+
+def _vertex_buffers(n3, pos, nrm, tan, bit, f32):
+    """wt_vertex_buffers over float32 tensors of at least n3 elements; pos and nrm are required."""
+    if pos is None:
+        raise ValueError("pos is required")
+    _check_min_array(pos, f32, n3, "pos")
+    if nrm is None:
+        raise ValueError("nrm is required")
+    _check_min_array(nrm, f32, n3, "nrm")
+    if tan is not None:
+        _check_min_array(tan, f32, n3, "tan")
+    if bit is not None:
+        _check_min_array(bit, f32, n3, "bit")
+    return VertexBuffers(pos.data_ptr(), nrm.data_ptr(), _ptr(tan), _ptr(bit))
 
 
 def _heightmap(heightmap, hm_format, hm_wrap):
-    """wt_heightmap over a 2-D device tensor whose dtype matches the texel format
-    (uint8 for WT_TEXEL_R8_UNORM, float32 for WT_TEXEL_R32F)."""
-    import torch
+    """Pointer to a wt_heightmap over a 2-D device tensor whose dtype matches the texel
+    format (uint8 for WT_TEXEL_R8_UNORM, float32 for WT_TEXEL_R32F), or None."""
     if heightmap is None:
         return None
-    if heightmap.dim() != 2:
-        raise ValueError("heightmap: need a 2-D (height, width) tensor, got %s" % (tuple(heightmap.shape),))
-    want = {WT_TEXEL_R8_UNORM: torch.uint8, WT_TEXEL_R32F: torch.float32}.get(hm_format)
-    if want is None:
+    import torch
+    shape = heightmap.shape
+    if len(shape) != 2:
+        raise ValueError("heightmap: need a 2-D (height, width) tensor, got %s" % (tuple(shape),))
+    if hm_format == WT_TEXEL_R32F:
+        want = torch.float32
+    elif hm_format == WT_TEXEL_R8_UNORM:
+        want = torch.uint8
+    else:
         raise ValueError("heightmap: unknown texel format %r" % (hm_format,))
-    h, w = heightmap.shape
+    h, w = shape
     _check_array(heightmap, want, h * w, "heightmap")
-    return Heightmap(heightmap.data_ptr(), w, h, hm_format, hm_wrap)
+    return ctypes.byref(Heightmap(heightmap.data_ptr(), w, h, hm_format, hm_wrap))
+
+
+_current = None  # torch's is_initialized, current device and current stream handle, once loaded
 
 
 def _stream(stream):
-    if stream is None:
+    """Handle of a torch stream, or of the current stream of the current device.
+    torch.cuda.current_stream() builds a Stream object on each call: 2.7 us of a 10 us
+    pass over a 128 x 128 grid, where the handle alone takes 0.2."""
+    if stream is not None:
+        return stream.cuda_stream
+    global _current
+    if _current is None:
         import torch
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+        torch.cuda.current_stream()  # initialises the runtime, or raises
+        _current = (torch.cuda.is_initialized, torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream)
+    is_initialized, device, raw_stream = _current
+    if not is_initialized():  # a forked child of an initialised process
+        import torch
+        return torch.cuda.current_stream().cuda_stream
+    return raw_stream(device())
+
+
+_F16 = ctypes.c_float * 16
+
+
+def _column_major(m):
+    """A 4x4 matrix m[r][c] as column-major floats."""
+    import numpy as np
+    return _F16(*np.asarray(m, dtype=np.float64).T.reshape(-1).tolist())
 
 
 class Context:
@@ -218,19 +261,15 @@ class Context:
         """waves: device tensor (W, 8) float32; pos/nrm/tan/bit: device float tensors
         with gridLength^2 * 3 elements; heightmap: device tensor (H, W) or None."""
         import torch
+        f32 = torch.float32
         W = int(waves.shape[0]) if wave_count is None else int(wave_count)
-        _check_waves(waves, W)
-        n3 = int(params.gridLength) ** 2 * 3
-        for name, t in (("pos", pos), ("nrm", nrm), ("tan", tan), ("bit", bit)):
-            if t is not None or name in ("pos", "nrm"):
-                if t is None:
-                    raise ValueError("%s is required" % name)
-                _check_min_array(t, torch.float32, n3, name)
-        vb = VertexBuffers(_ptr(pos), _ptr(nrm), _ptr(tan), _ptr(bit))
+        _check_waves(waves, W, f32)
+        vb = _vertex_buffers(params.gridLength ** 2 * 3, pos, nrm, tan, bit, f32)
         hm = _heightmap(heightmap, hm_format, hm_wrap)
-        st = lib().wt_water_displace(self.handle, ctypes.byref(params), _ptr(waves) if W else None, W,
-                                     ctypes.byref(hm) if hm is not None else None, ctypes.byref(vb), _stream(stream))
-        self._check(st)
+        st = lib().wt_water_displace(self.handle, ctypes.byref(params), waves.data_ptr() if W else None, W, hm,
+                                     ctypes.byref(vb), _stream(stream))
+        if st:
+            self._check(st)
 
     def varyings(self, params, view_projection, view_only_yaw, pos, nrm, vertex_count, clip=None, ndc0=None,
                  view=None, nview=None, sample=None, heightmap=None, hm_format=WT_TEXEL_R32F, hm_wrap=WT_WRAP_REPEAT,
@@ -238,22 +277,20 @@ class Context:
         """The water program's varyings from positions / normals (wt_vertex_varyings).
         Matrices: 4x4 arrays in the usual row / column indexing (m[r][c]); they are
         passed column-major as the reference uploads them."""
-        import numpy as np
         import torch
         n = int(vertex_count)
+        f32 = torch.float32
         for name, t, k in (("pos", pos, 3), ("nrm", nrm, 3), ("clip", clip, 4), ("ndc0", ndc0, 2), ("view", view, 3),
                            ("nview", nview, 3), ("sample", sample, 1)):
             if t is not None:
-                _check_min_array(t, torch.float32, n * k, name)
-        f16 = ctypes.c_float * 16
-        vp = f16(*[float(v) for v in np.asarray(view_projection, dtype=np.float64).T.reshape(-1)])
-        vy = f16(*[float(v) for v in np.asarray(view_only_yaw, dtype=np.float64).T.reshape(-1)])
+                _check_min_array(t, f32, n * k, name)
+        vp, vy = _column_major(view_projection), _column_major(view_only_yaw)
         out = VaryingBuffers(_ptr(clip), _ptr(ndc0), _ptr(view), _ptr(nview), _ptr(sample))
         hm = _heightmap(heightmap, hm_format, hm_wrap)
-        st = lib().wt_vertex_varyings(self.handle, ctypes.byref(params), ctypes.byref(hm) if hm is not None else None,
-                                      vp, vy, _ptr(pos), _ptr(nrm), int(vertex_count), ctypes.byref(out),
-                                      _stream(stream))
-        self._check(st)
+        st = lib().wt_vertex_varyings(self.handle, ctypes.byref(params), hm, vp, vy, _ptr(pos), _ptr(nrm), n,
+                                      ctypes.byref(out), _stream(stream))
+        if st:
+            self._check(st)
 
     def set_launch_config(self, wave_split=0, steps=0, lanes_per_row=0, wave_chunk=0):
         cfg = LaunchConfig(wave_split, steps, lanes_per_row, wave_chunk)
@@ -360,19 +397,15 @@ class Batch:
     def displace(self, waves, pos, nrm, tan=None, bit=None, heightmap=None, hm_format=WT_TEXEL_R32F,
                  hm_wrap=WT_WRAP_REPEAT, time_offset=0.0, stream=None):
         import torch
-        _check_waves(waves, int(waves.shape[0]))
-        n3 = int(self.vertices) * 3
-        for name, t in (("pos", pos), ("nrm", nrm), ("tan", tan), ("bit", bit)):
-            if t is not None or name in ("pos", "nrm"):
-                if t is None:
-                    raise ValueError("%s is required" % name)
-                _check_min_array(t, torch.float32, n3, name)
-        vb = VertexBuffers(_ptr(pos), _ptr(nrm), _ptr(tan), _ptr(bit))
+        f32 = torch.float32
+        W = int(waves.shape[0])
+        _check_waves(waves, W, f32)
+        vb = _vertex_buffers(int(self.vertices) * 3, pos, nrm, tan, bit, f32)
         hm = _heightmap(heightmap, hm_format, hm_wrap)
-        st = lib().wt_water_displace_batched(self.ctx.handle, self.handle, _ptr(waves), int(waves.shape[0]),
-                                             ctypes.byref(hm) if hm is not None else None, ctypes.byref(vb),
+        st = lib().wt_water_displace_batched(self.ctx.handle, self.handle, waves.data_ptr(), W, hm, ctypes.byref(vb),
                                              float(time_offset), _stream(stream))
-        self.ctx._check(st)
+        if st:
+            self.ctx._check(st)
 
     def set_cameras(self, cameras, amplitudes, status=None, stream=None):
         """Re-aim every patch from its own camera on the device (wt_batch_set_cameras):
