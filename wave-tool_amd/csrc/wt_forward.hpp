@@ -467,6 +467,10 @@ __device__ __forceinline__ void forward_segments(const FwdParams& p, long long s
     __syncthreads();
     xchg_put<K, KS>(acc, sh.xchg(grp, sid), lane);
     __syncthreads();
+    // the second wavefront of a pair finishes the upper half of the segment's columns: past
+    // the grid's edge there is nothing to sample or store (513 x 513, 4 waves, per launch in a graph: 7.7 us with
+    // that half's epilogue, 7.1 without)
+    if (back && col_base + KS * LC >= p.N) return;
     xchg_finish<K, KS>(acc, sh.xchg(grp, sid ^ 1), lane, fin);
   } else {
 #pragma unroll
