@@ -80,3 +80,31 @@ def test_non_finite_target_reaches_loss_and_gradient(torch_cuda, wtctx, bad):
     assert not np.isfinite(loss)
     # dQ sums the x and z residuals alone; every other derivative takes the y residual
     assert not np.isfinite(g[:, [0, 1, 2, 4]]).any()
+
+
+# (n, S) whose 16-pair tiles are cut into parts of 1, 2, 4 and 8 tiles, at the last size of each rule and the next
+PARTS = [(64, 64, 16), (128, 32, 16), (129, 32, 20), (181, 20, 33), (182, 20, 100), (256, 16, 64), (257, 17, 8),
+         (360, 16, 12), (420, 24, 5)]
+
+
+@pytest.mark.parametrize("n,S,W", [(n, min(S, 32), W) for n, S, W in PARTS])
+def test_parts_of_a_small_problem(torch_cuda, wtctx, n, S, W):
+    """Against the oracle, and bit for bit the same when the problem's parts share workgroups side by side in a batch."""
+    torch = torch_cuda
+    print("[case] fit parts n=%d S=%d W=%d" % (n, S, W), flush=True)
+    params, target = problem(7100 + n + S, n, S, W)
+    loss, g, ref_loss, ref = evaluate(torch, wtctx, n, S, W, params, target)
+    assert abs(loss - ref_loss) <= LOSS_TOL * ref_loss
+    assert np.abs(g - ref).max() <= GRAD_TOL * np.abs(ref).max()
+    dev = torch.device("cuda")
+    x0 = -0.25 * (n - 1)
+    tt = torch.from_numpy(np.ascontiguousarray(target, dtype=np.float32)).to(dev)
+    tp = torch.from_numpy(np.ascontiguousarray(params, dtype=np.float32)).to(dev)
+    for count in (3, 40):
+        fit = wt.Fit(wtctx, [wt.fit_problem(n, S, W, 0.5, x0, x0, 0.0, 0.25, tt, tp)] * count)
+        grad, losses = torch.zeros(count * W * 5, device=dev), torch.zeros(count, device=dev)
+        fit.loss_grad(grad, losses)
+        torch.cuda.synchronize()
+        fit.close()
+        assert torch.equal(grad.cpu(), torch.from_numpy(g.astype(np.float32)).reshape(-1).repeat(count)), count
+        assert (losses == loss).all(), count

@@ -37,20 +37,24 @@
 // What bounds it: VALU issue and the matrix cores together, which do not overlap on one
 //   SIMD (two wavefronts of one SIMD, one issuing only matrix instructions and one only
 //   FMAs, take the sum of their times): per tile of 64 waves about 1300 VALU instructions
-//   and 216 matrix instructions of 16 cycles. 512^2 x 16 x 32: 18 us (62 us with FP32
-//   recurrences over the snapshots on the VALU); the 256-problem batch 1.25 ms (3.6 ms).
+//   and 216 matrix instructions of 16 cycles. 512^2 x 16 x 32: 17 us (62 us with FP32
+//   recurrences over the snapshots on the VALU); the 256-problem batch 1.21 ms (3.6 ms).
 //   Two wavefronts per SIMD at up to 256 VGPRs: a 32-column strip at three or four
 //   wavefronts repeats P, B and the sums per point (1.7 ms), and a spilled register is a
 //   round trip to cold scratch memory (5 us per workgroup).
-// reduce_adam_kernel: one workgroup per (problem, parameter row): fixed-order sum of
-//   the block partials, scaling to the mean misfit, and either an Adam step on the
-//   parameter or a plain gradient / loss write-out.
-// Both kernels find their problem through a block (row) -> problem map built at
+// reduce_adam_kernel: one workgroup per 16 parameter rows of a problem: fixed-order sum of
+//   the block partials in FP64, scaling to the mean misfit, and either an Adam step on the
+//   parameters or a plain gradient / loss write-out. Bound by its memory round trips: the
+//   rows are consecutive in memory and 64 parts are read side by side, so a sum over 256
+//   parts is one round of loads (a workgroup per row took 58 us for the
+//   256-problem batch, 24 so).
+// Both kernels find their problem through a unit (reduce block) -> problem map built at
 // creation, so one launch per wave-count class covers a whole batch; a single problem is
 // a table of one. A problem's blocks and the order of every sum depend on the problem
 // alone, so a batch repeats the bits of its problems run one by one.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
 #include <utility>
 
 #include "wt_fit.hpp"
@@ -281,6 +285,19 @@ __device__ __forceinline__ void load_targets(const FitDesc& P, bool whole, bool 
   }
 }
 
+// Reads one float of nearly every cache line of a tile's runs of 64 columns (16 runs of
+// 768 bytes, eight reads 108 bytes apart each), which brings them to the L2 ahead of
+// load_targets: issued before the set-up, whose tables need no memory, 512^2 x 16 x 32
+// takes 21.1 us where it took 22.7. For every tile ahead of its time it was slower.
+__device__ __forceinline__ void touch_targets(const FitDesc& P, int strip, int tile, int lane, float& a, float& b) {
+  const uint32_t pairs = (uint32_t)P.n * (uint32_t)P.S, q = min((uint32_t)tile * 16u + (uint32_t)(lane & 15), pairs - 1u);
+  const uint32_t j = q / (uint32_t)P.S, sn = q - j * (uint32_t)P.S;
+  const int col0 = max(0, min(strip * kStrip, P.n - kStrip)), last = 3 * (P.n - col0) - 1;
+  const float* t = P.target + 3 * ((size_t)sn * (size_t)P.n * (size_t)P.n + (size_t)j * (size_t)P.n + (size_t)col0);
+  a = t[min(27 * (lane >> 4), last)];
+  b = t[min(27 * (lane >> 4) + 108, last)];
+}
+
 // One run through the wavefront's LDS buffer: from 64-byte pieces of every pair to lane
 // g's twelve floats at 12 * column group `at`.
 __device__ __forceinline__ void unshuffle(float* run, int n16, int g, int at, float (&v)[12]) {
@@ -330,7 +347,9 @@ __device__ __forceinline__ void fit_tiles(const FitDesc& P, const FitUnit& unit,
   float sq = 0.0f;
 
 
-  int part = unit.part, part_end = first + P.tiles_per_block;
+  // a round of the parts of a workgroup: one part, or as many side by side as it has
+  // wavefronts for (parts of fewer tiles than wavefronts, powers of two)
+  int part = unit.strip * P.blocks_per_strip + unit.part, part_end = first + max(P.tiles_per_block, NW);
 #pragma unroll 1
   for (int base = first; base < end; base += NW) {
     const int tile = base + wid;
@@ -600,22 +619,36 @@ __device__ __forceinline__ void fit_tiles(const FitDesc& P, const FitUnit& unit,
     if (lane == 63) sh.loss[wid] = lsum;
     sq = 0.0f;
     __syncthreads();
-    const int part_index = unit.strip * P.blocks_per_strip + part;
-    if (tid < P.W) {
+    const int waves_per = min(P.tiles_per_block, NW), side_by = NW >> __builtin_ctz(waves_per);
+    const int wave_rows = (P.W + 63) >> 6;
+#pragma unroll 1
+    for (int it = wid; it < side_by * wave_rows; it += NW) {
+      int wi = lane;
+      asm volatile("" : "+v"(wi));  // keeps this block's addresses out of the tile loop's live registers
+      const int mine = wave_rows > 1 ? it >> 1 : it;
+      if (wave_rows > 1) wi += 64 * (it & 1);
+      const int w0 = mine * waves_per;
+      if (part_end - max(P.tiles_per_block, NW) + w0 >= end || wi >= P.W) continue;  // no such part
       double v[8];
+      auto sum_waves = [&](auto whole) {  // the part's wavefronts, all loads in flight together
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float2 t = sh.sums[0][tid >> 4][16 * r + (tid & 15)];
-        for (int i = 1; i < NW; ++i) {
-          const float2 u = sh.sums[i][tid >> 4][16 * r + (tid & 15)];
-          t.x += u.x;
-          t.y += u.y;
+        for (int r = 0; r < 4; ++r) {
+          const float2* from = &sh.sums[whole ? 0 : w0][wi >> 4][16 * r + (wi & 15)];
+          float2 t = *from;
+#pragma unroll
+          for (int i = 1; i < (whole ? NW : NW / 2); ++i) {
+            const float2 u = from[(whole || i < waves_per ? i : 0) * (KMAX * 64)];
+            t.x += whole || i < waves_per ? u.x : 0.0f;
+            t.y += whole || i < waves_per ? u.y : 0.0f;
+          }
+          const int k = ((r & 1) << 1) | (r >> 1);
+          v[k] = (double)t.x;
+          v[4 + k] = (double)t.y;
         }
-        const int k = ((r & 1) << 1) | (r >> 1);
-        v[k] = (double)t.x;
-        v[4 + k] = (double)t.y;
-      }
-      const FitWaveGrad w = sh.grad[tid];
+      };
+      if (waves_per == NW) sum_waves(std::true_type{});
+      else sum_waves(std::false_type{});
+      const FitWaveGrad w = sh.grad[wi];
       // sums of r . dd/dtheta: plain, times t, times the world x and z
       const double A = w.A, Dx = w.Dx, Dz = w.Dz;
       const double g0 = A * v[3], gt = A * (P.t0 * v[3] + P.dt * v[4]);
@@ -624,19 +657,19 @@ __device__ __forceinline__ void fit_tiles(const FitDesc& P, const FitUnit& unit,
       const double sec = Dx * v[0] + Dz * v[1], sepc = Dx * v[1] - Dz * v[0];
       const float out[5] = {(float)(w.Q * sec + v[2]), (float)-(w.wL * (Dx * gx + Dz * gz) + w.om2L * gt),
                             (float)(w.w * (Dx * gz - Dz * gx) + w.Q * A * sepc), (float)(A * sec), (float)g0};
-      float* o = P.partials + (size_t)(5 * tid) * P.nblocks + part_index;
+      float* o = P.partials + (size_t)(part + mine) * (5 * P.W + 1);
 #pragma unroll
-      for (int k = 0; k < 5; ++k) o[(size_t)k * P.nblocks] = out[k];
-    }
-    if (tid == 0) {
-      float t = sh.loss[0];
-      for (int i = 1; i < NW; ++i) t += sh.loss[i];
-      P.partials[(size_t)(5 * P.W) * P.nblocks + part_index] = t;
+      for (int k = 0; k < 5; ++k) o[5 * wi + k] = out[k];
+      if (wi == 0) {
+        float t = sh.loss[w0];
+        for (int i = w0 + 1; i < w0 + waves_per; ++i) t += sh.loss[i];
+        o[5 * P.W] = t;
+      }
     }
     __syncthreads();  // the sums have been read
     for (int kc = 0; kc < chunks; ++kc) sh.sums[wid][kc][lane] = make_float2(0.0f, 0.0f);
-    ++part;
-    part_end += P.tiles_per_block;
+    part += side_by;
+    part_end += max(P.tiles_per_block, NW);
   }
 }
 
@@ -653,14 +686,19 @@ void adjoint_kernel(const FitDesc* __restrict__ probs, const FitUnit* __restrict
   if (bump_step && unit.strip == 0 && unit.part == 0 && tid == 0) P.step[0] += 1;  // Adam step of this iteration
   const int chunks = (P.W + 15) >> 4, padded = 16 * chunks;
 
-  // ---- the waves' constants, one thread per wave
+  // ---- the waves' constants, one thread per wave; the parameters' loads first, so that
+  // they are not waited for behind the targets'
+  const float* pr = P.params + 5 * min(tid, P.W - 1);
+  const float p0 = pr[0], p1 = pr[1], p2 = pr[2], p3 = pr[3], p4 = pr[4];
+  float touch_a, touch_b;
+  const int tile = P.tiles_per_block * unit.part + min(tid >> 6, P.tiles_per_block * unit.parts - 1);
+  touch_targets(P, unit.strip, min(tile, (P.n * P.S - 1) >> 4), tid & 63, touch_a, touch_b);
   if (tid == 0) sh.max = 0;
   __syncthreads();
   FitWaveLds wv{};
   float bx = 0.0f, by = 0.0f, bz = 0.0f;
   if (tid < P.W) {
-    const float* pr = P.params + 5 * tid;
-    const double A = pr[0], L = pr[1] > 1e-3f ? pr[1] : 1e-3f, al = pr[2], Q = pr[3], ph0 = pr[4];
+    const double A = p0, L = p1 > 1e-3f ? p1 : 1e-3f, al = p2, Q = p3, ph0 = p4;
     const double w = kTwoPi / L, om = sqrt(P.g * w);
     double sa, ca;
     sincos(al, &sa, &ca);
@@ -731,6 +769,7 @@ void adjoint_kernel(const FitDesc* __restrict__ probs, const FitUnit* __restrict
       *reinterpret_cast<float2*>(&sh.time[sn * (2 * padded + 4) + 2 * wi]) = make_float2(cv, sv);
     }
     __syncthreads();
+    asm volatile("" ::"v"(touch_a), "v"(touch_b));  // the touches are over
     fit_tiles<true>(P, unit, sh, chunks, coef_exp);
   } else {
     __syncthreads();
@@ -739,37 +778,48 @@ void adjoint_kernel(const FitDesc* __restrict__ probs, const FitUnit* __restrict
 }
 
 __global__ __launch_bounds__(kReduceThreads) void reduce_adam_kernel(const FitDesc* __restrict__ probs,
-                                                                  const int* __restrict__ row_prob, FitAdam adam,
+                                                                  const int* __restrict__ reduce_prob, FitAdam adam,
                                                                   int mode, float* __restrict__ grad_out,
                                                                   float* __restrict__ loss_out) {
-  static_assert(kReduceThreads == 256, "the final sum reads four wavefront partials");
-  __shared__ float s[kReduceThreads / 64];
-  const int s_prob = load_uniform(row_prob, (long long)blockIdx.x);
-  const FitDesc P = load_uniform(probs, s_prob);
-  const int row = (int)(blockIdx.x - P.row_offset);
+  constexpr int kSide = kReduceThreads / kReduceRows;  // parts read side by side
+  __shared__ double s[kReduceThreads / 64][kReduceRows];
+  const int prob = load_uniform(reduce_prob, (long long)blockIdx.x);
+  const FitDesc P = load_uniform(probs, prob);
+  const int r = threadIdx.x & (kReduceRows - 1), side = threadIdx.x / kReduceRows;
+  const int row = (int)(blockIdx.x - P.reduce_offset) * kReduceRows + r;
   const int nparam = P.W * 5;
   // the row's Adam state, loaded while the partials are summed (a kernel this short is
   // bound by its chain of memory round trips)
   float m_old = 0.0f, v_old = 0.0f, p_old = 0.0f;
   int t = 0;
-  if (threadIdx.x == 0 && mode != 0 && row != nparam) {
+  if (side == 0 && mode != 0 && row < nparam) {
     m_old = P.adam_m[row];
     v_old = P.adam_v[row];
     p_old = P.params[row];
     t = P.step[0];
   }
-  const float* src = P.partials + (size_t)row * P.nblocks;
-  float acc = 0.0f;
-  for (int b = threadIdx.x; b < P.nblocks; b += blockDim.x) acc += src[b];
-  // fixed order: per wavefront by DPP, then the wavefronts in index order
-  acc = wave_sum63(acc);
-  if ((threadIdx.x & 63) == 63) s[threadIdx.x >> 6] = acc;
+  const float* src = P.partials + min(row, nparam);
+  const size_t stride = (size_t)nparam + 1;
+  double acc = 0.0;
+  for (int b = side; b < P.nblocks; b += 4 * kSide) {
+    float v[4];  // four loads in flight
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = src[(size_t)min(b + k * kSide, P.nblocks - 1) * stride];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc += b + k * kSide < P.nblocks ? (double)v[k] : 0.0;
+  }
+  // fixed order: a wavefront's parts, then the wavefronts in index order
+#pragma unroll
+  for (int d = kReduceRows; d < 64; d *= 2) acc += __shfl_xor(acc, d);
+  if ((threadIdx.x & 63) < kReduceRows) s[threadIdx.x >> 6][r] = acc;
   __syncthreads();
-  if (threadIdx.x != 0) return;
-  const double inv = 1.0 / ((double)P.S * (double)P.n * (double)P.n);
-  const float total = (float)((double)(((s[0] + s[1]) + s[2]) + s[3]) * inv);
+  if (side != 0 || row > nparam) return;
+  double sum = s[0][r];
+#pragma unroll
+  for (int i = 1; i < kReduceThreads / 64; ++i) sum += s[i][r];
+  const float total = (float)(sum * (1.0 / ((double)P.S * (double)P.n * (double)P.n)));
   if (row == nparam) {  // loss row
-    if (loss_out) loss_out[s_prob] = total;
+    if (loss_out) loss_out[prob] = total;
     P.loss[0] = total;
     return;
   }
@@ -948,7 +998,7 @@ hipError_t launch_fit_iteration(const FitLaunch& L, const FitAdam& adam, int mod
       if ((e = hipStreamWaitEvent(st, L.join[j], 0)) != hipSuccess) return e;
     }
   }
-  hipLaunchKernelGGL(reduce_adam_kernel, dim3((unsigned)L.total_rows), dim3(kReduceThreads), 0, st, L.probs, L.row_prob,
+  hipLaunchKernelGGL(reduce_adam_kernel, dim3((unsigned)L.reduce_blocks), dim3(kReduceThreads), 0, st, L.probs, L.reduce_prob,
                      adam, mode, grad_out, loss_out);
   return hipGetLastError();
 }

@@ -12,7 +12,10 @@ namespace wt {
 
 constexpr int kFitMaxWaves = 128;
 constexpr int kFitMaxSnapshots = 32;
-constexpr int kReduceThreads = 256;
+// The reduction: blocks of 16 rows (parameters, and the loss), 16 wavefronts of four parts
+// each side by side.
+constexpr int kReduceRows = 16, kReduceThreads = 1024;
+inline int reduce_blocks(int W) { return (5 * W + 1 + kReduceRows - 1) / kReduceRows; }
 // Wave-count classes W <= 64 and W <= 128: the chunks of 16 waves the adjoint kernel's LDS
 // has room for. From 65 waves on the time table does not fit beside the rest.
 constexpr int kFitClasses = 2;
@@ -26,12 +29,19 @@ struct FitBlocks {
 };
 inline FitBlocks fit_blocks(int n, int S) {
   const long long strips = (n + 63) / 64, tiles = ((long long)n * S + 15) / 16;
-  // enough tiles per wavefront to pay for a block's set-up, unless the problem is too
-  // small to fill the GPU's wavefronts that way
-  long long per_wave = (strips * tiles + 2047) / 2048;
-  if (per_wave > 8) per_wave = 8;
+  // enough tiles per wavefront to pay for a block's set-up; a problem too small to fill
+  // the GPU's wavefronts that way is cut into parts of 4, 2 or 1 tiles, about one for each
+  // CU, and each tile then has more of a CU's load path to itself: the eight tiles of a
+  // workgroup took 3.5 us to fetch on one CU (64 x 64, 8 snapshots, 16 waves: 14.0 us an
+  // iteration with 4 parts of 8 tiles, 11.3 with 32 of one; 256 x 256, 16 snapshots, 64
+  // waves: 23.0 with 128 of 8, 19.5 with 256 of 4)
+  const long long total = strips * tiles;
+  long long per_block = (total + 2047) / 2048 * kFitWavefronts;
+  if (per_block > 8 * kFitWavefronts) per_block = 8 * kFitWavefronts;
+  for (; per_block > 1 && total <= per_block * 128; per_block /= 2) {
+  }
   FitBlocks b;
-  b.tiles_per_block = (int)(per_wave * kFitWavefronts);
+  b.tiles_per_block = (int)per_block;
   b.blocks_per_strip = (int)((tiles + b.tiles_per_block - 1) / b.tiles_per_block);
   b.nblocks = (int)(strips * b.blocks_per_strip);
   return b;
@@ -39,7 +49,8 @@ inline FitBlocks fit_blocks(int n, int S) {
 
 // One adjoint workgroup: parts [part, part + parts) of one strip of a problem. A part's
 // sums are the same whichever workgroup takes it; a workgroup of several parts sets the
-// strip's tables up once.
+// strip's tables up once, and takes parts of fewer tiles than it has wavefronts side by
+// side.
 struct FitUnit {
   int problem, strip, part, parts;
 };
@@ -52,12 +63,12 @@ struct FitDesc {
   float* params;        // [W][5] {A, L, alpha, Q, phi0}
   float* adam_m;        // [W*5]
   float* adam_v;        // [W*5]
-  float* partials;      // [W*5 + 1][nblocks]: per-block sums of r . dd/dp and of |r|^2 / 2
+  float* partials;      // [nblocks][W*5 + 1]: per-block sums of r . dd/dp and of |r|^2 / 2
   float* loss;          // [1] loss of the last evaluation
   int* step;            // [1] Adam step counter
   int n, S, W;
   int tiles_per_block, blocks_per_strip, nblocks;  // FitBlocks
-  long long row_offset;        // first row of this problem in the reduce grid
+  long long reduce_offset;     // first block of this problem in the reduce grid
   long long param_out_offset;  // first parameter of this problem in a concatenated gradient
 };
 
@@ -66,7 +77,7 @@ struct FitAdam {
 };
 
 // Device tables of a batch: problems, adjoint units (grouped by wave-count class, class c
-// at [class_begin[c], + class_blocks[c])), reduce row -> problem.
+// at [class_begin[c], + class_blocks[c])), reduce block -> problem.
 // Streams beside the caller's on which the classes' adjoint launches run
 // concurrently (one class's tail overlaps the next class's blocks), joined by events
 // before the reduction.
@@ -75,10 +86,10 @@ constexpr int kFitSideStreams = 3;
 struct FitLaunch {
   const FitDesc* probs;
   const FitUnit* units;
-  const int* row_prob;
+  const int* reduce_prob;
   long long class_begin[kFitClasses];
   long long class_blocks[kFitClasses];
-  long long total_rows;
+  long long reduce_blocks;
   hipStream_t side[kFitSideStreams];  // null: every class on the caller's stream
   hipEvent_t fork;
   hipEvent_t join[kFitSideStreams];

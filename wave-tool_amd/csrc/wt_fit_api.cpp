@@ -21,11 +21,11 @@ wt_status ctx_fail(wt_ctx* ctx, wt_status s, const std::string& msg);
 struct wt_fit {
   wt_ctx* ctx = nullptr;
   int count = 0;
-  long long total_rows = 0, total_params = 0;
+  long long total_reduce = 0, total_params = 0;
   std::vector<wt::FitDesc> host;
   wt::FitDesc* d_desc = nullptr;
   wt::FitUnit* d_units = nullptr;
-  int* d_rows = nullptr;    // reduce row -> problem
+  int* d_rows = nullptr;    // reduce block -> problem
   char* d_state = nullptr;  // moments, partials, loss, step for every problem
   size_t state_bytes = 0;
   wt::FitLaunch launch{};
@@ -150,7 +150,7 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
   // state layout per problem: m[W*5], v[W*5], partials[(W*5+1)*nblocks], loss, step
   std::vector<size_t> off(count);
   size_t bytes = 0;
-  long long rounds = 0;  // tiles per wavefront over all blocks
+  long long rounds = 0, parts = 0;  // tiles per wavefront over all blocks, and the blocks
   for (uint32_t i = 0; i < count; ++i) {
     std::string why;
     if (!problem_ok(problems[i], &why)) {
@@ -176,10 +176,11 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
     d.tiles_per_block = fb.tiles_per_block;
     d.blocks_per_strip = fb.blocks_per_strip;
     d.nblocks = nblocks;
-    d.row_offset = f->total_rows;
+    d.reduce_offset = f->total_reduce;
     d.param_out_offset = f->total_params;
-    rounds += (long long)nblocks * (fb.tiles_per_block / wt::kFitWavefronts);
-    f->total_rows += np + 1;
+    rounds += ((long long)nblocks * fb.tiles_per_block + wt::kFitWavefronts - 1) / wt::kFitWavefronts;
+    parts += nblocks;
+    f->total_reduce += wt::reduce_blocks(d.W);
     f->total_params += np;
     off[i] = bytes;
     bytes += sizeof(float) * ((size_t)2 * np + (size_t)(np + 1) * nblocks + 1) + sizeof(int);
@@ -196,8 +197,11 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
     for (uint32_t i = 0; i < count; ++i) {
       const wt::FitDesc& d = f->host[i];
       if (wt::fit_class(d.W) != c) continue;
-      const int part_rounds = d.tiles_per_block / wt::kFitWavefronts;
-      const int per = (int)std::max<long long>(1, unit_rounds / part_rounds);
+      // parts that run side by side share a workgroup once every CU has one
+      const int side_by = std::max(1, wt::kFitWavefronts / d.tiles_per_block);
+      const int part_rounds = std::max(1, d.tiles_per_block / wt::kFitWavefronts);
+      const int per = unit_rounds > 1 ? (int)std::max<long long>(1, unit_rounds / part_rounds) * side_by
+                                      : (int)std::min<long long>(side_by, std::max<long long>(1, parts / 256));
       const int strips = d.nblocks / d.blocks_per_strip;
       for (int st = 0; st < strips; ++st)
         for (int b = 0; b < d.blocks_per_strip; b += per)
@@ -212,7 +216,7 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
     f->launch.class_blocks[c] = (long long)units.size() - unit_begin;
     unit_begin = (long long)units.size();
   }
-  if (units.size() >= (1ull << 31) || f->total_rows >= (1ll << 31)) {
+  if (units.size() >= (1ull << 31) || f->total_reduce >= (1ll << 31)) {
     delete f;
     return wt::ctx_fail(ctx, WT_ERR_UNSUPPORTED, "batch too large for one launch");
   }
@@ -232,10 +236,10 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
     d.loss = d.partials + (size_t)(np + 1) * d.nblocks;
     d.step = reinterpret_cast<int*>(d.loss + 1);
   }
-  std::vector<int> rows((size_t)f->total_rows);
+  std::vector<int> rows((size_t)f->total_reduce);
   for (uint32_t i = 0; i < count; ++i) {
     const wt::FitDesc& d = f->host[i];
-    for (int r = 0; r <= d.W * 5; ++r) rows[(size_t)d.row_offset + r] = (int)i;
+    for (int r = 0; r < wt::reduce_blocks(d.W); ++r) rows[(size_t)d.reduce_offset + r] = (int)i;
   }
   e = hipMalloc(&f->d_desc, sizeof(wt::FitDesc) * count);
   if (e == hipSuccess) e = hipMalloc(&f->d_units, sizeof(wt::FitUnit) * units.size());
@@ -253,8 +257,8 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
   }
   f->launch.probs = f->d_desc;
   f->launch.units = f->d_units;
-  f->launch.row_prob = f->d_rows;
-  f->launch.total_rows = f->total_rows;
+  f->launch.reduce_prob = f->d_rows;
+  f->launch.reduce_blocks = f->total_reduce;
   // side streams (default priority, not synchronising with the null stream) and their
   // fork / join events, for batches spanning several wave-count classes
   int classes = 0;
@@ -359,7 +363,7 @@ wt_status wt_fit_loss_grad_static(wt_ctx* ctx, const wt_fit_problem* p, float* d
   d.tiles_per_block = fb.tiles_per_block;
   d.blocks_per_strip = fb.blocks_per_strip;
   d.nblocks = (int)nblocks;
-  d.row_offset = 0;
+  d.reduce_offset = 0;
   d.param_out_offset = 0;
   const hipStream_t st = (hipStream_t)stream;
   wt::FitDesc* d_desc = reinterpret_cast<wt::FitDesc*>(b);
@@ -373,10 +377,10 @@ wt_status wt_fit_loss_grad_static(wt_ctx* ctx, const wt_fit_problem* p, float* d
   wt::FitLaunch L{};
   L.probs = d_desc;
   L.units = d_units;
-  L.row_prob = rows;
+  L.reduce_prob = rows;
   L.class_begin[cls] = 0;
   L.class_blocks[cls] = nblocks;
-  L.total_rows = np + 1;
+  L.reduce_blocks = wt::reduce_blocks(d.W);
   const wt::FitAdam a{0.0f, 0.0f, 0.0f, 0.0f};
   e = wt::launch_fit_iteration(L, a, 0, d_grad, d_loss, st);
   return e == hipSuccess ? WT_OK : hip_err(ctx, e, "fit gradient launch");
