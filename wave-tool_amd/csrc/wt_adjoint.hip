@@ -683,7 +683,9 @@ void adjoint_kernel(const FitDesc* __restrict__ probs, const FitUnit* __restrict
   // descriptor sits in SGPRs rather than VGPRs
   const FitUnit unit = load_uniform(units, (long long)blockIdx.x);
   const FitDesc P = load_uniform(probs, unit.problem);
-  if (bump_step && unit.strip == 0 && unit.part == 0 && tid == 0) P.step[0] += 1;  // Adam step of this iteration
+  // Adam step of this iteration, without a result to wait for: the load of `+= 1` held this
+  // one workgroup up, and so the launch, by a round trip to memory
+  if (bump_step && unit.strip == 0 && unit.part == 0 && tid == 0) atomicAdd(P.step, 1);
   const int chunks = (P.W + 15) >> 4, padded = 16 * chunks;
 
   // ---- the waves' constants, one thread per wave; the parameters' loads first, so that
