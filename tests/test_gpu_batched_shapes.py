@@ -50,3 +50,28 @@ def test_mixed_shapes_equal_plain(torch_cuda, wtctx, texture):
         wtctx.set_launch_config()
         batch.close()
     assert len(shapes) == 3
+
+
+@pytest.mark.parametrize("side,waves", [(64, 33), (65, 1), (128, 2), (129, 130), (640, 65), (641, 7)])
+def test_half_segments_equal_whole(torch_cuda, wtctx, side, waves):
+    """The plain kernel takes segments in halves up to 640 workgroups (side 640 here), the batch only those patches whose
+    upper halves are empty (side 64): the same bits from both, tangents included, with a heightmap and without."""
+    torch = torch_cuda
+    print("[case] halves, side %d" % side, flush=True)
+    spec = dict(scenes.batched_patches(seed=23, count=1)[0], N=side, W=waves)
+    patches, w, V = wt.batch_inputs([spec])
+    p = patches[0]
+    w = torch.from_numpy(w).cuda()
+    params = wt.water_params(np.ctypeslib.as_array(p.corners).copy(), spec["camera"][4:7], side, spec["time"], 0.02, 0.05,
+                             0.0, (0.3, 0.0))
+    batch = wt.Batch(wtctx, patches)
+    try:
+        wtctx.set_launch_config(*batch.patch_launch_config(0))
+        for kw in ({}, dict(heightmap=torch.from_numpy(scenes.value_noise(3, 64)).cuda())):
+            a, b = (torch.full((4, V * 3), float("nan"), device="cuda") for _ in range(2))
+            batch.displace(w, *a, **kw)
+            wtctx.displace(params, w, *b, **kw)
+            assert torch.equal(a, b) and torch.isfinite(a).all()
+    finally:
+        wtctx.set_launch_config()
+        batch.close()

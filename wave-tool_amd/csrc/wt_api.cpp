@@ -634,16 +634,19 @@ static wt_status batch_create(wt_ctx* ctx, const wt_patch* patches, uint32_t cou
     max_n = std::max(max_n, p.gridLength);
   }
   // units: one workgroup's segments of one patch, in that patch's segment shape; most
-  // expensive first, over all shapes: a unit covers 1024 vertices in each shape, so it
-  // costs about its patch's wave count
+  // expensive first, over all shapes: a unit covers 1024 vertices in each shape (half of
+  // them in half segments), so it costs about its patch's wave count
   std::vector<uint32_t> order(count);
   std::iota(order.begin(), order.end(), 0u);
   std::stable_sort(order.begin(), order.end(),
                    [&](uint32_t x, uint32_t y) { return b->patches[x].W > b->patches[y].W; });
   std::vector<wt::BatchUnit> units;
   for (uint32_t i : order) {
-    const wt::PatchDesc& d = b->patches[i];
-    const long long groups = wt::forward_segment_groups(d.N, wt::kBatchShape[d.shape]);
+    wt::PatchDesc& d = b->patches[i];
+    wt::LaunchShape s = wt::kBatchShape[d.shape];
+    d.half = d.N <= s.lanes_per_row * s.steps / 2;
+    if (d.half) s.steps /= 2;
+    const long long groups = wt::forward_segment_groups(d.N, s);
     for (long long gidx = 0; gidx < groups; ++gidx) units.push_back(wt::BatchUnit{(int)i, (int)gidx});
   }
   if (units.size() >= (1ull << 31)) {

@@ -226,9 +226,20 @@ __device__ __forceinline__ RowOut row_out(const EpilogueArgs& e, size_t row_firs
   return RowOut{e.pos + o, e.nrm + o, e.tan ? e.tan + o : nullptr, e.bit ? e.bit + o : nullptr};
 }
 
+// x^2 + y^2 + z^2 and x a + y b + z c as the untextured epilogue forms them: the product
+// of the first or the second pair rounded, the others fused onto it.
+__device__ __forceinline__ float dot3_from(bool second, float x, float y, float z, float a, float b, float c) {
+  const float p = second ? y : x, pa = second ? b : a, q = second ? x : y, qa = second ? a : b;
+  return fmaf(z, c, fmaf(q, qa, p * pa));
+}
+
+// lead: the vertex a lane finishes first of a segment. Without a heightmap the sums of
+// three products are written out, which differ by it in the product they start from: left
+// to the compiler, their rounding depends on the number of vertices a lane finishes, and a
+// segment has to give the same bits whole and in halves.
 template <int M>
 __device__ __forceinline__ void vertex_finish(const EpilogueArgs& e, const VertexPending& v, const float acc[8],
-                                              const RowOut& ro, uint32_t col) {
+                                              const RowOut& ro, uint32_t col, bool lead) {
   const float Cx = acc[2], Cz = acc[3];
   const float Y = acc[4], Sxx = acc[5], Sxz = acc[6], Szz = acc[7];
   const float px = v.px, pz = v.pz;
@@ -248,12 +259,23 @@ __device__ __forceinline__ void vertex_finish(const EpilogueArgs& e, const Verte
   }
   py += e.bounce;  // water-grid.vert:147
   // N = normalize(B x T): y-up for the undisplaced plane
-  float nx = by * tz - bz * ty, ny = bz * tx - bx * tz, nz = bx * ty - by * tx;
-  const float inv_n = __builtin_amdgcn_rsqf(nx * nx + ny * ny + nz * nz);
+  constexpr bool kFlat = M == kTexNone;
+  float nx, ny, nz;
+  if constexpr (kFlat) {
+    nx = fmaf(by, tz, -(bz * ty));
+    ny = fmaf(bz, tx, -(bx * tz));
+    nz = fmaf(bx, ty, -(by * tx));
+  } else {
+    nx = by * tz - bz * ty;
+    ny = bz * tx - bx * tz;
+    nz = bx * ty - by * tx;
+  }
+  const float inv_n =
+      __builtin_amdgcn_rsqf(kFlat ? dot3_from(!lead, nx, ny, nz, nx, ny, nz) : nx * nx + ny * ny + nz * nz);
   nx *= inv_n; ny *= inv_n; nz *= inv_n;
   // flip toward the camera (water-grid.vert:190)
   const float vx = e.cam[0] - px, vy = e.cam[1] - py, vz = e.cam[2] - pz;
-  if (nx * vx + ny * vy + nz * vz < 0.0f) { nx = -nx; ny = -ny; nz = -nz; }
+  if ((kFlat ? dot3_from(!lead, nx, ny, nz, vx, vy, vz) : nx * vx + ny * vy + nz * vz) < 0.0f) { nx = -nx; ny = -ny; nz = -nz; }
   // the outputs are written once per frame and not read back by this kernel: stream
   // them past the caches (4% faster on the 1024^2 x 64-wave frame)
   // byte offset within the row as a 32-bit value (a row is at most 32768 x 12 bytes), so
@@ -263,11 +285,12 @@ __device__ __forceinline__ void vertex_finish(const EpilogueArgs& e, const Verte
   store3_nt(row_at(ro.pos, b), px, py, pz);
   store3_nt(row_at(ro.nrm, b), nx, ny, nz);
   if (ro.tan) {
-    const float it = __builtin_amdgcn_rsqf(tx * tx + ty * ty + tz * tz);
+    const float it = __builtin_amdgcn_rsqf(kFlat ? __fadd_rn(lead ? fmaf(tx, tx, ty * ty) : fmaf(ty, ty, tx * tx), tz * tz)
+                                                 : tx * tx + ty * ty + tz * tz);
     store3_nt(row_at(ro.tan, b), tx * it, ty * it, tz * it);
   }
   if (ro.bit) {
-    const float ib = __builtin_amdgcn_rsqf(bx * bx + by * by + bz * bz);
+    const float ib = __builtin_amdgcn_rsqf(kFlat ? fmaf(bz, bz, fmaf(by, by, bx * bx)) : bx * bx + by * by + bz * bz);
     store3_nt(row_at(ro.bit, b), bx * ib, by * ib, bz * ib);
   }
 }

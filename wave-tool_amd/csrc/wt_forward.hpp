@@ -237,9 +237,11 @@ __device__ __forceinline__ void steps_rotation(float (&acc)[K][8], float& c, flo
 
 // The same steps with the three-term recurrence; step 0 -> 1 is a rotation, which also
 // sets the previous values (cm, sm).
-template <int K, int J0, int J1, bool kInit = false>
+// later (the upper half of a lane's steps, kHalf): (cm, sm) are set, and step 0 -> 1 takes
+// the recurrence too.
+template <int K, int J0, int J1, bool kHalf, bool kInit = false>
 __device__ __forceinline__ void steps_chebyshev(float (&acc)[K][8], float& c, float& s, float& cm, float& sm,
-                                                const float4& cc, const float4& cs, const float4& rot) {
+                                                const float4& cc, const float4& cs, const float4& rot, bool later) {
 #pragma unroll
   for (int j = J0; j < J1; ++j) {
     accumulate<K, kInit>(acc[j], c, s, cc, cs);
@@ -248,6 +250,10 @@ __device__ __forceinline__ void steps_chebyshev(float (&acc)[K][8], float& c, fl
       if (j == 0) {
         cn = fmaf(s, rot.z, c * rot.x);
         sn = fmaf(c, rot.y, s * rot.x);
+        if (kHalf) {
+          cn = later ? fmaf(rot.w, c, -cm) : cn;
+          sn = later ? fmaf(rot.w, s, -sm) : sn;
+        }
       } else {
         cn = fmaf(rot.w, c, -cm);
         sn = fmaf(rot.w, s, -sm);
@@ -261,12 +267,33 @@ __device__ __forceinline__ void steps_chebyshev(float (&acc)[K][8], float& c, fl
   }
 }
 
+// The K steps that a wavefront of the upper half of a lane's 2 K leaves to the lower half:
+// only the sequence runs, by the same operations.
+template <int K, bool kCheb>
+__device__ __forceinline__ void skip_steps(float& c, float& s, float& cm, float& sm, const float4& rot) {
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    float cn, sn;
+    if (j == 0 || !kCheb) {
+      cn = fmaf(s, rot.z, c * rot.x);
+      sn = fmaf(c, rot.y, s * rot.x);
+    } else {
+      cn = fmaf(rot.w, c, -cm);
+      sn = fmaf(rot.w, s, -sm);
+    }
+    cm = c;
+    sm = s;
+    c = cn;
+    s = sn;
+  }
+}
+
 // Epilogue of a lane's KS finished vertices, fin[u] at column col0 + u * dcol (dcol = LC,
 // or -LC for a wavefront that stepped back): all texel loads first, then the per-vertex
 // math and stores.
 template <int KS, int kTex>
 __device__ __forceinline__ void epilogue_steps(const FwdParams& p, const RowGeom& g, const float (&fin)[KS][8],
-                                               int col0, int dcol, int row, bool active) {
+                                               int col0, int dcol, int row, bool active, bool later) {
   VertexPending pend[KS];
 #pragma unroll
   for (int u = 0; u < KS; ++u) {
@@ -278,7 +305,7 @@ __device__ __forceinline__ void epilogue_steps(const FwdParams& p, const RowGeom
 #pragma unroll
   for (int u = 0; u < KS; ++u) {
     const int col = col0 + u * dcol;
-    if (active && row < p.N && col < p.N) vertex_finish<kTex>(p.ep, pend[u], fin[u], ro, (uint32_t)col);
+    if (active && row < p.N && col < p.N) vertex_finish<kTex>(p.ep, pend[u], fin[u], ro, (uint32_t)col, u == 0 && !later);
   }
 }
 
@@ -328,6 +355,7 @@ struct SegIds {
   float rsgn;    // +1 stepping towards higher columns, -1 stepping back
   float lcf;
   int lane;
+  bool later;  // the wavefront takes the upper half of its lanes' steps (kHalf)
 };
 
 // One chunk of waves [w0, w0 + CH): the step table, then this wavefront's waves summed
@@ -336,7 +364,7 @@ struct SegIds {
 // k's steps (scheduling barriers keep the compiler from hoisting its dependent chain
 // back to the top of the iteration). kFirst: the first chunk with W >= S, where every
 // wavefront has a wave; its first entry writes the sums (kInit).
-template <bool kFirst, int K, int LC, int S, int CH>
+template <bool kFirst, int K, int LC, int S, int CH, bool kHalf>
 __device__ __forceinline__ void chunk_pass(const FwdParams& p, SegShared<K, LC, S, CH>& sh, const SegIds& id, int w0,
                                            float (&acc)[K][8]) {
   constexpr int LR = 64 / LC;
@@ -360,12 +388,14 @@ __device__ __forceinline__ void chunk_pass(const FwdParams& p, SegShared<K, LC, 
     const float4 sd = tab[1 < nmine ? 1 : 0].seed;
     float cn, sn;
     if (ncheb > 0) {
-      steps_chebyshev<K, 0, K / 2, true>(acc, c, s, cm, sm, cc, cs, rot);
+      if (kHalf && id.later) skip_steps<K, true>(c, s, cm, sm, rot);
+      steps_chebyshev<K, 0, K / 2, kHalf, true>(acc, c, s, cm, sm, cc, cs, rot, id.later);
       __builtin_amdgcn_sched_barrier(0);
       seed_trig(sd, lcf, &cn, &sn);
       __builtin_amdgcn_sched_barrier(0);
-      steps_chebyshev<K, K / 2, K, true>(acc, c, s, cm, sm, cc, cs, rot);
+      steps_chebyshev<K, K / 2, K, kHalf, true>(acc, c, s, cm, sm, cc, cs, rot, id.later);
     } else {
+      if (kHalf && id.later) skip_steps<K, false>(c, s, cm, sm, rot);
       steps_rotation<K, 0, K / 2, true>(acc, c, s, cc, cs, rot);
       __builtin_amdgcn_sched_barrier(0);
       seed_trig(sd, lcf, &cn, &sn);
@@ -381,11 +411,12 @@ __device__ __forceinline__ void chunk_pass(const FwdParams& p, SegShared<K, LC, 
     const float4 rot = t.rot, cc = t.cc, cs = t.cs;
     const float4 sd = tab[k + 1 < nmine ? k + 1 : k].seed;
     float cn, sn;
-    steps_chebyshev<K, 0, K / 2>(acc, c, s, cm, sm, cc, cs, rot);
+    if (kHalf && id.later) skip_steps<K, true>(c, s, cm, sm, rot);
+    steps_chebyshev<K, 0, K / 2, kHalf>(acc, c, s, cm, sm, cc, cs, rot, id.later);
     __builtin_amdgcn_sched_barrier(0);
     seed_trig(sd, lcf, &cn, &sn);
     __builtin_amdgcn_sched_barrier(0);
-    steps_chebyshev<K, K / 2, K>(acc, c, s, cm, sm, cc, cs, rot);
+    steps_chebyshev<K, K / 2, K, kHalf>(acc, c, s, cm, sm, cc, cs, rot, id.later);
     c = cn;
     s = sn;
   }
@@ -394,6 +425,7 @@ __device__ __forceinline__ void chunk_pass(const FwdParams& p, SegShared<K, LC, 
     const float4 rot = t.rot, cc = t.cc, cs = t.cs;
     const float4 sd = tab[k + 1 < nmine ? k + 1 : k].seed;
     float cn, sn;
+    if (kHalf && id.later) skip_steps<K, false>(c, s, cm, sm, rot);
     steps_rotation<K, 0, K / 2>(acc, c, s, cc, cs, rot);
     __builtin_amdgcn_sched_barrier(0);
     seed_trig(sd, lcf, &cn, &sn);
@@ -406,7 +438,11 @@ __device__ __forceinline__ void chunk_pass(const FwdParams& p, SegShared<K, LC, 
 
 // One workgroup's segments of one grid: the whole forward program for the vertices of
 // segment group `seg_group` (kSegPerWG segments). Every thread of the block calls it.
-template <int K, int LC, int S, int kTex, int CH = kChunk>
+// kHalf: the segments are halves of segments of 2 K steps, each taken by a pair of
+// wavefronts of its own. Both pairs seed where the whole segment does and run its
+// sequences, so every sum has the same bits; the pair's wavefront that comes to the half
+// second skips the other half's sums.
+template <int K, int LC, int S, int kTex, int CH = kChunk, bool kHalf = false>
 __device__ __forceinline__ void forward_segments(const FwdParams& p, long long seg_group, SegShared<K, LC, S, CH>& sh) {
   constexpr int LR = 64 / LC;
   constexpr int KS = K / S;                       // vertices per lane in the epilogue
@@ -445,16 +481,20 @@ __device__ __forceinline__ void forward_segments(const FwdParams& p, long long s
   // S = 2: the second wavefront of a pair steps its vertices back from the far column
   // (seed there, rotation by -d), so the exchange is the same code on both sides
   const bool back = S > 1 && sid == 1;
-  const SegIds ids{sid, wid, lr, row_base, col_base + (back ? (K - 1) * LC : 0), back ? -1.0f : 1.0f, lcf, lane};
+  static_assert(!kHalf || S == 2, "halves are taken by pairs");
+  const bool upper = kHalf && (seg & 1);  // the half of the higher columns
+  const int seed_base = kHalf ? (seg >> 1) * (2 * LC * K) : col_base;
+  const SegIds ids{sid, wid, lr, row_base, seed_base + (back ? ((kHalf ? 2 : 1) * K - 1) * LC : 0), back ? -1.0f : 1.0f,
+                   lcf, lane, kHalf && upper != back};
   if (p.W < S) {
 #pragma unroll
     for (int j = 0; j < K; ++j)
 #pragma unroll
       for (int q = 0; q < 8; ++q) acc[j][q] = 0.0f;
-    for (int w0 = 0; w0 < p.W; w0 += CH) chunk_pass<false, K, LC, S, CH>(p, sh, ids, w0, acc);
+    for (int w0 = 0; w0 < p.W; w0 += CH) chunk_pass<false, K, LC, S, CH, kHalf>(p, sh, ids, w0, acc);
   } else {
-    chunk_pass<true, K, LC, S, CH>(p, sh, ids, 0, acc);
-    for (int w0 = CH; w0 < p.W; w0 += CH) chunk_pass<false, K, LC, S, CH>(p, sh, ids, w0, acc);
+    chunk_pass<true, K, LC, S, CH, kHalf>(p, sh, ids, 0, acc);
+    for (int w0 = CH; w0 < p.W; w0 += CH) chunk_pass<false, K, LC, S, CH, kHalf>(p, sh, ids, w0, acc);
   }
   const RowGeom g = row_geom(p, row < p.N ? row : p.N - 1);
 
@@ -478,13 +518,13 @@ __device__ __forceinline__ void forward_segments(const FwdParams& p, long long s
 #pragma unroll
       for (int q = 0; q < 8; ++q) fin[j][q] = acc[j][q];
   }
-  epilogue_steps<KS, kTex>(p, g, fin, col0 + (back ? (K - 1) * LC : 0), back ? -LC : LC, row, active);
+  epilogue_steps<KS, kTex>(p, g, fin, col0 + (back ? (K - 1) * LC : 0), back ? -LC : LC, row, active, ids.later);
 }
 
-template <int K, int LC, int S, int kTex, int CH>
+template <int K, int LC, int S, int kTex, int CH, bool kHalf = false>
 __global__ __launch_bounds__(256) void water_forward_kernel(FwdParams p) {
   __shared__ SegShared<K, LC, S, CH> sh;
-  forward_segments<K, LC, S, kTex, CH>(p, (long long)blockIdx.x, sh);
+  forward_segments<K, LC, S, kTex, CH, kHalf>(p, (long long)blockIdx.x, sh);
 }
 
 // ------------------------------------------------------------------ batched
@@ -542,24 +582,27 @@ __device__ __forceinline__ FwdParams patch_params(const BatchArgs& a, const Patc
 // tails one after another: 24 patches of sides 32 to 160 (camera update and displacement)
 // took 33.3 us so and take 25.4; a batch of 512 large patches is VALU-bound and takes the
 // same time either way.
-template <int kTex, int kShape>
+template <int kShape, bool kHalf>
+using BatchLds = SegShared<kBatchShape[kShape].steps / (kHalf ? 2 : 1), kBatchShape[kShape].lanes_per_row, 2>;
+
+template <int kTex, int kShape, bool kHalf>
 __device__ __forceinline__ void batched_unit(const BatchArgs& a, BatchUnit unit, void* lds) {
-  constexpr int K = kBatchShape[kShape].steps, LC = kBatchShape[kShape].lanes_per_row;
+  constexpr int K = kBatchShape[kShape].steps / (kHalf ? 2 : 1), LC = kBatchShape[kShape].lanes_per_row;
   static_assert(kBatchShape[kShape].split == 2, "batched shapes pair two wavefronts per segment");
   // the index is opaque per branch, so that no branch's part is hoisted above the switch,
   // where it would be held in registers through the others' (138 VGPRs)
   asm volatile("" : "+s"(unit.patch));
   const PatchDesc pd = load_uniform(a.patches, unit.patch);
-  forward_segments<K, LC, 2, kTex>(patch_params(a, pd), (long long)unit.group, *static_cast<SegShared<K, LC, 2>*>(lds));
+  forward_segments<K, LC, 2, kTex, kChunk, kHalf>(patch_params(a, pd), (long long)unit.group,
+                                                  *static_cast<BatchLds<kShape, kHalf>*>(lds));
 }
 
 template <int kTex>
 __global__ __launch_bounds__(256, 4) void water_forward_batched_kernel(BatchArgs a) {
-  static_assert(kBatchShapes == 3, "one branch per shape below");
-  constexpr size_t kBytes =
-      cmax(cmax(sizeof(SegShared<kBatchShape[0].steps, kBatchShape[0].lanes_per_row, 2>),
-                sizeof(SegShared<kBatchShape[1].steps, kBatchShape[1].lanes_per_row, 2>)),
-           sizeof(SegShared<kBatchShape[2].steps, kBatchShape[2].lanes_per_row, 2>));
+  static_assert(kBatchShapes == 3, "two branches per shape below");
+  constexpr size_t kBytes = cmax(cmax(sizeof(BatchLds<0, false>), sizeof(BatchLds<1, false>)),
+                                 cmax(sizeof(BatchLds<2, false>), sizeof(BatchLds<2, true>)));
+  static_assert(sizeof(BatchLds<0, true>) <= kBytes && sizeof(BatchLds<1, true>) <= kBytes, "whole segments need more");
   __shared__ alignas(16) unsigned char lds[kBytes];
   // the unit and patch tables do not change during the launch: read them through the
   // constant address space so they load with scalar loads into SGPRs (a vector load
@@ -567,10 +610,13 @@ __global__ __launch_bounds__(256, 4) void water_forward_batched_kernel(BatchArgs
   const BatchUnit unit = load_uniform(a.units, a.unit_begin + (long long)blockIdx.x);
   const PatchDesc pd = load_uniform(a.patches, unit.patch);
   if (!pd.active) return;  // workgroup-uniform
-  switch (pd.shape) {
-    case 0: batched_unit<kTex, 0>(a, unit, lds); break;
-    case 1: batched_unit<kTex, 1>(a, unit, lds); break;
-    default: batched_unit<kTex, 2>(a, unit, lds); break;
+  switch (2 * pd.shape + pd.half) {
+    case 0: batched_unit<kTex, 0, false>(a, unit, lds); break;
+    case 1: batched_unit<kTex, 0, true>(a, unit, lds); break;
+    case 2: batched_unit<kTex, 1, false>(a, unit, lds); break;
+    case 3: batched_unit<kTex, 1, true>(a, unit, lds); break;
+    case 4: batched_unit<kTex, 2, false>(a, unit, lds); break;
+    default: batched_unit<kTex, 2, true>(a, unit, lds); break;
   }
 }
 
@@ -582,12 +628,21 @@ hipError_t launch_batched_mode(const BatchArgs& a, hipStream_t st) {
 }
 
 // ------------------------------------------------------------------ launch helpers
+
 template <int K, int LC, int S, int kTex, int CH = kChunk>
 hipError_t launch_t(const FwdParams& p, hipStream_t st) {
   constexpr int LR = 64 / LC;
   constexpr int kSegPerWG = kWavesPerWG / S;
-  const long long segs = (long long)((p.N + LC * K - 1) / (LC * K)) * ((p.N + LR - 1) / LR);
-  const long long blocks = (segs + kSegPerWG - 1) / kSegPerWG;
+  const long long row_groups = (p.N + LR - 1) / LR;
+  const long long blocks = ((p.N + LC * K - 1) / (LC * K) * row_groups + kSegPerWG - 1) / kSegPerWG;
+  if constexpr (K == 8 && S == 2 && LC >= 16 && CH == kChunk) {
+    if (blocks <= kHalvesBlocks) {
+      constexpr int H = K / 2;
+      const long long halves = ((p.N + LC * H - 1) / (LC * H) * row_groups + kSegPerWG - 1) / kSegPerWG;
+      hipLaunchKernelGGL((water_forward_kernel<H, LC, S, kTex, CH, true>), dim3((unsigned)halves), dim3(256), 0, st, p);
+      return hipGetLastError();
+    }
+  }
   hipLaunchKernelGGL((water_forward_kernel<K, LC, S, kTex, CH>), dim3((unsigned)blocks), dim3(256), 0, st, p);
   return hipGetLastError();
 }

@@ -42,7 +42,11 @@ struct PatchDesc {
   int shape;                // segment shape of this patch in the batched kernel (kBatchShapes)
   long long vertex_offset;  // first vertex of the patch in the output arrays
   int active;               // 0: the patch's camera misses the water; its units write nothing
-  int reserved;
+  // 1: taken in half segments. Where the upper halves have no columns, that drops their
+  // sums and takes no more workgroups (256 patches of sides 17 to 40: 15.0 -> 12.4 us);
+  // elsewhere a batch's units fill the card, and halves repeat work (64 patches of sides
+  // 60 to 130: 30.9 -> 35.8 us)
+  int half;
 };
 
 // Corner algebra of a grid from its corners [4][4] (BL, TL, BR, TR; x and z used).
@@ -57,6 +61,15 @@ __host__ __device__ inline void set_corner_algebra(D& d, const double (*c)[4]) {
   d.duv_x = c[3][0] - c[1][0] - c[2][0] + c[0][0];
   d.duv_z = c[3][2] - c[1][2] - c[2][2] + c[0][2];
 }
+
+// Launches of up to this many workgroups take segments of 8 steps and two wavefronts in
+// halves of 4 steps, a pair of wavefronts each: they leave SIMDs idle, and a wavefront's
+// chain of sums and vertices, which bounds them, is about half as long (the upper half
+// repeats the lower one's sequence). Above, the repeated work costs more than the idle
+// SIMDs. Whole / in halves, us per launch in a graph: 128 x 128 with 16 waves 5.3 / 4.5,
+// 256 x 256 with 100 waves 15.4 / 12.5, 513 x 513 with 64 waves (513 workgroups) 17.9 / 16.0,
+// 600 x 600 with 100 waves (600) 26.2 / 24.7, 700 x 700 with 100 waves (700) 28.0 / 28.8.
+constexpr long long kHalvesBlocks = 640;
 
 // One workgroup's segment group of one patch.
 struct BatchUnit {
