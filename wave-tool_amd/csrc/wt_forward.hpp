@@ -577,7 +577,7 @@ __device__ __forceinline__ FwdParams patch_params(const BatchArgs& a, const Patc
 // them like a longest-first work queue, with no atomics: a device-wide unit counter
 // serialises every fetch through one address and measured twice as slow as this on a
 // single 1024 x 1024, 64-wave patch. All shapes step K = 8 vertices per lane with the same
-// LDS size, and the branch over them costs no wavefront per SIMD (126 VGPRs, and the widest
+// LDS size, and the branch over them costs no wavefront per SIMD (127 VGPRs, and the widest
 // shape alone takes 128), so one launch covers a batch. A launch per shape ran the shapes'
 // tails one after another: 24 patches of sides 32 to 160 (camera update and displacement)
 // took 33.3 us so and take 25.4; a batch of 512 large patches is VALU-bound and takes the
