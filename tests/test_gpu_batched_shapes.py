@@ -52,10 +52,11 @@ def test_mixed_shapes_equal_plain(torch_cuda, wtctx, texture):
     assert len(shapes) == 3
 
 
-@pytest.mark.parametrize("side,waves", [(64, 33), (65, 1), (128, 2), (129, 130), (640, 65), (641, 7)])
+@pytest.mark.parametrize("side,waves", [(64, 33), (65, 1), (128, 2), (129, 130), (640, 65), (641, 7), (1100, 3)])
 def test_half_segments_equal_whole(torch_cuda, wtctx, side, waves):
-    """The plain kernel takes segments in halves up to 640 workgroups (side 640 here), the batch only those patches whose
-    upper halves are empty (side 64): the same bits from both, tangents included, with a heightmap and without."""
+    """The plain kernel takes every segment in halves up to 640 workgroups (side 640 here), past that, as the batch at any
+    size, only those at the rows' ends whose upper halves are empty: the same bits, tangents included, with a heightmap
+    and without."""
     torch = torch_cuda
     print("[case] halves, side %d" % side, flush=True)
     spec = dict(scenes.batched_patches(seed=23, count=1)[0], N=side, W=waves)

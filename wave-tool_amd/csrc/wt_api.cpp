@@ -643,10 +643,11 @@ static wt_status batch_create(wt_ctx* ctx, const wt_patch* patches, uint32_t cou
   std::vector<wt::BatchUnit> units;
   for (uint32_t i : order) {
     wt::PatchDesc& d = b->patches[i];
-    wt::LaunchShape s = wt::kBatchShape[d.shape];
-    d.half = d.N <= s.lanes_per_row * s.steps / 2;
-    if (d.half) s.steps /= 2;
-    const long long groups = wt::forward_segment_groups(d.N, s);
+    const wt::LaunchShape& s = wt::kBatchShape[d.shape];
+    const wt::RowCut cut = wt::row_cut(d.N, s);
+    d.whole_groups = (int)cut.whole_groups;
+    d.whole_per_row = cut.whole_per_row;
+    const long long groups = cut.whole_groups + cut.end_groups;
     for (long long gidx = 0; gidx < groups; ++gidx) units.push_back(wt::BatchUnit{(int)i, (int)gidx});
   }
   if (units.size() >= (1ull << 31)) {

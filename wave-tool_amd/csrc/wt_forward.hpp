@@ -442,8 +442,10 @@ __device__ __forceinline__ void chunk_pass(const FwdParams& p, SegShared<K, LC, 
 // wavefronts of its own. Both pairs seed where the whole segment does and run its
 // sequences, so every sum has the same bits; the pair's wavefront that comes to the half
 // second skips the other half's sums.
+// per_row, first: the segments (or halves) of a row that the groups cover, and the first.
 template <int K, int LC, int S, int kTex, int CH = kChunk, bool kHalf = false>
-__device__ __forceinline__ void forward_segments(const FwdParams& p, long long seg_group, SegShared<K, LC, S, CH>& sh) {
+__device__ __forceinline__ void forward_segments(const FwdParams& p, long long seg_group, int per_row, int first,
+                                                 SegShared<K, LC, S, CH>& sh) {
   constexpr int LR = 64 / LC;
   constexpr int KS = K / S;                       // vertices per lane in the epilogue
   constexpr int kSegPerWG = kWavesPerWG / S;
@@ -452,11 +454,10 @@ __device__ __forceinline__ void forward_segments(const FwdParams& p, long long s
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
   const int grp = wid / S, sid = wid - grp * S;
   const long long seg_global = seg_group * kSegPerWG + grp;
-  const int segs_per_rg = (p.N + LC * K - 1) / (LC * K);
   const int n_rg = (p.N + LR - 1) / LR;
-  const bool active = seg_global < (long long)segs_per_rg * n_rg;
+  const bool active = seg_global < (long long)per_row * n_rg;
   const int seg_id = active ? (int)seg_global : 0;
-  const int rg = seg_id / segs_per_rg, seg = seg_id - rg * segs_per_rg;
+  const int rg = seg_id / per_row, seg = first + (seg_id - rg * per_row);
   const int row_base = rg * LR;
   // A wave64 VALU instruction runs as four passes of 16 lanes; with kInterleave, lanes l,
   // l + 16, l + 32, l + 48 take neighbouring vertices (adjacent columns; for LC <= 16
@@ -524,7 +525,29 @@ __device__ __forceinline__ void forward_segments(const FwdParams& p, long long s
 template <int K, int LC, int S, int kTex, int CH, bool kHalf = false>
 __global__ __launch_bounds__(256) void water_forward_kernel(FwdParams p) {
   __shared__ SegShared<K, LC, S, CH> sh;
-  forward_segments<K, LC, S, kTex, CH, kHalf>(p, (long long)blockIdx.x, sh);
+  forward_segments<K, LC, S, kTex, CH, kHalf>(p, (long long)blockIdx.x, (p.N + LC * K - 1) / (LC * K), 0, sh);
+}
+
+// Rows that end in the lower half of a segment: whole segments in the first `whole`
+// workgroups, the halves at the rows' ends in the others, which as whole segments sum and
+// sample columns past the edge (per launch in a graph, so / in halves: 700 x 700 with 64
+// waves 20.5 / 18.5 us, 1100 x 1100 with 100 waves 54.9 / 48.5; with 4 waves 8.75 / 8.77 and
+// 15.6 / 14.2).
+template <int K, int LC, int kTex>
+__global__ __launch_bounds__(256, 4) void water_forward_tail_kernel(FwdParams p, int whole) {
+  static_assert(sizeof(SegShared<K / 2, LC, 2>) <= sizeof(SegShared<K, LC, 2>), "one allocation for both");
+  __shared__ SegShared<K, LC, 2> sh;
+  int group = (int)blockIdx.x;
+  // opaque in each branch, so that neither's part is hoisted into the other's registers
+  if (group < whole) {
+    asm volatile("" : "+s"(group), "+s"(p.N));
+    forward_segments<K, LC, 2, kTex>(p, (long long)group, p.N / (LC * K), 0, sh);
+  } else {
+    group -= whole;
+    asm volatile("" : "+s"(group), "+s"(p.N));
+    forward_segments<K / 2, LC, 2, kTex, kChunk, true>(p, (long long)group, 1, p.N / (LC * K) * 2,
+                                                       *reinterpret_cast<SegShared<K / 2, LC, 2>*>(&sh));
+  }
 }
 
 // ------------------------------------------------------------------ batched
@@ -593,7 +616,9 @@ __device__ __forceinline__ void batched_unit(const BatchArgs& a, BatchUnit unit,
   // where it would be held in registers through the others' (138 VGPRs)
   asm volatile("" : "+s"(unit.patch));
   const PatchDesc pd = load_uniform(a.patches, unit.patch);
-  forward_segments<K, LC, 2, kTex, kChunk, kHalf>(patch_params(a, pd), (long long)unit.group,
+  const int per_row = kHalf ? 1 : pd.whole_per_row, first = kHalf ? 2 * pd.whole_per_row : 0;
+  const int group = kHalf ? unit.group - pd.whole_groups : unit.group;
+  forward_segments<K, LC, 2, kTex, kChunk, kHalf>(patch_params(a, pd), (long long)group, per_row, first,
                                                   *static_cast<BatchLds<kShape, kHalf>*>(lds));
 }
 
@@ -610,7 +635,7 @@ __global__ __launch_bounds__(256, 4) void water_forward_batched_kernel(BatchArgs
   const BatchUnit unit = load_uniform(a.units, a.unit_begin + (long long)blockIdx.x);
   const PatchDesc pd = load_uniform(a.patches, unit.patch);
   if (!pd.active) return;  // workgroup-uniform
-  switch (2 * pd.shape + pd.half) {
+  switch (2 * pd.shape + (unit.group >= pd.whole_groups ? 1 : 0)) {
     case 0: batched_unit<kTex, 0, false>(a, unit, lds); break;
     case 1: batched_unit<kTex, 0, true>(a, unit, lds); break;
     case 2: batched_unit<kTex, 1, false>(a, unit, lds); break;
@@ -640,6 +665,12 @@ hipError_t launch_t(const FwdParams& p, hipStream_t st) {
       constexpr int H = K / 2;
       const long long halves = ((p.N + LC * H - 1) / (LC * H) * row_groups + kSegPerWG - 1) / kSegPerWG;
       hipLaunchKernelGGL((water_forward_kernel<H, LC, S, kTex, CH, true>), dim3((unsigned)halves), dim3(256), 0, st, p);
+      return hipGetLastError();
+    }
+    const RowCut cut = row_cut(p.N, LaunchShape{S, K, LC, CH});
+    if (cut.end_groups > 0 && cut.whole_groups > 0) {
+      hipLaunchKernelGGL((water_forward_tail_kernel<K, LC, kTex>), dim3((unsigned)(cut.whole_groups + cut.end_groups)),
+                         dim3(256), 0, st, p, (int)cut.whole_groups);
       return hipGetLastError();
     }
   }

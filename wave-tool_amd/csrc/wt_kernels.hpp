@@ -42,11 +42,12 @@ struct PatchDesc {
   int shape;                // segment shape of this patch in the batched kernel (kBatchShapes)
   long long vertex_offset;  // first vertex of the patch in the output arrays
   int active;               // 0: the patch's camera misses the water; its units write nothing
-  // 1: taken in half segments. Where the upper halves have no columns, that drops their
-  // sums and takes no more workgroups (256 patches of sides 17 to 40: 15.0 -> 12.4 us);
-  // elsewhere a batch's units fill the card, and halves repeat work (64 patches of sides
-  // 60 to 130: 30.9 -> 35.8 us)
-  int half;
+  // units [0, whole_groups) are of whole segments, whole_per_row to a row; the others of
+  // the half segments that end the rows where their upper halves have no columns (row_cut;
+  // 256 patches of sides 17 to 40: 15.0 -> 12.3 us). A batch's units fill the card, so
+  // segments with columns in both halves stay whole: all in halves, 64 patches of sides 60
+  // to 130 took 35.8 us against 30.9
+  int whole_groups, whole_per_row;
 };
 
 // Corner algebra of a grid from its corners [4][4] (BL, TL, BR, TR; x and z used).
@@ -70,6 +71,24 @@ __host__ __device__ inline void set_corner_algebra(D& d, const double (*c)[4]) {
 // 256 x 256 with 100 waves 15.4 / 12.5, 513 x 513 with 64 waves (513 workgroups) 17.9 / 16.0,
 // 600 x 600 with 100 waves (600) 26.2 / 24.7, 700 x 700 with 100 waves (700) 28.0 / 28.8.
 constexpr long long kHalvesBlocks = 640;
+
+// How the rows of a grid are cut in a shape of two wavefronts per segment: whole segments,
+// and half segments at the rows' ends where the upper halves have no columns. Workgroups
+// take two segments of either kind.
+struct RowCut {
+  int whole_per_row;
+  long long whole_groups, end_groups;
+};
+inline RowCut row_cut(int N, const LaunchShape& s) {
+  const int columns = s.lanes_per_row * s.steps, tail = N % columns;
+  const long long rows = (N + 64 / s.lanes_per_row - 1) / (64 / s.lanes_per_row);
+  const bool half = tail > 0 && tail <= columns / 2;
+  RowCut c;
+  c.whole_per_row = N / columns + (tail > 0 && !half ? 1 : 0);
+  c.whole_groups = (c.whole_per_row * rows + 1) / 2;
+  c.end_groups = half ? (rows + 1) / 2 : 0;
+  return c;
+}
 
 // One workgroup's segment group of one patch.
 struct BatchUnit {
