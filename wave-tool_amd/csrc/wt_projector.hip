@@ -58,13 +58,41 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// v of lane kLane of each row of 16 lanes (DPP row_newbcast).
+// v of another lane of the row of 16, by a DPP control.
+template <int kCtrl>
+__device__ __forceinline__ double dpp(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, kCtrl, 0xf, 0xf, false);
+  const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), kCtrl, 0xf, 0xf, false);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// v of lane kLane of each row of 16 lanes (row_newbcast).
 template <int kLane>
 __device__ __forceinline__ double row_value(double v) {
-  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, 0x150 | kLane, 0xf, 0xf, false);
-  const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), 0x150 | kLane, 0xf, 0xf, false);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+  return dpp<0x150 | kLane>(v);
+}
+
+__device__ __forceinline__ double lesser(double a, double b) { return b < a ? b : a; }
+__device__ __forceinline__ double greater(double a, double b) { return b > a ? b : a; }
+
+// Least and greatest of v over the lanes 0-31 that are `in`, as NdcBounds forms them one by
+// one: NaN is passed over, unless the first lane holds it. Rows of 16 by DPP (quad_perm
+// neighbours and pairs, row_half_mirror, row_mirror), then the two rows.
+__device__ __forceinline__ void bounds(double v, bool in, int first, double* least, double* most) {
+  const bool use = in && v == v;
+  double a = use ? v : __builtin_inf(), b = use ? v : -__builtin_inf();
+  a = lesser(a, dpp<0xB1>(a));
+  b = greater(b, dpp<0xB1>(b));
+  a = lesser(a, dpp<0x4E>(a));
+  b = greater(b, dpp<0x4E>(b));
+  a = lesser(a, dpp<0x141>(a));
+  b = greater(b, dpp<0x141>(b));
+  a = lesser(a, dpp<0x140>(a));
+  b = greater(b, dpp<0x140>(b));
+  const double lead = lane_value(v, first);
+  *least = lead == lead ? lesser(lane_value(a, 0), lane_value(a, 16)) : lead;
+  *most = lead == lead ? greater(lane_value(b, 0), lane_value(b, 16)) : lead;
 }
 
 // The matrix whose column c lane first + c holds.
@@ -209,21 +237,20 @@ __device__ __forceinline__ int projector_corners_wave(const wt_camera& c, double
     inside = -amp <= fc.y && fc.y <= amp;
     point = fc;
   }
-  unsigned long long points = __ballot(inside);
+  const unsigned long long points = __ballot(inside);
   if (points == 0) return WT_ERR_NO_INTERSECTION;
   if (!aim_ok || !((regular_lanes >> 16) & 1)) return WT_ERR_DEGENERATE;
   const Vec4 ndc = mat_apply(pvp, Vec4{point.x, 0.0, point.z, 1.0});
   const double nx = ndc.x / ndc.w, ny = ndc.y / ndc.w;
-  NdcBounds b;
-  for (; points; points &= points - 1) {  // at most 32, most often 4 to 10
-    const int i = __builtin_ctzll(points);
-    b.add_ndc(lane_value(nx, i), lane_value(ny, i));
-  }
+  double xmin, xmax, ymin, ymax;
+  const int lead = __builtin_ctzll(points);
+  bounds(nx, inside, lead, &xmin, &xmax);
+  bounds(ny, inside, lead, &ymin, &ymax);
 
   // projector matrix: column (lane & 3) of inverse * range in each lane
   const int col = lane & 3;
-  const double range_col[4] = {col == 0 ? b.xmax - b.xmin : (col == 3 ? b.xmin : 0.0),
-                               col == 1 ? b.ymax - b.ymin : (col == 3 ? b.ymin : 0.0), col == 2 ? 1.0 : 0.0,
+  const double range_col[4] = {col == 0 ? xmax - xmin : (col == 3 ? xmin : 0.0),
+                               col == 1 ? ymax - ymin : (col == 3 ? ymin : 0.0), col == 2 ? 1.0 : 0.0,
                                col == 3 ? 1.0 : 0.0};
   double m_col[4];
   mul_column(gather_columns(a, 20), range_col, m_col);

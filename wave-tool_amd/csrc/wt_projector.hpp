@@ -229,10 +229,7 @@ struct NdcBounds {
 
   WT_HD void add_point(const Mat4& pvp, const Vec3& p) {
     const Vec4 q = mat_apply(pvp, Vec4{p.x, 0.0, p.z, 1.0});
-    add_ndc(q.x / q.w, q.y / q.w);
-  }
-
-  WT_HD void add_ndc(double nx, double ny) {
+    const double nx = q.x / q.w, ny = q.y / q.w;
     if (count++ == 0) {
       xmin = xmax = nx;
       ymin = ymax = ny;
