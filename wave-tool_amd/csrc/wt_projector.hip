@@ -10,7 +10,7 @@
 // and pitch): a third of the instructions. Past that every SIMD has work either way and a
 // thread per camera does less in all. Every value is formed by the same operations in
 // both, so they agree bit for bit. Measured per launch in a graph, wavefront / thread per
-// camera: 24 cameras 7.8 / 15.0 us, 512 8.4 / 15.1, 2048 12.2 / 15.2, 4096 20.0 / 15.2.
+// camera: 24 cameras 7.5 / 15.0 us, 512 8.2 / 15.1, 2048 11.6 / 15.2, 4096 20.0 / 15.2.
 #include "wt_kernels.hpp"
 #include "wt_projector.hpp"
 
