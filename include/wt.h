@@ -221,15 +221,19 @@ wt_status wt_vertex_varyings(wt_ctx* ctx, const wt_water_params* params, const w
                              const float* normals, uint64_t vertex_count, const wt_varying_buffers* out, void* stream);
 
 /* Overrides (or with all-zero fields, restores) the launch shape of the plain
- * forward kernel. Returns WT_ERR_INVALID_ARG for unsupported values. */
+ * forward kernel, which then runs as asked. Returns WT_ERR_INVALID_ARG for
+ * unsupported values. */
 wt_status wt_set_launch_config(wt_ctx* ctx, const wt_launch_config* cfg);
-/* The launch shape wt_water_displace would use for this problem size. */
+/* The launch shape wt_water_displace would use for this problem size. Where neither
+ * wt_set_launch_config nor the autotuner chose another, the library may take segments of
+ * this shape in halves (half the steps per lane, twice the wavefronts), all of them on
+ * small grids or those that end the rows, with the same results bit for bit. */
 wt_status wt_get_launch_config(wt_ctx* ctx, uint32_t grid_length, uint32_t wave_count, wt_launch_config* cfg);
 
 /* Times every supported launch shape (steps per lane, lanes per row and wave split,
  * i.e. vertices per workgroup, and the wave chunk) for (grid_length, wave_count) on the
- * context's device with synthetic inputs and stores the fastest in the
- * context's table (per size bucket). best_ms (may be NULL) receives its
+ * context's device with synthetic inputs, each as it is and the default as the library
+ * runs it, and stores the fastest in the context's table (per size bucket). best_ms (may be NULL) receives its
  * per-launch time. Allocates and frees its own scratch buffers. */
 wt_status wt_autotune_forward(wt_ctx* ctx, uint32_t grid_length, uint32_t wave_count, int with_heightmap,
                               wt_launch_config* best, float* best_ms);

@@ -67,11 +67,15 @@ bool valid_shape(const wt::LaunchShape& s) {
 
 wt::LaunchShape default_shape(uint32_t N) {
   // lanes per row no wider than the row, steps so one segment spans about a row
-  wt::LaunchShape s{2, 8, 64, 64};
+  wt::LaunchShape s{2, 8, 64, 64, true};
   if (N <= 64) s.lanes_per_row = 16;
   else if (N <= 256) s.lanes_per_row = 32;
   if (N <= 64) s.steps = 4;
   return s;
+}
+
+bool same_shape(const wt::LaunchShape& a, const wt::LaunchShape& b) {
+  return a.split == b.split && a.steps == b.steps && a.lanes_per_row == b.lanes_per_row && a.wave_chunk == b.wave_chunk;
 }
 
 wt::LaunchShape pick_shape(wt_ctx* ctx, uint32_t N, uint32_t W) {
@@ -444,6 +448,8 @@ static wt_status autotune_forward(wt_ctx* ctx, uint32_t N, uint32_t W, int with_
     }
     return WT_OK;
   };
+  // the default as the library runs it, and every shape as it is
+  std::vector<wt::LaunchShape> cands{dflt};
   const int splits[2] = {1, 2}, ks[3] = {4, 8, 16}, lcs[4] = {64, 32, 16, 8}, chunks[3] = {64, 32, 128};
   for (int var : splits)
     for (int k : ks)
@@ -451,38 +457,38 @@ static wt_status autotune_forward(wt_ctx* ctx, uint32_t N, uint32_t W, int with_
         for (int ch : chunks) {
           if ((uint32_t)lc > N && lc != 8) continue;
           const wt::LaunchShape cand{var, k, lc, ch};
-          if (!valid_shape(cand)) continue;
-          ctx->forced = true;
-          ctx->forced_shape = cand;
-          wt_status s0 = frames((int)nfl);  // first launches of this shape
-          if (s0 == WT_OK && hipStreamSynchronize(st[0]) != hipSuccess) s0 = WT_ERR_HIP;
-          if (s0 != WT_OK) {
-            ctx->forced = saved_forced;
-            ctx->forced_shape = saved_shape;
-            cleanup();
-            return s0 == WT_ERR_HIP ? fail(ctx, s0, "autotune launch") : s0;
-          }
-          WT_TRY(hipEventRecord(e0, st[0]));
-          s0 = frames(reps);
-          WT_TRY(hipEventRecord(e1, st[0]));
-          WT_TRY(hipEventSynchronize(e1));
-          if (s0 != WT_OK) {
-            ctx->forced = saved_forced;
-            ctx->forced_shape = saved_shape;
-            cleanup();
-            return s0 == WT_ERR_HIP ? fail(ctx, s0, "autotune launch") : s0;
-          }
-          float ms = 0.0f;
-          WT_TRY(hipEventElapsedTime(&ms, e0, e1));
-          ms /= reps;
-          if (cand.split == dflt.split && cand.steps == dflt.steps && cand.lanes_per_row == dflt.lanes_per_row &&
-              cand.wave_chunk == dflt.wave_chunk)
-            default_t = ms;
-          if (ms < best_t) {
-            best_t = ms;
-            best_s = cand;
-          }
+          if (valid_shape(cand)) cands.push_back(cand);
         }
+  for (const wt::LaunchShape& cand : cands) {
+    ctx->forced = true;
+    ctx->forced_shape = cand;
+    wt_status s0 = frames((int)nfl);  // first launches of this shape
+    if (s0 == WT_OK && hipStreamSynchronize(st[0]) != hipSuccess) s0 = WT_ERR_HIP;
+    if (s0 != WT_OK) {
+      ctx->forced = saved_forced;
+      ctx->forced_shape = saved_shape;
+      cleanup();
+      return s0 == WT_ERR_HIP ? fail(ctx, s0, "autotune launch") : s0;
+    }
+    WT_TRY(hipEventRecord(e0, st[0]));
+    s0 = frames(reps);
+    WT_TRY(hipEventRecord(e1, st[0]));
+    WT_TRY(hipEventSynchronize(e1));
+    if (s0 != WT_OK) {
+      ctx->forced = saved_forced;
+      ctx->forced_shape = saved_shape;
+      cleanup();
+      return s0 == WT_ERR_HIP ? fail(ctx, s0, "autotune launch") : s0;
+    }
+    float ms = 0.0f;
+    WT_TRY(hipEventElapsedTime(&ms, e0, e1));
+    ms /= reps;
+    if (cand.own) default_t = ms;
+    if (ms < best_t) {
+      best_t = ms;
+      best_s = cand;
+    }
+  }
 #undef WT_TRY
   // shapes within timing noise of each other trade places from run to run: keep the
   // default shape unless another is more than 3% faster
@@ -518,10 +524,10 @@ wt_status wt_autotune_save(wt_ctx* ctx, const char* path) {
   if (!ctx || !path) return WT_ERR_INVALID_ARG;
   FILE* f = std::fopen(path, "w");
   if (!f) return fail(ctx, WT_ERR_INVALID_ARG, std::string("cannot open ") + path);
-  std::fprintf(f, "# wt forward autotune: n_bucket w_bucket wave_split steps lanes_per_row wave_chunk\n");
+  std::fprintf(f, "# wt forward autotune: n_bucket w_bucket wave_split steps lanes_per_row wave_chunk own\n");
   for (const auto& kv : ctx->table)
-    std::fprintf(f, "%d %d %d %d %d %d\n", kv.first.first, kv.first.second, kv.second.split, kv.second.steps,
-                 kv.second.lanes_per_row, kv.second.wave_chunk);
+    std::fprintf(f, "%d %d %d %d %d %d %d\n", kv.first.first, kv.first.second, kv.second.split, kv.second.steps,
+                 kv.second.lanes_per_row, kv.second.wave_chunk, kv.second.own ? 1 : 0);
   std::fprintf(f, "# batched: b n_bucket w_bucket batch_shape\n");
   for (const auto& kv : ctx->batch_table) std::fprintf(f, "b %d %d %d\n", kv.first.first, kv.first.second, kv.second);
   std::fclose(f);
@@ -548,11 +554,16 @@ wt_status wt_autotune_load(wt_ctx* ctx, const char* path) {
       continue;
     }
     wt::LaunchShape s{};
-    if (std::sscanf(line, "%d %d %d %d %d %d", &nb, &wb, &s.split, &s.steps, &s.lanes_per_row, &s.wave_chunk) != 6 ||
-        !valid_shape(s)) {
+    int own = 0;
+    const int got =
+        std::sscanf(line, "%d %d %d %d %d %d %d", &nb, &wb, &s.split, &s.steps, &s.lanes_per_row, &s.wave_chunk, &own);
+    if (got < 6 || !valid_shape(s)) {
       std::fclose(f);
       return fail(ctx, WT_ERR_INVALID_ARG, "malformed autotune table");
     }
+    // tables of six columns hold the default's shape where the default was kept
+    const wt::LaunchShape dflt = default_shape(nb >= 0 && nb < 31 ? 1u << nb : 0u);
+    s.own = same_shape(s, dflt) && (got == 6 || own != 0);
     t[{nb, wb}] = s;
   }
   std::fclose(f);

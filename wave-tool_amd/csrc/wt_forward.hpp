@@ -654,21 +654,25 @@ hipError_t launch_batched_mode(const BatchArgs& a, hipStream_t st) {
 
 // ------------------------------------------------------------------ launch helpers
 
+// own: the shape is the library's choice (default_shape: 64 lanes per row, 32 up to sides of
+// 256), which may take segments in halves; a shape that was asked for runs as it is.
 template <int K, int LC, int S, int kTex, int CH = kChunk>
-hipError_t launch_t(const FwdParams& p, hipStream_t st) {
+hipError_t launch_t(const FwdParams& p, bool own, hipStream_t st) {
   constexpr int LR = 64 / LC;
   constexpr int kSegPerWG = kWavesPerWG / S;
   const long long row_groups = (p.N + LR - 1) / LR;
   const long long blocks = ((p.N + LC * K - 1) / (LC * K) * row_groups + kSegPerWG - 1) / kSegPerWG;
-  if constexpr (K == 8 && S == 2 && LC >= 16 && CH == kChunk) {
-    if (blocks <= kHalvesBlocks) {
+  if constexpr (K == 8 && S == 2 && LC >= 32 && CH == kChunk) {
+    if (own && blocks <= kHalvesBlocks) {
       constexpr int H = K / 2;
       const long long halves = ((p.N + LC * H - 1) / (LC * H) * row_groups + kSegPerWG - 1) / kSegPerWG;
       hipLaunchKernelGGL((water_forward_kernel<H, LC, S, kTex, CH, true>), dim3((unsigned)halves), dim3(256), 0, st, p);
       return hipGetLastError();
     }
+  }
+  if constexpr (K == 8 && S == 2 && LC == 64 && CH == kChunk) {
     const RowCut cut = row_cut(p.N, LaunchShape{S, K, LC, CH});
-    if (cut.end_groups > 0 && cut.whole_groups > 0) {
+    if (own && cut.end_groups > 0 && cut.whole_groups > 0) {
       hipLaunchKernelGGL((water_forward_tail_kernel<K, LC, kTex>), dim3((unsigned)(cut.whole_groups + cut.end_groups)),
                          dim3(256), 0, st, p, (int)cut.whole_groups);
       return hipGetLastError();
@@ -684,12 +688,12 @@ template <int kTex>
 hipError_t launch_forward_mode(const FwdParams& p, const LaunchShape& s, hipStream_t st) {
   auto by_split = [&](auto k_tag, auto lc_tag) -> hipError_t {
     constexpr int K = decltype(k_tag)::value, LC = decltype(lc_tag)::value;
-    if (s.split != 2) return launch_t<K, LC, 1, kTex>(p, st);
+    if (s.split != 2) return launch_t<K, LC, 1, kTex>(p, s.own, st);
     if constexpr (LC == 64) {  // the wave-chunk variants of the one-row shapes
-      if (s.wave_chunk == 32) return launch_t<K, LC, 2, kTex, 32>(p, st);
-      if (s.wave_chunk == 128) return launch_t<K, LC, 2, kTex, 128>(p, st);
+      if (s.wave_chunk == 32) return launch_t<K, LC, 2, kTex, 32>(p, s.own, st);
+      if (s.wave_chunk == 128) return launch_t<K, LC, 2, kTex, 128>(p, s.own, st);
     }
-    return launch_t<K, LC, 2, kTex>(p, st);
+    return launch_t<K, LC, 2, kTex>(p, s.own, st);
   };
   auto by_lc = [&](auto k_tag) -> hipError_t {
     switch (s.lanes_per_row) {

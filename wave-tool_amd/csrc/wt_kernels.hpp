@@ -27,6 +27,7 @@ struct LaunchShape {
   int steps;          // K: 4, 8, 16
   int lanes_per_row;  // LC: 64, 32, 16, 8
   int wave_chunk;     // waves per LDS pass (64 in this build)
+  bool own = false;   // the library's own choice for the size: segments may be taken in halves
 };
 
 hipError_t launch_forward(const FwdParams& p, const LaunchShape& s, hipStream_t st);
@@ -63,13 +64,16 @@ __host__ __device__ inline void set_corner_algebra(D& d, const double (*c)[4]) {
   d.duv_z = c[3][2] - c[1][2] - c[2][2] + c[0][2];
 }
 
-// Launches of up to this many workgroups take segments of 8 steps and two wavefronts in
-// halves of 4 steps, a pair of wavefronts each: they leave SIMDs idle, and a wavefront's
+// Launches of up to this many workgroups whose shape is the library's own choice take
+// segments of 8 steps and two wavefronts in halves of 4 steps, a pair of wavefronts each: they leave SIMDs idle, and a wavefront's
 // chain of sums and vertices, which bounds them, is about half as long (the upper half
 // repeats the lower one's sequence). Above, the repeated work costs more than the idle
-// SIMDs. Whole / in halves, us per launch in a graph: 128 x 128 with 16 waves 5.3 / 4.5,
-// 256 x 256 with 100 waves 15.4 / 12.5, 513 x 513 with 64 waves (513 workgroups) 17.9 / 16.0,
-// 600 x 600 with 100 waves (600) 26.2 / 24.7, 700 x 700 with 100 waves (700) 28.0 / 28.8.
+// SIMDs. Whole / in halves, us per launch in a graph: 128 x 128 with 16 waves 5.9 / 5.1,
+// 256 x 256 with 100 waves 16.4 / 13.1, 513 x 513 with 64 waves (513 workgroups) 17.0 / 15.0,
+// 600 x 600 with 100 waves (600) 26.2 / 22.7; 700 x 700 with 100 waves (700) 28.0 / 28.8. Per
+// launch with two frames in flight: 4.9 / 4.7, 9.9 / 8.0, 10.4 / 9.7, 16.2 / 15.7, and 512 x 512
+// with 100 waves (256) 10.2 / 10.3; with three, 512 x 512 loses (8.4 / 9.7): what
+// wt_autotune_forward_overlapped is for, which times whole segments too.
 constexpr long long kHalvesBlocks = 640;
 
 // How the rows of a grid are cut in a shape of two wavefronts per segment: whole segments,
