@@ -108,6 +108,18 @@ def test_own_choice_equals_whole_segments(torch_cuda, wtctx, side, waves, kernel
     assert torch.isfinite(a).all() and torch.equal(a, b)
 
 
+@pytest.mark.parametrize("side,waves,tail", [(641, 31, False), (768, 4, False), (768, 32, True), (1025, 1, True)])
+def test_few_waves_end_rows_in_whole_segments(torch_cuda, wtctx, side, waves, tail):
+    """Where every workgroup of whole segments runs at once, half segments at the rows' ends pay from 32 waves on."""
+    torch = torch_cuda
+    params, w, kw = scene(torch, side, waves)
+    out = [torch.empty(3 * side * side, device="cuda") for _ in range(2)]
+    wtctx.displace(params, w, *out)
+    torch.cuda.synchronize()
+    name, _ = launched(torch, lambda s: wtctx.displace(params, w, *out, stream=s))
+    assert ("tail_kernel" in name) == tail, name
+
+
 def test_tuned_shapes_run_as_they_were_timed(torch_cuda, tmp_path):
     """A table says whether a size keeps the library's choice; tables of six columns do where they hold its shape."""
     torch = torch_cuda

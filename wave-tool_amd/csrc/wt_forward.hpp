@@ -531,8 +531,7 @@ __global__ __launch_bounds__(256) void water_forward_kernel(FwdParams p) {
 // Rows that end in the lower half of a segment: whole segments in the first `whole`
 // workgroups, the halves at the rows' ends in the others, which as whole segments sum and
 // sample columns past the edge (per launch in a graph, so / in halves: 700 x 700 with 64
-// waves 20.5 / 18.5 us, 1100 x 1100 with 100 waves 54.9 / 48.5; with 4 waves 8.75 / 8.77 and
-// 15.6 / 14.2).
+// waves 18.5 / 16.2 us, 1100 x 1100 with 64 waves 35.1 / 31.7, with 4 waves 18.2 / 16.7).
 template <int K, int LC, int kTex>
 __global__ __launch_bounds__(256, 4) void water_forward_tail_kernel(FwdParams p, int whole) {
   static_assert(sizeof(SegShared<K / 2, LC, 2>) <= sizeof(SegShared<K, LC, 2>), "one allocation for both");
@@ -672,7 +671,7 @@ hipError_t launch_t(const FwdParams& p, bool own, hipStream_t st) {
   }
   if constexpr (K == 8 && S == 2 && LC == 64 && CH == kChunk) {
     const RowCut cut = row_cut(p.N, LaunchShape{S, K, LC, CH});
-    if (own && cut.end_groups > 0 && cut.whole_groups > 0) {
+    if (own && cut.end_groups > 0 && cut.whole_groups > 0 && (blocks > kOneRoundBlocks || p.W >= kRowEndWaves)) {
       hipLaunchKernelGGL((water_forward_tail_kernel<K, LC, kTex>), dim3((unsigned)(cut.whole_groups + cut.end_groups)),
                          dim3(256), 0, st, p, (int)cut.whole_groups);
       return hipGetLastError();

@@ -76,6 +76,16 @@ __host__ __device__ inline void set_corner_algebra(D& d, const double (*c)[4]) {
 // wt_autotune_forward_overlapped is for, which times whole segments too.
 constexpr long long kHalvesBlocks = 640;
 
+// Past that, rows that end in the lower half of a segment end in half segments
+// (water_forward_tail_kernel), but up to this many workgroups, four to a CU, only from
+// kRowEndWaves waves on: all of whole segments run at once there, and the sums past the
+// edge, which the halves save, cost them less than the second kind of workgroup. Whole /
+// with halves, us per launch in a graph: 768 x 768 with 1 wave 9.3 / 9.6, 16 waves 10.1 / 10.9,
+// 32 waves 12.6 / 12.5, 64 waves 18.6 / 16.3; 1025 x 1025 (1538 workgroups) with 1 wave
+// 16.3 / 14.9, 16 waves 18.3 / 17.6.
+constexpr long long kOneRoundBlocks = 1024;
+constexpr int kRowEndWaves = 32;
+
 // How the rows of a grid are cut in a shape of two wavefronts per segment: whole segments,
 // and half segments at the rows' ends where the upper halves have no columns. Workgroups
 // take two segments of either kind.
