@@ -48,7 +48,9 @@
 //   rows are consecutive in memory and 64 parts are read side by side, so a sum over 256
 //   parts is one round of loads (a workgroup per row took 58 us for the
 //   256-problem batch, 24 so).
-// Both kernels find their problem through a unit (reduce block) -> problem map built at
+// adjoint_few_kernel: the same for problems of up to 4 waves (6 where they are small), on the
+//   VALU (fit_few).
+// All find their problem through a unit (reduce block) -> problem map built at
 // creation, so one launch per wave-count class covers a whole batch; a single problem is
 // a table of one. A problem's blocks and the order of every sum depend on the problem
 // alone, so a batch repeats the bits of its problems run one by one.
@@ -73,6 +75,31 @@ struct FitWaveLds {
 struct FitWaveGrad {
   float A, Q, Dx, Dz, w, wL, om2L;  // wL = w / L, om2L = omega / (2 L)
 };
+
+// One wave's constants from its parameters, in FP64, rounded once.
+struct FitWave {
+  FitWaveLds lds;
+  FitWaveGrad grad;
+  float bx, by, bz;  // Q A Dx, A, Q A Dz
+  float2 dir;        // Q Dx, Q Dz
+};
+__device__ __forceinline__ FitWave fit_wave(const FitDesc& P, const float (&p)[5]) {
+  const double A = p[0], L = p[1] > 1e-3f ? p[1] : 1e-3f, al = p[2], Q = p[3], ph0 = p[4];
+  const double w = kTwoPi / L, om = sqrt(P.g * w);
+  double sa, ca;
+  sincos(al, &sa, &ca);
+  FitWave o;
+  o.lds.kx = w * ca * kInvTwoPi;
+  o.lds.kz = w * sa * kInvTwoPi;
+  o.lds.c0 = __builtin_amdgcn_fract(fma(om, P.t0, ph0) * kInvTwoPi);
+  o.lds.om = om * kInvTwoPi;
+  o.bx = (float)(Q * A * ca);
+  o.by = (float)A;
+  o.bz = (float)(Q * A * sa);
+  o.dir = make_float2((float)(Q * ca), (float)(Q * sa));
+  o.grad = FitWaveGrad{(float)A, (float)Q, (float)ca, (float)sa, (float)w, (float)(w / L), (float)(om / (2.0 * L))};
+  return o;
+}
 
 // Sum over the 64 lanes of a wavefront with DPP moves (VALU only, fixed order); the
 // total lands in lane 63. quad_perm [1,0,3,2] and [2,3,0,1] give quad sums,
@@ -203,6 +230,14 @@ constexpr float kFitTrigScale = 16.0f;  // scale of E in its fragments
 // the largest.
 constexpr float kFitResLow = 1.0f, kFitResHigh = 32768.0f;
 
+// What the wavefronts of a workgroup leave of a part: per wavefront, chunk and lane two of
+// the part's running sums of wave lane mod 16, and the loss.
+template <int KMAX, int NW>
+struct FitSums {
+  float2 sums[NW][KMAX][64];
+  float loss[NW];
+};
+
 constexpr int kRunFloats = 52;  // a run of 48 target floats, padded: rows of eight pairs on different banks
 
 // The workgroup's LDS for up to KMAX chunks of 16 waves (`chunks` of them in use).
@@ -211,7 +246,6 @@ constexpr int kRunFloats = 52;  // a run of 48 target floats, padded: rows of ei
 //    dimension of 32 (hi, then lo); a last odd chunk takes it as [hi | lo] of its 16 waves.
 //    fwd [16 offsets][cos / sin][chunk][lane], bwd [chunk][cos / sin][plain / times
 //    t + 1/2][hi / lo][lane].
-//  sums: per wavefront, chunk and lane two of the part's running sums of wave lane mod 16.
 //  time: exp(i omega s dt), [snapshot][wave] (cos, sin), then a row of zeros for the pairs
 //    past the last; rows padded by 16 bytes to keep the 16-byte reads of eight neighbouring
 //    rows on different banks.
@@ -225,10 +259,9 @@ struct FitShared {
   FitWaveLds wave[16 * KMAX];
   FitWaveGrad grad[16 * KMAX];
   uint32_t max;  // bits of the largest coefficient magnitude
-  float loss[NW];
   alignas(16) float row[NW][kTable ? 4 * 32 * KMAX : 4];
   alignas(16) float time[kTable ? (kFitMaxSnapshots + 1) * (32 * KMAX + 4) : 4];
-  float2 sums[NW][KMAX][64];
+  FitSums<KMAX, NW> end;
   alignas(16) float run[NW][kTable ? 16 * kRunFloats : 4];
   Half8 fwd[2 * 2 * KMAX * 64];
   Half8 bwd[KMAX * 2 * 2 * 2 * 64];
@@ -316,6 +349,63 @@ __device__ __forceinline__ void unshuffle(float* run, int n16, int g, int at, fl
   wavefront_lds_sync();
 }
 
+// The end of a round of parts: the wavefronts' sums in index order, then the parameter
+// derivatives and the loss of every part. Returns the parts that ran side by side.
+template <int KMAX, int NW>
+__device__ __forceinline__ int finish_parts(const FitDesc& P, const FitSums<KMAX, NW>& of, const FitWaveGrad* grad,
+                                            double x_mid, int part, int part_end, int end, int lane, int wid) {
+  __syncthreads();
+  const int waves_per = min(P.tiles_per_block, NW), side_by = NW >> __builtin_ctz(waves_per);
+  const int wave_rows = (P.W + 63) >> 6;
+#pragma unroll 1
+  for (int it = wid; it < side_by * wave_rows; it += NW) {
+    int wi = lane;
+    asm volatile("" : "+v"(wi));  // keeps this block's addresses out of the tile loop's live registers
+    const int mine = wave_rows > 1 ? it >> 1 : it;
+    if (wave_rows > 1) wi += 64 * (it & 1);
+    const int w0 = mine * waves_per;
+    if (part_end - max(P.tiles_per_block, NW) + w0 >= end || wi >= P.W) continue;  // no such part
+    double v[8];
+    auto sum_waves = [&](auto whole) {  // the part's wavefronts, all loads in flight together
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float2* from = &of.sums[whole ? 0 : w0][wi >> 4][16 * r + (wi & 15)];
+        float2 t = *from;
+#pragma unroll
+        for (int i = 1; i < (whole ? NW : NW / 2); ++i) {
+          const float2 u = from[(whole || i < waves_per ? i : 0) * (KMAX * 64)];
+          t.x += whole || i < waves_per ? u.x : 0.0f;
+          t.y += whole || i < waves_per ? u.y : 0.0f;
+        }
+        const int k = ((r & 1) << 1) | (r >> 1);
+        v[k] = (double)t.x;
+        v[4 + k] = (double)t.y;
+      }
+    };
+    if (waves_per == NW) sum_waves(std::true_type{});
+    else sum_waves(std::false_type{});
+    const FitWaveGrad w = grad[wi];
+    // sums of r . dd/dtheta: plain, times t, times the world x and z
+    const double A = w.A, Dx = w.Dx, Dz = w.Dz;
+    const double g0 = A * v[3], gt = A * fma(P.t0, v[3], P.dt * v[4]);
+    const double gx = A * fma(x_mid, v[3], P.spacing * v[6]);
+    const double gz = A * fma(P.z0, v[3], P.spacing * v[5]);
+    const double sec = fma(Dx, v[0], Dz * v[1]), sepc = fma(Dx, v[1], -(Dz * v[0]));
+    const float out[5] = {(float)fma((double)w.Q, sec, v[2]),
+                          (float)-fma((double)w.wL, fma(Dx, gx, Dz * gz), w.om2L * gt),
+                          (float)fma((double)w.w, fma(Dx, gz, -(Dz * gx)), w.Q * A * sepc), (float)(A * sec), (float)g0};
+    float* o = P.partials + (size_t)(part + mine) * (5 * P.W + 1);
+#pragma unroll
+    for (int k = 0; k < 5; ++k) o[5 * wi + k] = out[k];
+    if (wi == 0) {
+      float t = of.loss[w0];
+      for (int i = w0 + 1; i < w0 + waves_per; ++i) t += of.loss[i];
+      o[5 * P.W] = t;
+    }
+  }
+  return side_by;
+}
+
 // A unit's tiles and the sums of its parts. Lane (n16, g) works in the forward pass on
 // pair n16, the column offsets t = 16 mt + 4 g + r and the waves 4 g + u of a chunk; after the
 // backward contraction on wave n16 of a chunk and the pairs 4 g + r. kTable: P from the
@@ -343,7 +433,7 @@ __device__ __forceinline__ void fit_tiles(const FitDesc& P, const FitUnit& unit,
   const float inv_fwd = pow2f(-coef_exp) * (1.0f / kFitTrigScale), neg_half = -0.5f * fwd_scale;
   const double x_mid = P.x0 + ((double)col0 + 31.5) * P.spacing;  // the strip's centre
 
-  for (int kc = 0; kc < chunks; ++kc) sh.sums[wid][kc][lane] = make_float2(0.0f, 0.0f);
+  for (int kc = 0; kc < chunks; ++kc) sh.end.sums[wid][kc][lane] = make_float2(0.0f, 0.0f);
   float sq = 0.0f;
 
 
@@ -605,7 +695,7 @@ __device__ __forceinline__ void fit_tiles(const FitDesc& P, const FitUnit& unit,
         // 0, 2, 1, 3 and 4, 6, 5 and a zero
         const float lo = swap16_sum(swap32_sum(t[0], t[1]), swap32_sum(t[2], t[3]));
         const float hi = swap16_sum(swap32_sum(t[4], t[5]), swap32_sum(t[6], 0.0f));
-        float2* o = &sh.sums[wid][kc][lane];
+        float2* o = &sh.end.sums[wid][kc][lane];
         const float2 old = *o;
         *o = make_float2(fmaf(lo, inv_g, old.x), fmaf(hi, inv_g, old.y));
       }
@@ -613,68 +703,273 @@ __device__ __forceinline__ void fit_tiles(const FitDesc& P, const FitUnit& unit,
     }
     if (base + NW < part_end && base + NW < end) continue;
 
-    // ---- the end of a part: the wavefronts' sums in index order, then the parameter
-    // derivatives of the part
+    // ---- the end of a part
     const float lsum = wave_sum63(sq);
-    if (lane == 63) sh.loss[wid] = lsum;
+    if (lane == 63) sh.end.loss[wid] = lsum;
     sq = 0.0f;
-    __syncthreads();
-    const int waves_per = min(P.tiles_per_block, NW), side_by = NW >> __builtin_ctz(waves_per);
-    const int wave_rows = (P.W + 63) >> 6;
-#pragma unroll 1
-    for (int it = wid; it < side_by * wave_rows; it += NW) {
-      int wi = lane;
-      asm volatile("" : "+v"(wi));  // keeps this block's addresses out of the tile loop's live registers
-      const int mine = wave_rows > 1 ? it >> 1 : it;
-      if (wave_rows > 1) wi += 64 * (it & 1);
-      const int w0 = mine * waves_per;
-      if (part_end - max(P.tiles_per_block, NW) + w0 >= end || wi >= P.W) continue;  // no such part
-      double v[8];
-      auto sum_waves = [&](auto whole) {  // the part's wavefronts, all loads in flight together
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float2* from = &sh.sums[whole ? 0 : w0][wi >> 4][16 * r + (wi & 15)];
-          float2 t = *from;
-#pragma unroll
-          for (int i = 1; i < (whole ? NW : NW / 2); ++i) {
-            const float2 u = from[(whole || i < waves_per ? i : 0) * (KMAX * 64)];
-            t.x += whole || i < waves_per ? u.x : 0.0f;
-            t.y += whole || i < waves_per ? u.y : 0.0f;
-          }
-          const int k = ((r & 1) << 1) | (r >> 1);
-          v[k] = (double)t.x;
-          v[4 + k] = (double)t.y;
-        }
-      };
-      if (waves_per == NW) sum_waves(std::true_type{});
-      else sum_waves(std::false_type{});
-      const FitWaveGrad w = sh.grad[wi];
-      // sums of r . dd/dtheta: plain, times t, times the world x and z
-      const double A = w.A, Dx = w.Dx, Dz = w.Dz;
-      const double g0 = A * v[3], gt = A * (P.t0 * v[3] + P.dt * v[4]);
-      const double gx = A * (x_mid * v[3] + P.spacing * v[6]);
-      const double gz = A * (P.z0 * v[3] + P.spacing * v[5]);
-      const double sec = Dx * v[0] + Dz * v[1], sepc = Dx * v[1] - Dz * v[0];
-      const float out[5] = {(float)(w.Q * sec + v[2]), (float)-(w.wL * (Dx * gx + Dz * gz) + w.om2L * gt),
-                            (float)(w.w * (Dx * gz - Dz * gx) + w.Q * A * sepc), (float)(A * sec), (float)g0};
-      float* o = P.partials + (size_t)(part + mine) * (5 * P.W + 1);
-#pragma unroll
-      for (int k = 0; k < 5; ++k) o[5 * wi + k] = out[k];
-      if (wi == 0) {
-        float t = sh.loss[w0];
-        for (int i = w0 + 1; i < w0 + waves_per; ++i) t += sh.loss[i];
-        o[5 * P.W] = t;
-      }
-    }
+    const int side_by = finish_parts(P, sh.end, sh.grad, x_mid, part, part_end, end, lane, wid);
     __syncthreads();  // the sums have been read
-    for (int kc = 0; kc < chunks; ++kc) sh.sums[wid][kc][lane] = make_float2(0.0f, 0.0f);
+    for (int kc = 0; kc < chunks; ++kc) sh.end.sums[wid][kc][lane] = make_float2(0.0f, 0.0f);
     part += side_by;
     part_end += max(P.tiles_per_block, NW);
   }
 }
 
+// ---- few waves
+// A chunk of 16 waves would be mostly padding, and its tables and LDS leave two wavefronts
+// on a SIMD, too few to keep the targets coming. Here the sums run on the VALU in FP32: a
+// lane takes one column of the strip and steps through the pairs of the tile, theta's
+// cosine and sine being a column factor (the lane's, in registers) times P (the pair's, a
+// sine and cosine per lane for 64 of them, read back from LDS by the whole wavefront). The
+// targets of a pair are one 768-byte run; a tile's are loaded while the one before it is
+// summed, the first before the waves' constants are formed. Everything is a stated fused or
+// single operation, so that the two kernels that hold it give the same bits.
+// What bounds it: small problems the chain of loads, set-up, one tile and the part's end
+// (64 x 64 x 4 snapshots, 1 wave: 4.7 us, and the reduction 1.8), large ones the targets'
+// traffic (200 problems of 256 x 256 x 16, 1 wave: 5.7 TB/s) and, from 3 waves on, the sums.
+// Four wavefronts to a workgroup, not eight (5.3 us for the small problem), tiles of 4 and 8
+// pairs, not 16 (8.5 us with its reduction, where it takes 7.3), and a tile's rows formed by
+// its lanes and read by lane, not stepped through in scalar registers (7.7).
+template <int NW>
+struct FitFewShared {
+  FitWaveLds wave[8];
+  FitWaveGrad grad[kFitFewWavesSmall];
+  float4 coef[kFitFewWavesSmall];  // Q A Dx, A, Q A Dz
+  float2 dir[kFitFewWavesSmall];   // Q Dx, Q Dz
+  float2 column[kFitFewWavesSmall][kStrip];  // cos, sin of kx times the column's offset from the strip's centre
+  alignas(16) float2 phase[NW][64];  // P, [pair][wave], 4 or 8 waves to a pair
+  FitSums<1, NW> end[2];  // by turns: a part's sums are read while the next part's are formed
+};
+
+// The row of pair q = j S + s by a multiply-high: exact for q < 2^18, S <= 32.
+struct RowOf {
+  uint32_t magic;
+  bool one;
+  __device__ __forceinline__ explicit RowOf(int S) : magic(0xffffffffu / (uint32_t)S + 1u), one(S == 1) {}
+  __device__ __forceinline__ uint32_t operator()(uint32_t q) const { return one ? q : __umulhi(q, magic); }
+};
+
+// The pairs of a tile, pair i in every lane l with l mod kPairs = i.
+template <int kPairs>
+struct PairLanes {
+  int row;       // s n + j, the pair's row in the target; the last one's past the last pair
+  float j, s;
+  __device__ __forceinline__ PairLanes(const FitDesc& P, const RowOf& row_of, int tile, int lane) {
+    const uint32_t q = (uint32_t)(tile * kPairs + (lane & (kPairs - 1)));
+    const int jj = (int)row_of(q), ss = (int)q - jj * P.S;
+    row = ss * P.n + min(jj, P.n - 1);
+    j = (float)jj;
+    s = (float)ss;
+  }
+};
+
+// The lane's column of a strip's targets, clamped to the grid.
+struct TargetColumn {
+  const float* strip;  // the strip's first column in row 0, snapshot 0
+  size_t row;          // floats of a row
+  uint32_t lane_bytes;
+  __device__ __forceinline__ TargetColumn(const FitDesc& P, int strip_index, int lane) {
+    const int col0 = strip_index * kStrip;
+    strip = P.target + 3 * (size_t)col0;
+    row = 3 * (size_t)P.n;
+    lane_bytes = 12u * (uint32_t)min(lane, P.n - 1 - col0);
+  }
+  __device__ __forceinline__ Target3 load(int row_index) const {  // the same for the wavefront
+    const char* base = reinterpret_cast<const char*>(strip + (size_t)(uint32_t)row_index * row);
+    return *reinterpret_cast<const Target3*>(base + lane_bytes);
+  }
+};
+
+// v, the same in every lane, in a scalar register.
+__device__ __forceinline__ float uniform(float v) {
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+
+template <int kPairs, int kW, int NW>
+__device__ __forceinline__ void few_tiles(const FitDesc& P, const FitUnit& unit, const RowOf& row_of, FitFewShared<NW>& sh,
+                                          TargetColumn targets, Target3 (&next)[8], int tid) {
+  constexpr int kStride = kW <= 4 ? 4 : 8;
+  const int lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t pairs = (uint32_t)P.n * (uint32_t)P.S;
+  const int tiles = (int)((pairs + kPairs - 1) / kPairs);
+  const int first = unit.part * P.tiles_per_block, end = min(tiles, first + unit.parts * P.tiles_per_block);
+  const int col0 = unit.strip * kStrip;
+  const bool in_grid = lane < P.n - col0;
+  const float offset = (float)lane - 31.5f, half = in_grid ? 0.5f : 0.0f;
+  const double x_mid = fma((double)col0 + 31.5, P.spacing, P.x0);
+  // column factors (zero past the grid: such a lane's sums stay zero) and coefficients
+  float ec[kW], es[kW], bx[kW], by[kW], bz[kW], qx[kW], qz[kW];
+#pragma unroll
+  for (int w = 0; w < kW; ++w) {
+    const float2 e = sh.column[w][lane];
+    ec[w] = in_grid ? e.x : 0.0f;
+    es[w] = in_grid ? e.y : 0.0f;
+    const float4 b = sh.coef[w];
+    bx[w] = uniform(b.x);
+    by[w] = uniform(b.y);
+    bz[w] = uniform(b.z);
+    qx[w] = uniform(sh.dir[w].x);
+    qz[w] = uniform(sh.dir[w].y);
+  }
+  // per wave: sums of r_x cos, r_z cos, r_y sin, and of h = r_y cos - Q (D . r) sin plain,
+  // times s and times j
+  float t[kW][6];
+#pragma unroll
+  for (int w = 0; w < kW; ++w)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) t[w][k] = 0.0f;
+  float sq = 0.0f;
+
+  int part = unit.strip * P.blocks_per_strip + unit.part, part_end = first + max(P.tiles_per_block, NW);
+  int slot = 0, turn = 0;
+  PairLanes<kPairs> ahead(P, row_of, first + wid, lane);
+#pragma unroll 1
+  for (int base = first; base < end; base += NW) {
+    const int tile = base + wid;
+    if (tile < end) {
+      if (slot == 0) {  // P of this tile's pairs and of the wavefront's next tiles'
+        int l = lane;
+        asm volatile("" : "+v"(l));  // keeps the wave's constants out of the tile loop's live registers
+        const uint32_t i = (uint32_t)(l / kStride);
+        const uint32_t q = ((uint32_t)tile + i / kPairs * NW) * (uint32_t)kPairs + i % kPairs;
+        const uint32_t j = row_of(q), sn = q - j * (uint32_t)P.S;
+        const FitWaveLds& w = sh.wave[l & (kStride - 1)];
+        const double z = fma((double)j, P.spacing, P.z0), ts = (double)sn * P.dt;
+        float c, s;
+        sincos_turn(fma(w.om, ts, fma(w.kz, z, fma(w.kx, x_mid, w.c0))), &c, &s);
+        const float live = q < pairs ? 1.0f : 0.0f;
+        wavefront_lds_sync();  // the last ones have been read
+        sh.phase[wid][l] = make_float2(c * live, s * live);
+        wavefront_lds_sync();
+      }
+      // the targets to load meanwhile are the next tile's or, after the last, one place over
+      // and over
+      const PairLanes<kPairs> now = ahead;
+      if (tile + NW < end)
+        ahead = PairLanes<kPairs>(P, row_of, tile + NW, lane);
+      else
+        targets.lane_bytes = 0u;
+#pragma unroll
+      for (int i = 0; i < kPairs; ++i) {
+        const float2* phase = &sh.phase[wid][kStride * (slot + i)];
+        float c[kW], s[kW], rx = -next[i].v[0], ry = -next[i].v[1], rz = -next[i].v[2];
+#pragma unroll
+        for (int w = 0; w < kW; ++w) {
+          const float2 p = phase[w];
+          c[w] = fmaf(-es[w], p.y, ec[w] * p.x);
+          s[w] = fmaf(es[w], p.x, ec[w] * p.y);
+          rx = fmaf(bx[w], c[w], rx);
+          ry = fmaf(by[w], s[w], ry);
+          rz = fmaf(bz[w], c[w], rz);
+        }
+        next[i] = targets.load(__builtin_amdgcn_readlane(ahead.row, i));
+        const float r2 = fmaf(rz, rz, fmaf(ry, ry, rx * rx));
+        sq = fmaf((uint32_t)(tile * kPairs + i) < pairs ? half : 0.0f, r2, sq);
+        const float jf = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(now.j), i));
+        const float sf = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(now.s), i));
+#pragma unroll
+        for (int w = 0; w < kW; ++w) {
+          t[w][0] = fmaf(rx, c[w], t[w][0]);
+          t[w][1] = fmaf(rz, c[w], t[w][1]);
+          t[w][2] = fmaf(ry, s[w], t[w][2]);
+          const float d = fmaf(qx[w], rx, qz[w] * rz);
+          const float h = fmaf(-d, s[w], ry * c[w]);
+          t[w][3] += h;
+          t[w][4] = fmaf(sf, h, t[w][4]);
+          t[w][5] = fmaf(jf, h, t[w][5]);
+        }
+        if ((i & 1) || kW > 4) __builtin_amdgcn_sched_barrier(0);  // every pair's P at once would not fit the registers
+      }
+      slot = (slot + kPairs) & (64 / kStride - 1);
+    }
+    if (base + NW < part_end && base + NW < end) continue;
+
+    // ---- the end of a part: a wavefront's sums, row k of 16 lanes holding sums 0, 2, 1, 3
+    // and 4, 6, 5 and a zero
+    FitSums<1, NW>& of = sh.end[turn];
+    const float lsum = wave_sum63(sq);
+    if (lane == 63) of.loss[wid] = lsum;
+    sq = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kW; ++w) {
+      const float lo = row_sum(swap16_sum(swap32_sum(t[w][0], t[w][1]), swap32_sum(t[w][2], t[w][3])));
+      const float hi = row_sum(swap16_sum(swap32_sum(t[w][4], t[w][5]), swap32_sum(t[w][3] * offset, 0.0f)));
+      if ((lane & 15) == w) of.sums[wid][0][lane] = make_float2(lo, hi);
+#pragma unroll
+      for (int k = 0; k < 6; ++k) t[w][k] = 0.0f;
+    }
+    part += finish_parts(P, of, sh.grad, x_mid, part, part_end, end, lane, wid);
+    part_end += max(P.tiles_per_block, NW);
+    turn ^= 1;
+  }
+}
+
+// A unit of a problem of few waves, by NW wavefronts of a workgroup.
+template <int NW>
+__device__ __forceinline__ void fit_few(const FitDesc& P, const FitUnit& unit, const float (&params)[5],
+                                        FitFewShared<NW>& sh, int tid) {
+  const int lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  Target3 next[8];
+  const RowOf row_of(P.S);
+  const bool wide = P.tile_pairs == 8;
+  const TargetColumn targets(P, unit.strip, lane);
+  auto first_targets = [&](auto count) {
+    const PairLanes<count> at(P, row_of, unit.part * P.tiles_per_block + wid, lane);
+#pragma unroll
+    for (int i = 0; i < count; ++i) next[i] = targets.load(__builtin_amdgcn_readlane(at.row, i));
+  };
+  if (wide) first_targets(std::integral_constant<int, 8>{});
+  else first_targets(std::integral_constant<int, 4>{});
+  if (tid < 8) {
+    FitWave w{};
+    if (tid < P.W) w = fit_wave(P, params);
+    sh.wave[tid] = w.lds;
+    if (tid < kFitFewWavesSmall) {
+      sh.grad[tid] = w.grad;
+      sh.coef[tid] = make_float4(w.bx, w.by, w.bz, 0.0f);
+      sh.dir[tid] = w.dir;
+    }
+  }
+  __syncthreads();
+  static_assert(kStrip == 64, "a lane per column");
+  for (int w = wid; w < kFitFewWavesSmall && w < ((P.W + 1) & ~1); w += NW) {
+    float c, s;
+    sincos_turn(sh.wave[w].kx * P.spacing * ((double)lane - 31.5), &c, &s);
+    sh.column[w][lane] = make_float2(c, s);
+  }
+  __syncthreads();
+  if (wide) {
+    switch (P.W) {
+      case 1: few_tiles<8, 1>(P, unit, row_of, sh, targets, next, tid); break;
+      case 2: few_tiles<8, 2>(P, unit, row_of, sh, targets, next, tid); break;
+      case 3: few_tiles<8, 3>(P, unit, row_of, sh, targets, next, tid); break;
+      default: few_tiles<8, kFitFewWaves>(P, unit, row_of, sh, targets, next, tid); break;
+    }
+  } else {
+    switch (P.W) {
+      case 1: few_tiles<4, 1>(P, unit, row_of, sh, targets, next, tid); break;
+      case 2: few_tiles<4, 2>(P, unit, row_of, sh, targets, next, tid); break;
+      case 3: few_tiles<4, 3>(P, unit, row_of, sh, targets, next, tid); break;
+      case 4: few_tiles<4, 4>(P, unit, row_of, sh, targets, next, tid); break;
+      default: few_tiles<4, kFitFewWavesSmall>(P, unit, row_of, sh, targets, next, tid); break;
+    }
+  }
+}
+
+__global__ __launch_bounds__(64 * kFitFewWavefronts) __attribute__((amdgpu_waves_per_eu(4)))
+void adjoint_few_kernel(const FitDesc* __restrict__ probs, const FitUnit* __restrict__ units, int bump_step) {
+  __shared__ FitFewShared<kFitFewWavefronts> sh;
+  const FitUnit unit = load_uniform(units, (long long)blockIdx.x);
+  const FitDesc P = load_uniform(probs, unit.problem);
+  if (bump_step && unit.strip == 0 && unit.part == 0 && threadIdx.x == 0) atomicAdd(P.step, 1);  // as in adjoint_kernel
+  const float* pr = P.params + 5 * min((int)threadIdx.x, P.W - 1);
+  const float params[5] = {pr[0], pr[1], pr[2], pr[3], pr[4]};
+  fit_few(P, unit, params, sh, (int)threadIdx.x);
+}
+
 // One workgroup: a unit's strip and parts. KMAX bounds the problem's chunks of 16 waves.
-template <int KMAX, int NW, bool kTable>
+// kFew: units of problems of few waves are among them.
+template <int KMAX, int NW, bool kTable, bool kFew>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4)))
 void adjoint_kernel(const FitDesc* __restrict__ probs, const FitUnit* __restrict__ units, int bump_step) {
   __shared__ FitShared<KMAX, NW, kTable> sh;
@@ -690,8 +985,22 @@ void adjoint_kernel(const FitDesc* __restrict__ probs, const FitUnit* __restrict
 
   // ---- the waves' constants, one thread per wave; the parameters' loads first, so that
   // they are not waited for behind the targets'
-  const float* pr = P.params + 5 * min(tid, P.W - 1);
-  const float p0 = pr[0], p1 = pr[1], p2 = pr[2], p3 = pr[3], p4 = pr[4];
+  const float* pr = P.params + 5 * min(kFew && P.tile_pairs < 16 ? tid & (64 * kFitFewWavefronts - 1) : tid, P.W - 1);
+  const float params[5] = {pr[0], pr[1], pr[2], pr[3], pr[4]};
+  if constexpr (kFew) {  // problems of few waves beside the others
+    if (P.tile_pairs < 16) {
+      // either half of the workgroup takes half of the parts. They pass the same barriers, and a
+      // barrier waits for no wavefront that has ended
+      static_assert(kFitWavefronts == 2 * kFitFewWavefronts && 2 * sizeof(FitFewShared<kFitFewWavefronts>) <= sizeof(sh));
+      const int half = __builtin_amdgcn_readfirstlane(tid / (64 * kFitFewWavefronts)), lower = (unit.parts + 1) >> 1;
+      FitUnit few{unit.problem, unit.strip, unit.part + half * lower, half ? unit.parts - lower : lower};
+      asm volatile("" : "+s"(few.part));  // opaque, so that neither branch's work is hoisted above it
+      if (few.parts == 0) return;
+      fit_few(P, few, params, reinterpret_cast<FitFewShared<kFitFewWavefronts>*>(&sh)[half],
+              tid & (64 * kFitFewWavefronts - 1));
+      return;
+    }
+  }
   float touch_a, touch_b;
   const int tile = P.tiles_per_block * unit.part + min(tid >> 6, P.tiles_per_block * unit.parts - 1);
   touch_targets(P, unit.strip, min(tile, (P.n * P.S - 1) >> 4), tid & 63, touch_a, touch_b);
@@ -700,19 +1009,13 @@ void adjoint_kernel(const FitDesc* __restrict__ probs, const FitUnit* __restrict
   FitWaveLds wv{};
   float bx = 0.0f, by = 0.0f, bz = 0.0f;
   if (tid < P.W) {
-    const double A = p0, L = p1 > 1e-3f ? p1 : 1e-3f, al = p2, Q = p3, ph0 = p4;
-    const double w = kTwoPi / L, om = sqrt(P.g * w);
-    double sa, ca;
-    sincos(al, &sa, &ca);
-    wv.kx = w * ca * kInvTwoPi;
-    wv.kz = w * sa * kInvTwoPi;
-    wv.c0 = __builtin_amdgcn_fract((om * P.t0 + ph0) * kInvTwoPi);
-    wv.om = om * kInvTwoPi;
-    bx = (float)(Q * A * ca);
-    by = (float)A;
-    bz = (float)(Q * A * sa);
-    sh.dir[tid] = make_float2((float)(Q * ca), (float)(Q * sa));
-    sh.grad[tid] = FitWaveGrad{(float)A, (float)Q, (float)ca, (float)sa, (float)w, (float)(w / L), (float)(om / (2.0 * L))};
+    const FitWave w = fit_wave(P, params);
+    wv = w.lds;
+    bx = w.bx;
+    by = w.by;
+    bz = w.bz;
+    sh.dir[tid] = w.dir;
+    sh.grad[tid] = w.grad;
     atomicMax(&sh.max, __float_as_uint(fmaxf(fmaxf(fabsf(bx), fabsf(bz)), fabsf(by))));
   }
   __syncthreads();
@@ -960,8 +1263,14 @@ hipError_t launch_fit_setup_single(const FitDesc& d, FitDesc* d_desc, FitUnit* d
 template <int C>
 hipError_t launch_adjoint_class(const FitLaunch& L, int c, int bump, hipStream_t st) {
   if (c == C) {
-    hipLaunchKernelGGL((adjoint_kernel<kFitClassChunks[C], kFitWavefronts, C == 0>), dim3((unsigned)L.class_blocks[C]),
-                       dim3(64 * kFitWavefronts), 0, st, L.probs, L.units + L.class_begin[C], bump);
+    const dim3 grid((unsigned)L.class_blocks[C]), block(64 * (C == 0 ? kFitFewWavefronts : kFitWavefronts));
+    const FitUnit* units = L.units + L.class_begin[C];
+    if constexpr (C == 0)
+      hipLaunchKernelGGL(adjoint_few_kernel, grid, block, 0, st, L.probs, units, bump);
+    else
+      hipLaunchKernelGGL((C == 1 && L.mixed ? adjoint_kernel<kFitClassChunks[C], kFitWavefronts, C == 1, C == 1>
+                                            : adjoint_kernel<kFitClassChunks[C], kFitWavefronts, C == 1, false>),
+                         grid, block, 0, st, L.probs, units, bump);
     return hipGetLastError();
   }
   if constexpr (C + 1 < kFitClasses) return launch_adjoint_class<C + 1>(L, c, bump, st);

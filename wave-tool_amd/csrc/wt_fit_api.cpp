@@ -158,7 +158,7 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
       return wt::ctx_fail(ctx, WT_ERR_INVALID_ARG, "problem " + std::to_string(i) + ": " + why);
     }
     const wt_fit_problem& p = problems[i];
-    const wt::FitBlocks fb = wt::fit_blocks((int)p.grid_side, (int)p.snapshots);
+    const wt::FitBlocks fb = wt::fit_blocks((int)p.grid_side, (int)p.snapshots, (int)p.wave_count);
     const int nblocks = fb.nblocks;
     const int np = (int)p.wave_count * 5;
     wt::FitDesc& d = f->host[i];
@@ -173,6 +173,7 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
     d.n = (int)p.grid_side;
     d.S = (int)p.snapshots;
     d.W = (int)p.wave_count;
+    d.tile_pairs = fb.tile_pairs;
     d.tiles_per_block = fb.tiles_per_block;
     d.blocks_per_strip = fb.blocks_per_strip;
     d.nblocks = nblocks;
@@ -186,22 +187,38 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
     bytes += sizeof(float) * ((size_t)2 * np + (size_t)(np + 1) * nblocks + 1) + sizeof(int);
     bytes = (bytes + 255) & ~(size_t)255;
   }
-  // adjoint units by wave-count class, the longest first (the dispatcher starts
-  // workgroups in index order). A workgroup takes several parts of a strip where the batch
-  // has many more parts than the GPU has room for workgroups (256 CUs, one or two on
-  // each), so that setting the strip's tables up is paid for by several rounds of tiles.
+  // adjoint units by class, the longest first (the dispatcher starts workgroups in index
+  // order). A workgroup takes several parts of a strip where the batch has many more parts
+  // than the GPU has room for workgroups (256 CUs, one or two on each, four of the
+  // few-waves kernel), so that setting the strip's tables up is paid for by several rounds
+  // of tiles. Problems of few waves beside ones of up to 64 go with these, whose kernel
+  // takes both: a launch more, forked and joined, costs more than they do in any small
+  // batch (24 problems of sides to 64 with 2-16 waves 29 us, so 19).
   const long long unit_rounds = std::min<long long>(16, std::max<long long>(1, rounds / 2048));
+  auto own_class = [&](const wt::FitDesc& d) {
+    return wt::fit_class(wt::FitBlocks{d.tile_pairs, d.tiles_per_block, d.blocks_per_strip, d.nblocks}, d.W);
+  };
+  const bool matrix = std::any_of(f->host.begin(), f->host.end(), [&](const wt::FitDesc& d) { return own_class(d) == 1; });
   std::vector<wt::FitUnit> units;
   long long unit_begin = 0;
   for (int c = 0; c < wt::kFitClasses; ++c) {
     for (uint32_t i = 0; i < count; ++i) {
       const wt::FitDesc& d = f->host[i];
-      if (wt::fit_class(d.W) != c) continue;
-      // parts that run side by side share a workgroup once every CU has one
-      const int side_by = std::max(1, wt::kFitWavefronts / d.tiles_per_block);
-      const int part_rounds = std::max(1, d.tiles_per_block / wt::kFitWavefronts);
-      const int per = unit_rounds > 1 ? (int)std::max<long long>(1, unit_rounds / part_rounds) * side_by
-                                      : (int)std::min<long long>(side_by, std::max<long long>(1, parts / 256));
+      const int own = own_class(d);
+      if ((own == 0 && matrix ? 1 : own) != c) continue;
+      f->launch.mixed |= own != c;
+      int per;
+      if (own == 0) {
+        // beside others two at a time, in a workgroup that has the CU to itself
+        per = (int)(matrix ? 2 * std::min<long long>(8, std::max<long long>(1, parts / 512))
+                           : std::min<long long>(16, (parts + 1023) / 1024));
+      } else {
+        // parts that run side by side share a workgroup once every CU has one
+        const int side_by = std::max(1, wt::kFitWavefronts / d.tiles_per_block);
+        const int part_rounds = std::max(1, d.tiles_per_block / wt::kFitWavefronts);
+        per = unit_rounds > 1 ? (int)std::max<long long>(1, unit_rounds / part_rounds) * side_by
+                              : (int)std::min<long long>(side_by, std::max<long long>(1, parts / 256));
+      }
       const int strips = d.nblocks / d.blocks_per_strip;
       for (int st = 0; st < strips; ++st)
         for (int b = 0; b < d.blocks_per_strip; b += per)
@@ -209,8 +226,10 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
       if (units.size() >= (1ull << 31)) break;
     }
     std::stable_sort(units.begin() + unit_begin, units.end(), [&](const wt::FitUnit& x, const wt::FitUnit& y) {
-      return (long long)x.parts * f->host[x.problem].tiles_per_block >
-             (long long)y.parts * f->host[y.problem].tiles_per_block;
+      auto pairs = [&](const wt::FitUnit& u) {
+        return (long long)u.parts * f->host[u.problem].tiles_per_block * f->host[u.problem].tile_pairs;
+      };
+      return pairs(x) > pairs(y);
     });
     f->launch.class_begin[c] = unit_begin;
     f->launch.class_blocks[c] = (long long)units.size() - unit_begin;
@@ -324,8 +343,8 @@ wt_status wt_fit_loss_grad_static(wt_ctx* ctx, const wt_fit_problem* p, float* d
   if (!ctx || !p || !d_grad) return WT_ERR_INVALID_ARG;
   std::string why;
   if (!problem_ok(*p, &why)) return wt::ctx_fail(ctx, WT_ERR_INVALID_ARG, why);
-  const int cls = wt::fit_class((int)p->wave_count);
-  const wt::FitBlocks fb = wt::fit_blocks((int)p->grid_side, (int)p->snapshots);
+  const wt::FitBlocks fb = wt::fit_blocks((int)p->grid_side, (int)p->snapshots, (int)p->wave_count);
+  const int cls = wt::fit_class(fb, (int)p->wave_count);
   const long long nblocks = fb.nblocks;
   const int np = (int)p->wave_count * 5;
   size_t off_units = 0, off_rows = 0, off_partials = 0;
@@ -360,6 +379,7 @@ wt_status wt_fit_loss_grad_static(wt_ctx* ctx, const wt_fit_problem* p, float* d
   d.n = (int)p->grid_side;
   d.S = (int)p->snapshots;
   d.W = (int)p->wave_count;
+  d.tile_pairs = fb.tile_pairs;
   d.tiles_per_block = fb.tiles_per_block;
   d.blocks_per_strip = fb.blocks_per_strip;
   d.nblocks = (int)nblocks;
