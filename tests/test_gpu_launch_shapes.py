@@ -88,7 +88,7 @@ def test_a_requested_shape_runs(torch_cuda, wtctx, side, lanes):
 @pytest.mark.parametrize("mode", list(MAPS))
 @pytest.mark.parametrize("side,waves,kernel", [(100, 3, "Lb1E"), (256, 65, "Lb1E"), (257, 1, "Lb1E"), (640, 9, "Lb1E"),
                                                (641, 32, "tail"), (700, 66, "tail"), (768, 33, "tail"), (769, 2, "whole"),
-                                               (1024, 3, "whole"), (1025, 7, "tail"), (1281, 2, "whole")])
+                                               (1024, 3, "whole"), (1025, 32, "tail"), (1281, 2, "whole")])
 def test_own_choice_equals_whole_segments(torch_cuda, wtctx, side, waves, kernel, mode):
     """Tangents and bitangents included."""
     torch = torch_cuda
@@ -117,6 +117,22 @@ def test_few_waves_end_rows_in_whole_segments(torch_cuda, wtctx, side, waves, ta
     wtctx.displace(params, w, *out)
     torch.cuda.synchronize()
     name, _ = launched(torch, lambda s: wtctx.displace(params, w, *out, stream=s))
+    assert ("tail_kernel" in name) == tail, name
+
+
+@pytest.mark.parametrize("side,waves,mode,outputs,tail", [
+    (1025, 1, "none", 2, True), (1537, 7, "none", 2, False), (1537, 8, "none", 2, True), (1600, 1, "none", 2, True),
+    (1025, 15, "none", 3, False), (1025, 16, "none", 3, True), (1280, 11, "none", 3, False), (1280, 12, "none", 3, True),
+    (1025, 31, "none", 4, False), (1280, 23, "none", 4, False), (1280, 24, "none", 4, True),
+    (1025, 2, "r32_repeat", 4, True), (2049, 23, "r8_mirror", 4, False), (2049, 24, "r8_mirror", 4, True),
+    (2049, 2, "r32_mirror", 3, True), (2304, 2, "r8_repeat", 4, True)])
+def test_rows_bound_by_their_stores_end_in_whole_segments(torch_cuda, wtctx, side, waves, mode, outputs, tail):
+    torch = torch_cuda
+    params, w, kw = scene(torch, side, waves, mode)
+    out = [torch.empty(3 * side * side, device="cuda") for _ in range(outputs)]
+    wtctx.displace(params, w, *out, **kw)
+    torch.cuda.synchronize()
+    name, _ = launched(torch, lambda s: wtctx.displace(params, w, *out, stream=s, **kw))
     assert ("tail_kernel" in name) == tail, name
 
 

@@ -671,7 +671,9 @@ hipError_t launch_t(const FwdParams& p, bool own, hipStream_t st) {
   }
   if constexpr (K == 8 && S == 2 && LC == 64 && CH == kChunk) {
     const RowCut cut = row_cut(p.N, LaunchShape{S, K, LC, CH});
-    if (own && cut.end_groups > 0 && cut.whole_groups > 0 && (blocks > kOneRoundBlocks || p.W >= kRowEndWaves)) {
+    const int outputs = 2 + (p.ep.tan ? 1 : 0) + (p.ep.bit ? 1 : 0);
+    if (own && cut.end_groups > 0 && cut.whole_groups > 0 &&
+        rows_end_in_halves(blocks, p.N, p.W, kTex != kTexNone, outputs)) {
       hipLaunchKernelGGL((water_forward_tail_kernel<K, LC, kTex>), dim3((unsigned)(cut.whole_groups + cut.end_groups)),
                          dim3(256), 0, st, p, (int)cut.whole_groups);
       return hipGetLastError();

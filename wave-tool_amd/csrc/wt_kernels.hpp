@@ -77,14 +77,27 @@ __host__ __device__ inline void set_corner_algebra(D& d, const double (*c)[4]) {
 constexpr long long kHalvesBlocks = 640;
 
 // Past that, rows that end in the lower half of a segment end in half segments
-// (water_forward_tail_kernel), but up to this many workgroups, four to a CU, only from
-// kRowEndWaves waves on: all of whole segments run at once there, and the sums past the
-// edge, which the halves save, cost them less than the second kind of workgroup. Whole /
-// with halves, us per launch in a graph: 768 x 768 with 1 wave 9.3 / 9.6, 16 waves 10.1 / 10.9,
-// 32 waves 12.6 / 12.5, 64 waves 18.6 / 16.3; 1025 x 1025 (1538 workgroups) with 1 wave
-// 16.3 / 14.9, 16 waves 18.3 / 17.6.
+// (water_forward_tail_kernel), with these exceptions, where the sums past the edge, which
+// the halves save, cost less than what they bring along. Per launch in a graph, with halves
+// over whole:
+// - up to kOneRoundBlocks workgroups, four to a CU, and few waves: all of whole segments run
+//   at once there, and a second kind of workgroup is only more of them. 768 x 768 with 1 wave
+//   9.6 / 9.3 us, 16 waves 10.9 / 10.1, 32 waves 12.5 / 12.6, 64 waves 16.3 / 18.6; 1025 x 1025
+//   (1538 workgroups) with 1 wave 14.9 / 16.3, 16 waves 17.6 / 18.3.
+// - few waves, bound by the stores: a row's end is then stored by another workgroup at
+//   another time. Without a map and 3 or 4 outputs 1.03-1.11 up to 8 and 16 waves; where rows
+//   are no whole 64-byte pieces, so that the two also share one, up to 12 and 24 waves
+//   1.04-1.22 (2 outputs, sides past 1536: 1.00-1.10 up to 4 waves). Beyond these 0.89-0.97.
+//   With a map, whose texels past the edge the halves save too, 0.86-1.03, but 4 outputs at
+//   sides past 2048 in shared pieces 1.02-1.17 from 8 to 16 waves.
 constexpr long long kOneRoundBlocks = 1024;
 constexpr int kRowEndWaves = 32;
+inline bool rows_end_in_halves(long long blocks, int N, int W, bool map, int outputs) {
+  if (blocks <= kOneRoundBlocks && W < kRowEndWaves) return false;
+  const bool pieces = N % 16 == 0;
+  if (map) return pieces || outputs < 4 || N <= 2048 || W >= 24;
+  return W >= 12 * (outputs - 2) && (pieces || W >= (8 << (outputs - 2)) || (outputs == 2 && N <= 1536));
+}
 
 // How the rows of a grid are cut in a shape of two wavefronts per segment: whole segments,
 // and half segments at the rows' ends where the upper halves have no columns. Workgroups
