@@ -108,15 +108,18 @@ def test_own_choice_equals_whole_segments(torch_cuda, wtctx, side, waves, kernel
     assert torch.isfinite(a).all() and torch.equal(a, b)
 
 
-@pytest.mark.parametrize("side,waves,tail", [(641, 31, False), (768, 4, False), (768, 32, True), (1025, 1, True)])
-def test_few_waves_end_rows_in_whole_segments(torch_cuda, wtctx, side, waves, tail):
-    """Where every workgroup of whole segments runs at once, half segments at the rows' ends pay from 32 waves on."""
+@pytest.mark.parametrize("side,waves,mode,tail", [(641, 31, "r32_repeat", False), (768, 4, "r8_mirror", False),
+                                                  (768, 32, "r32_repeat", True), (1025, 1, "r32_repeat", True),
+                                                  (641, 1, "none", True), (768, 31, "none", True)])
+def test_few_waves_end_rows_in_whole_segments(torch_cuda, wtctx, side, waves, mode, tail):
+    """Where every workgroup of whole segments runs at once, half segments at the rows' ends pay from 32 waves on, or
+    without a map."""
     torch = torch_cuda
-    params, w, kw = scene(torch, side, waves)
+    params, w, kw = scene(torch, side, waves, mode)
     out = [torch.empty(3 * side * side, device="cuda") for _ in range(2)]
-    wtctx.displace(params, w, *out)
+    wtctx.displace(params, w, *out, **kw)
     torch.cuda.synchronize()
-    name, _ = launched(torch, lambda s: wtctx.displace(params, w, *out, stream=s))
+    name, _ = launched(torch, lambda s: wtctx.displace(params, w, *out, stream=s, **kw))
     assert ("tail_kernel" in name) == tail, name
 
 

@@ -80,10 +80,11 @@ constexpr long long kHalvesBlocks = 640;
 // (water_forward_tail_kernel), with these exceptions, where the sums past the edge, which
 // the halves save, cost less than what they bring along. Per launch in a graph, with halves
 // over whole:
-// - up to kOneRoundBlocks workgroups, four to a CU, and few waves: all of whole segments run
-//   at once there, and a second kind of workgroup is only more of them. 768 x 768 with 1 wave
-//   9.6 / 9.3 us, 16 waves 10.9 / 10.1, 32 waves 12.5 / 12.6, 64 waves 16.3 / 18.6; 1025 x 1025
-//   (1538 workgroups) with 1 wave 14.9 / 16.3, 16 waves 17.6 / 18.3.
+// - up to kOneRoundBlocks workgroups, four to a CU, a map and few waves: all of whole segments
+//   run at once there, and a second kind of workgroup is only more of them. 768 x 768 with 1
+//   wave 9.6 / 9.3 us, 16 waves 10.9 / 10.1, 32 waves 12.5 / 12.6, 64 waves 16.3 / 18.6 (without
+//   a map 5.9 / 6.3, 8.1 / 8.9 and 10.9 / 11.9: halves); 1025 x 1025 (1538
+//   workgroups) with 1 wave 14.9 / 16.3, 16 waves 17.6 / 18.3.
 // - few waves, bound by the stores: a row's end is then stored by another workgroup at
 //   another time. Without a map and 3 or 4 outputs 1.03-1.11 up to 8 and 16 waves; where rows
 //   are no whole 64-byte pieces, so that the two also share one, up to 12 and 24 waves
@@ -93,7 +94,7 @@ constexpr long long kHalvesBlocks = 640;
 constexpr long long kOneRoundBlocks = 1024;
 constexpr int kRowEndWaves = 32;
 inline bool rows_end_in_halves(long long blocks, int N, int W, bool map, int outputs) {
-  if (blocks <= kOneRoundBlocks && W < kRowEndWaves) return false;
+  if (blocks <= kOneRoundBlocks) return !map || W >= kRowEndWaves;
   const bool pieces = N % 16 == 0;
   if (map) return pieces || outputs < 4 || N <= 2048 || W >= 24;
   return W >= 12 * (outputs - 2) && (pieces || W >= (8 << (outputs - 2)) || (outputs == 2 && N <= 1536));
