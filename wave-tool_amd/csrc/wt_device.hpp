@@ -93,7 +93,8 @@ __host__ __device__ inline int tex_mode(const void* texels, int fmt, int wrap) {
 // issue the texel loads of all its vertices before it needs any of them.
 // heightmap_fetch: (s, t) are texture coordinates already reduced to one wrap period
 // ([0, 1) for REPEAT, [0, 2) for MIRRORED_REPEAT); index arithmetic is clamped so any
-// input stays in bounds. heightmap_eval: value and dH/ds, dH/dt of the same cell.
+// input stays in bounds. heightmap_eval: value and dH/ds, dH/dt of the same cell;
+// heightmap_value: the value alone.
 struct HmTap {
   float t00, t10, t01, t11, a, b;
 };
@@ -132,7 +133,7 @@ template <int M>
 __device__ __forceinline__ HmTap heightmap_fetch(const void* __restrict__ texels, int W, int H, float s, float t) {
   const int period_w = tex_mirror(M) ? 2 * W : W;
   const int period_h = tex_mirror(M) ? 2 * H : H;
-  const float u = s * (float)W - 0.5f, v = t * (float)H - 0.5f;
+  const float u = fmaf(s, (float)W, -0.5f), v = fmaf(t, (float)H, -0.5f);
   const float fu = floorf(u), fv = floorf(v);
   HmTap h;
   h.a = u - fu;
@@ -154,13 +155,31 @@ __device__ __forceinline__ HmTap heightmap_fetch(const void* __restrict__ texels
 
 template <int M>
 __device__ __forceinline__ float heightmap_eval(HmTap h, int W, int H, float* dds, float* ddt) {
+  // value differences along s (of the two rows) and t (of the two columns)
+  float s0 = h.t10 - h.t00, s1 = h.t11 - h.t01, d0 = h.t01 - h.t00, d1 = h.t11 - h.t10;
   if (tex_r8(M)) {  // unorm8: c / 255
+    const float k = 1.0f / 255.0f;
+    const HmTap c = h;
+    h.t00 *= k; h.t10 *= k; h.t01 *= k;
+    s0 = fmaf(c.t10, k, -h.t00);
+    s1 = fmaf(c.t11, k, -h.t01);
+    d0 = fmaf(c.t01, k, -h.t00);
+    d1 = fmaf(c.t11, k, -h.t10);
+  }
+  const float lo = fmaf(h.a, s0, h.t00), hi = fmaf(h.a, s1, h.t01);
+  *dds = (float)W * fmaf(h.b, s1 - s0, s0);
+  *ddt = (float)H * fmaf(h.a, d1 - d0, d0);
+  return fmaf(h.b, hi - lo, lo);
+}
+
+// The value alone.
+template <int M>
+__device__ __forceinline__ float heightmap_value(HmTap h) {
+  if (tex_r8(M)) {
     const float k = 1.0f / 255.0f;
     h.t00 *= k; h.t10 *= k; h.t01 *= k; h.t11 *= k;
   }
   const float lo = fmaf(h.a, h.t10 - h.t00, h.t00), hi = fmaf(h.a, h.t11 - h.t01, h.t01);
-  *dds = (float)W * fmaf(h.b, (h.t11 - h.t01) - (h.t10 - h.t00), h.t10 - h.t00);
-  *ddt = (float)H * fmaf(h.a, (h.t11 - h.t10) - (h.t01 - h.t00), h.t01 - h.t00);
   return fmaf(h.b, hi - lo, lo);
 }
 
@@ -226,17 +245,23 @@ __device__ __forceinline__ RowOut row_out(const EpilogueArgs& e, size_t row_firs
   return RowOut{e.pos + o, e.nrm + o, e.tan ? e.tan + o : nullptr, e.bit ? e.bit + o : nullptr};
 }
 
-// x^2 + y^2 + z^2 and x a + y b + z c as the untextured epilogue forms them: the product
-// of the first or the second pair rounded, the others fused onto it.
+// x a + y b + z c: the product of the first or the second pair rounded, the others fused
+// onto it.
 __device__ __forceinline__ float dot3_from(bool second, float x, float y, float z, float a, float b, float c) {
   const float p = second ? y : x, pa = second ? b : a, q = second ? x : y, qa = second ? a : b;
   return fmaf(z, c, fmaf(q, qa, p * pa));
 }
 
-// lead: the vertex a lane finishes first of a segment. Without a heightmap the sums of
-// three products are written out, which differ by it in the product they start from: left
-// to the compiler, their rounding depends on the number of vertices a lane finishes, and a
-// segment has to give the same bits whole and in halves.
+// x^2 + y^2 + z^2, z^2 rounded before it is added.
+__device__ __forceinline__ float tangent_square(bool first, float x, float y, float z) {
+#pragma clang fp contract(off)
+  return (first ? fmaf(x, x, y * y) : fmaf(y, y, x * x)) + z * z;
+}
+
+// Every sum of products is written out, fused or not: left to the compiler, its rounding
+// could depend on the number of vertices a lane finishes, and a segment has to give the
+// same bits whole and in halves. lead: the vertex a lane finishes first of a segment,
+// without a heightmap; the others' sums of three start from another product there.
 template <int M>
 __device__ __forceinline__ void vertex_finish(const EpilogueArgs& e, const VertexPending& v, const float acc[8],
                                               const RowOut& ro, uint32_t col, bool lead) {
@@ -251,31 +276,21 @@ __device__ __forceinline__ void vertex_finish(const EpilogueArgs& e, const Verte
   if constexpr (M != kTexNone) {
     float dds, ddt;
     const float r = heightmap_eval<M>(v.tap, e.tex_w, e.tex_h, &dds, &ddt);
-    py += e.two_sd * (r - 0.5f);  // water-grid.vert:108-110: s_d * 2 (r - 0.5)
+    py = fmaf(e.two_sd, r - 0.5f, py);  // water-grid.vert:108-110: s_d * 2 (r - 0.5)
     const float k = e.bump_k;
     const float hpx = k * dds, hpz = -k * ddt;  // d(bump)/dPx, d(bump)/dPz
-    ty += hpx * tx + hpz * tz;
-    by += hpx * bx + hpz * bz;
+    ty += fmaf(hpx, tx, hpz * tz);
+    by += fmaf(hpz, bz, hpx * bx);
   }
   py += e.bounce;  // water-grid.vert:147
   // N = normalize(B x T): y-up for the undisplaced plane
-  constexpr bool kFlat = M == kTexNone;
-  float nx, ny, nz;
-  if constexpr (kFlat) {
-    nx = fmaf(by, tz, -(bz * ty));
-    ny = fmaf(bz, tx, -(bx * tz));
-    nz = fmaf(bx, ty, -(by * tx));
-  } else {
-    nx = by * tz - bz * ty;
-    ny = bz * tx - bx * tz;
-    nz = bx * ty - by * tx;
-  }
-  const float inv_n =
-      __builtin_amdgcn_rsqf(kFlat ? dot3_from(!lead, nx, ny, nz, nx, ny, nz) : nx * nx + ny * ny + nz * nz);
+  const bool first = M != kTexNone || lead;
+  float nx = fmaf(by, tz, -(bz * ty)), ny = fmaf(bz, tx, -(bx * tz)), nz = fmaf(bx, ty, -(by * tx));
+  const float inv_n = __builtin_amdgcn_rsqf(dot3_from(!first, nx, ny, nz, nx, ny, nz));
   nx *= inv_n; ny *= inv_n; nz *= inv_n;
   // flip toward the camera (water-grid.vert:190)
   const float vx = e.cam[0] - px, vy = e.cam[1] - py, vz = e.cam[2] - pz;
-  if ((kFlat ? dot3_from(!lead, nx, ny, nz, vx, vy, vz) : nx * vx + ny * vy + nz * vz) < 0.0f) { nx = -nx; ny = -ny; nz = -nz; }
+  if (dot3_from(!first, nx, ny, nz, vx, vy, vz) < 0.0f) { nx = -nx; ny = -ny; nz = -nz; }
   // the outputs are written once per frame and not read back by this kernel: stream
   // them past the caches (4% faster on the 1024^2 x 64-wave frame)
   // byte offset within the row as a 32-bit value (a row is at most 32768 x 12 bytes), so
@@ -285,12 +300,11 @@ __device__ __forceinline__ void vertex_finish(const EpilogueArgs& e, const Verte
   store3_nt(row_at(ro.pos, b), px, py, pz);
   store3_nt(row_at(ro.nrm, b), nx, ny, nz);
   if (ro.tan) {
-    const float it = __builtin_amdgcn_rsqf(kFlat ? __fadd_rn(lead ? fmaf(tx, tx, ty * ty) : fmaf(ty, ty, tx * tx), tz * tz)
-                                                 : tx * tx + ty * ty + tz * tz);
+    const float it = __builtin_amdgcn_rsqf(tangent_square(first, tx, ty, tz));
     store3_nt(row_at(ro.tan, b), tx * it, ty * it, tz * it);
   }
   if (ro.bit) {
-    const float ib = __builtin_amdgcn_rsqf(kFlat ? fmaf(bz, bz, fmaf(by, by, bx * bx)) : bx * bx + by * by + bz * bz);
+    const float ib = __builtin_amdgcn_rsqf(fmaf(bz, bz, fmaf(by, by, bx * bx)));
     store3_nt(row_at(ro.bit, b), bx * ib, by * ib, bz * ib);
   }
 }

@@ -94,8 +94,7 @@ __global__ __launch_bounds__(256) void vertex_varyings_kernel(VaryingArgs a) {
     }
     if constexpr (kTex != kTexNone) {
       if (a.sample) {
-        float dds, ddt;
-        __builtin_nontemporal_store(heightmap_eval<kTex>(tap[r], a.tex_w, a.tex_h, &dds, &ddt), a.sample + v);
+        __builtin_nontemporal_store(heightmap_value<kTex>(tap[r]), a.sample + v);
       }
     }
   }
