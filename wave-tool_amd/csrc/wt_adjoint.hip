@@ -56,6 +56,7 @@
 // alone, so a batch repeats the bits of its problems run one by one.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -1082,16 +1083,18 @@ void adjoint_kernel(const FitDesc* __restrict__ probs, const FitUnit* __restrict
   }
 }
 
+// Block `first` + its own index of the batch's reduce blocks.
 __global__ __launch_bounds__(kReduceThreads) void reduce_adam_kernel(const FitDesc* __restrict__ probs,
-                                                                  const int* __restrict__ reduce_prob, FitAdam adam,
-                                                                  int mode, float* __restrict__ grad_out,
+                                                                  const int* __restrict__ reduce_prob, long long first,
+                                                                  FitAdam adam, int mode, float* __restrict__ grad_out,
                                                                   float* __restrict__ loss_out) {
   constexpr int kSide = kReduceThreads / kReduceRows;  // parts read side by side
   __shared__ double s[kReduceThreads / 64][kReduceRows];
-  const int prob = load_uniform(reduce_prob, (long long)blockIdx.x);
+  const long long block = first + (long long)blockIdx.x;
+  const int prob = load_uniform(reduce_prob, block);
   const FitDesc P = load_uniform(probs, prob);
   const int r = threadIdx.x & (kReduceRows - 1), side = threadIdx.x / kReduceRows;
-  const int row = (int)(blockIdx.x - P.reduce_offset) * kReduceRows + r;
+  const int row = (int)(block - P.reduce_offset) * kReduceRows + r;
   const int nparam = P.W * 5;
   // the row's Adam state, loaded while the partials are summed (a kernel this short is
   // bound by its chain of memory round trips)
@@ -1259,19 +1262,33 @@ hipError_t launch_fit_setup_single(const FitDesc& d, FitDesc* d_desc, FitUnit* d
   return hipGetLastError();
 }
 
-// The adjoint launch of wave-count class c on stream st.
+// Calls launch(first, blocks) for the runs of `blocks` workgroups of `threads` that one launch
+// may have: past 2^32 threads a launch reports no error and leaves workgroups out.
+template <class Launch>
+hipError_t in_launches(long long blocks, int threads, Launch launch) {
+  const long long most = (1ll << 31) / threads;
+  for (long long first = 0; first < blocks; first += most) {
+    launch(first, dim3((unsigned)std::min(most, blocks - first)));
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+// The adjoint launch of class c on stream st.
 template <int C>
 hipError_t launch_adjoint_class(const FitLaunch& L, int c, int bump, hipStream_t st) {
   if (c == C) {
-    const dim3 grid((unsigned)L.class_blocks[C]), block(64 * (C == 0 ? kFitFewWavefronts : kFitWavefronts));
-    const FitUnit* units = L.units + L.class_begin[C];
-    if constexpr (C == 0)
-      hipLaunchKernelGGL(adjoint_few_kernel, grid, block, 0, st, L.probs, units, bump);
-    else
-      hipLaunchKernelGGL((C == 1 && L.mixed ? adjoint_kernel<kFitClassChunks[C], kFitWavefronts, C == 1, C == 1>
-                                            : adjoint_kernel<kFitClassChunks[C], kFitWavefronts, C == 1, false>),
-                         grid, block, 0, st, L.probs, units, bump);
-    return hipGetLastError();
+    const int threads = 64 * (C == 0 ? kFitFewWavefronts : kFitWavefronts);
+    return in_launches(L.class_blocks[C], threads, [&](long long first, dim3 grid) {
+      const FitUnit* units = L.units + L.class_begin[C] + first;
+      if constexpr (C == 0)
+        hipLaunchKernelGGL(adjoint_few_kernel, grid, dim3(threads), 0, st, L.probs, units, bump);
+      else
+        hipLaunchKernelGGL((C == 1 && L.mixed ? adjoint_kernel<kFitClassChunks[C], kFitWavefronts, C == 1, C == 1>
+                                              : adjoint_kernel<kFitClassChunks[C], kFitWavefronts, C == 1, false>),
+                           grid, dim3(threads), 0, st, L.probs, units, bump);
+    });
   }
   if constexpr (C + 1 < kFitClasses) return launch_adjoint_class<C + 1>(L, c, bump, st);
   return hipErrorInvalidValue;
@@ -1309,9 +1326,10 @@ hipError_t launch_fit_iteration(const FitLaunch& L, const FitAdam& adam, int mod
       if ((e = hipStreamWaitEvent(st, L.join[j], 0)) != hipSuccess) return e;
     }
   }
-  hipLaunchKernelGGL(reduce_adam_kernel, dim3((unsigned)L.reduce_blocks), dim3(kReduceThreads), 0, st, L.probs, L.reduce_prob,
-                     adam, mode, grad_out, loss_out);
-  return hipGetLastError();
+  return in_launches(L.reduce_blocks, kReduceThreads, [&](long long first, dim3 grid) {
+    hipLaunchKernelGGL(reduce_adam_kernel, grid, dim3(kReduceThreads), 0, st, L.probs, L.reduce_prob, first, adam, mode,
+                       grad_out, loss_out);
+  });
 }
 
 }  // namespace wt
