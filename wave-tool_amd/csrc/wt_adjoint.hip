@@ -1297,34 +1297,25 @@ hipError_t launch_adjoint_class(const FitLaunch& L, int c, int bump, hipStream_t
 hipError_t launch_fit_iteration(const FitLaunch& L, const FitAdam& adam, int mode, float* grad_out, float* loss_out,
                                 hipStream_t st) {
   const int bump = mode == 1 ? 1 : 0;
-  // classes present, the most work (blocks x waves) first
-  int order[kFitClasses], n = 0;
-  for (int c = 0; c < kFitClasses; ++c)
-    if (L.class_blocks[c] > 0) order[n++] = c;
+  // the class with the most work (blocks x waves), and the other one if there are two
   auto work = [&](int c) { return (double)L.class_blocks[c] * kFitClassChunks[c]; };
-  for (int i = 1; i < n; ++i)
-    for (int j = i; j > 0 && work(order[j]) > work(order[j - 1]); --j) std::swap(order[j], order[j - 1]);
-  if (n <= 1 || !L.side[0]) {
-    for (int i = 0; i < n; ++i) {
-      const hipError_t e = launch_adjoint_class<0>(L, order[i], bump, st);
-      if (e != hipSuccess) return e;
-    }
-  } else {
-    // class i on the caller's stream (i = 0) or side stream (i - 1) mod kFitSideStreams;
-    // the classes write disjoint partials and step counters, so they may overlap
-    hipError_t e = hipEventRecord(L.fork, st);
-    if (e != hipSuccess) return e;
-    const int used = n - 1 < kFitSideStreams ? n - 1 : kFitSideStreams;
-    for (int j = 0; j < used; ++j)
-      if ((e = hipStreamWaitEvent(L.side[j], L.fork, 0)) != hipSuccess) return e;
-    for (int i = 0; i < n; ++i)
-      if ((e = launch_adjoint_class<0>(L, order[i], bump, i == 0 ? st : L.side[(i - 1) % kFitSideStreams])) !=
-          hipSuccess)
-        return e;
-    for (int j = 0; j < used; ++j) {
-      if ((e = hipEventRecord(L.join[j], L.side[j])) != hipSuccess) return e;
-      if ((e = hipStreamWaitEvent(st, L.join[j], 0)) != hipSuccess) return e;
-    }
+  int big = 0, other = -1;
+  for (int c = 1; c < kFitClasses; ++c)
+    if (work(c) > work(big)) big = c;
+  for (int c = 0; c < kFitClasses; ++c)
+    if (c != big && L.class_blocks[c] > 0) other = c;
+  hipError_t e = hipSuccess;
+  if (other >= 0) {
+    // on the side stream: the classes write disjoint partials and step counters, so they
+    // may overlap
+    if ((e = hipEventRecord(L.fork, st)) != hipSuccess) return e;
+    if ((e = hipStreamWaitEvent(L.side, L.fork, 0)) != hipSuccess) return e;
+  }
+  if ((e = launch_adjoint_class<0>(L, big, bump, st)) != hipSuccess) return e;
+  if (other >= 0) {
+    if ((e = launch_adjoint_class<0>(L, other, bump, L.side)) != hipSuccess) return e;
+    if ((e = hipEventRecord(L.join, L.side)) != hipSuccess) return e;
+    if ((e = hipStreamWaitEvent(st, L.join, 0)) != hipSuccess) return e;
   }
   return in_launches(L.reduce_blocks, kReduceThreads, [&](long long first, dim3 grid) {
     hipLaunchKernelGGL(reduce_adam_kernel, grid, dim3(kReduceThreads), 0, st, L.probs, L.reduce_prob, first, adam, mode,

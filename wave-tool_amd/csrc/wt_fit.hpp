@@ -93,13 +93,11 @@ struct FitAdam {
   float lr, beta1, beta2, eps;
 };
 
-// Device tables of a batch: problems, adjoint units (grouped by wave-count class, class c
-// at [class_begin[c], + class_blocks[c])), reduce block -> problem.
-// Streams beside the caller's on which the classes' adjoint launches run
-// concurrently (one class's tail overlaps the next class's blocks), joined by events
-// before the reduction.
-constexpr int kFitSideStreams = 3;
-
+// Device tables of a batch: problems, adjoint units (grouped by class, class c at
+// [class_begin[c], + class_blocks[c])), reduce block -> problem. At most two classes have
+// units: that of up to 64 waves takes the few-waves units too. side: a stream beside the
+// caller's on which the smaller class's launch runs (one's tail overlaps the other's
+// blocks), forked and joined by events before the reduction; null for one class.
 struct FitLaunch {
   const FitDesc* probs;
   const FitUnit* units;
@@ -108,9 +106,8 @@ struct FitLaunch {
   long long class_blocks[kFitClasses];
   long long reduce_blocks;
   bool mixed;  // class 1 holds units of few waves too
-  hipStream_t side[kFitSideStreams];  // null: every class on the caller's stream
-  hipEvent_t fork;
-  hipEvent_t join[kFitSideStreams];
+  hipStream_t side;
+  hipEvent_t fork, join;
 };
 
 // mode 0: gradient + loss only (grad_out receives the concatenated gradients);

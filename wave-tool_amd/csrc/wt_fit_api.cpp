@@ -278,18 +278,16 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
   f->launch.units = f->d_units;
   f->launch.reduce_prob = f->d_rows;
   f->launch.reduce_blocks = f->total_reduce;
-  // side streams (default priority, not synchronising with the null stream) and their
-  // fork / join events, for batches spanning several wave-count classes
+  // the side stream (default priority, not synchronising with the null stream) and its
+  // fork / join events, for batches of two classes
   int classes = 0;
   for (int c = 0; c < wt::kFitClasses; ++c) classes += f->launch.class_blocks[c] > 0;
   if (classes > 1) {
     e = hipEventCreateWithFlags(&f->launch.fork, hipEventDisableTiming);
-    for (int j = 0; j < wt::kFitSideStreams && e == hipSuccess; ++j) {
-      e = hipStreamCreateWithFlags(&f->launch.side[j], hipStreamNonBlocking);
-      if (e == hipSuccess) e = hipEventCreateWithFlags(&f->launch.join[j], hipEventDisableTiming);
-    }
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&f->launch.side, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&f->launch.join, hipEventDisableTiming);
     if (e != hipSuccess) {
-      wt_status s = hip_err(ctx, e, "wt_fit_create streams");
+      wt_status s = hip_err(ctx, e, "wt_fit_create stream");
       wt_fit_destroy(f);
       return s;
     }
@@ -300,10 +298,8 @@ wt_status wt_fit_create(wt_ctx* ctx, const wt_fit_problem* problems, uint32_t co
 
 void wt_fit_destroy(wt_fit* f) {
   if (!f) return;
-  for (int j = 0; j < wt::kFitSideStreams; ++j) {
-    if (f->launch.side[j]) (void)hipStreamDestroy(f->launch.side[j]);
-    if (f->launch.join[j]) (void)hipEventDestroy(f->launch.join[j]);
-  }
+  if (f->launch.side) (void)hipStreamDestroy(f->launch.side);
+  if (f->launch.join) (void)hipEventDestroy(f->launch.join);
   if (f->launch.fork) (void)hipEventDestroy(f->launch.fork);
   if (f->d_desc) (void)hipFree(f->d_desc);
   if (f->d_units) (void)hipFree(f->d_units);
