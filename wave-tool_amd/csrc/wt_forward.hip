@@ -20,13 +20,6 @@ hipError_t launch_forward(const FwdParams& p, const LaunchShape& s, hipStream_t 
   }
 }
 
-long long forward_segment_groups(int N, const LaunchShape& s) {
-  const int LC = s.lanes_per_row, K = s.steps, LR = 64 / LC;
-  const long long segs = (long long)((N + LC * K - 1) / (LC * K)) * ((N + LR - 1) / LR);
-  const int per_wg = kWavesPerWG / s.split;
-  return (segs + per_wg - 1) / per_wg;
-}
-
 int batch_shape_for(int N) {
   // padded vertices per shape (the shapes share K, so the seeds per vertex are equal);
   // the first, widest shape wins ties

@@ -159,9 +159,6 @@ struct VaryingArgs {
 };
 hipError_t launch_varyings(const VaryingArgs& a, hipStream_t st);
 
-// Segments a launch shape covers per workgroup for a grid of side N.
-long long forward_segment_groups(int N, const LaunchShape& s);
-
 // Segment shapes the batched kernel chooses from, per patch (all K = 8, S = 2): 512 x 1
 // for wide grids, 256 x 2 and 128 x 4 for narrower ones.
 constexpr int kBatchShapes = WT_BATCH_SHAPES;
