@@ -16,7 +16,7 @@
 //   backward  G[wave, (j,s)] = sum over offsets of cos(kx delta) x (r+ + r-) and of
 //             sin(kx delta) x (r+ - r-), and the same weighted with the offset, from which
 //             P gives every wave's sums of r cos theta and r sin theta.
-// Folding halves the products of the plain split into 64 columns (fit_batch of 256 uneven
+// Folding halves the products of the plain split into 64 columns (a batch of 256 uneven
 // problems on one MI355X: 1.3 ms an iteration against 1.5 ms).
 // adjoint_kernel: a workgroup takes one strip and a run of (row, snapshot) pairs q = j S + s,
 //   16 consecutive pairs (a tile) per wavefront at a time, so any snapshot count packs the
@@ -31,14 +31,15 @@
 //   (about 2^-22 per product). Powers of two keep both halves in FP16's range: the column
 //   factors are scaled by 2^4, the coefficients by their largest magnitude in the problem,
 //   and the residuals by the largest of the wavefront's tile where that leaves the range.
-//   Against the FP64 adjoint the gradients of 2- to 32-snapshot problems are as close or
-//   closer than with FP32 recurrences over the snapshots (rms of the relative error over 16
-//   problems: 200^2 x 2 x 64 1.1e-7 against 1.1e-7, 128^2 x 16 x 32 1.0e-7 against 8.6e-7).
+//   Against the FP64 adjoint the gradients of 84 drawn problems (sides 32-400, 2-32
+//   snapshots, 4-64 waves) are closer than with FP32 recurrences over the snapshots: rms of
+//   the relative error 7.9e-8 against 1.3e-6, of 65-128 waves 6.4e-8 against 5.5e-7.
 // What bounds it: VALU issue and the matrix cores together, which do not overlap on one
 //   SIMD (two wavefronts of one SIMD, one issuing only matrix instructions and one only
 //   FMAs, take the sum of their times): per tile of 64 waves about 1300 VALU instructions
-//   and 216 matrix instructions of 16 cycles. 512^2 x 16 x 32: 17 us (62 us with FP32
-//   recurrences over the snapshots on the VALU); the 256-problem batch 1.21 ms (3.6 ms).
+//   and 216 matrix instructions of 16 cycles. With the reduction, in a graph: 512^2 x 16 x 32
+//   21.5 us (66 us with FP32 recurrences over the snapshots on the VALU); the 256-problem batch
+//   1.23 ms an iteration (3.67 ms).
 //   Two wavefronts per SIMD at up to 256 VGPRs: a 32-column strip at three or four
 //   wavefronts repeats P, B and the sums per point (1.7 ms), and a spilled register is a
 //   round trip to cold scratch memory (5 us per workgroup).
@@ -322,7 +323,7 @@ __device__ __forceinline__ void load_targets(const FitDesc& P, bool whole, bool 
 // Reads one float of nearly every cache line of a tile's runs of 64 columns (16 runs of
 // 768 bytes, eight reads 108 bytes apart each), which brings them to the L2 ahead of
 // load_targets: issued before the set-up, whose tables need no memory, 512^2 x 16 x 32
-// takes 21.1 us where it took 22.7. For every tile ahead of its time it was slower.
+// takes 21.1 us with its reduction where it took 22.7. For every tile ahead of its time it was slower.
 __device__ __forceinline__ void touch_targets(const FitDesc& P, int strip, int tile, int lane, float& a, float& b) {
   const uint32_t pairs = (uint32_t)P.n * (uint32_t)P.S, q = min((uint32_t)tile * 16u + (uint32_t)(lane & 15), pairs - 1u);
   const uint32_t j = q / (uint32_t)P.S, sn = q - j * (uint32_t)P.S;
