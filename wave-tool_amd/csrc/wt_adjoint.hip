@@ -1086,16 +1086,16 @@ void adjoint_kernel(const FitDesc* __restrict__ probs, const FitUnit* __restrict
 
 // Block `first` + its own index of the batch's reduce blocks.
 __global__ __launch_bounds__(kReduceThreads) void reduce_adam_kernel(const FitDesc* __restrict__ probs,
-                                                                  const int* __restrict__ reduce_prob, long long first,
+                                                                  const int* __restrict__ reduce_prob, int first,
                                                                   FitAdam adam, int mode, float* __restrict__ grad_out,
                                                                   float* __restrict__ loss_out) {
   constexpr int kSide = kReduceThreads / kReduceRows;  // parts read side by side
   __shared__ double s[kReduceThreads / 64][kReduceRows];
-  const long long block = first + (long long)blockIdx.x;
-  const int prob = load_uniform(reduce_prob, block);
+  const int block = first + (int)blockIdx.x;
+  const int prob = load_uniform(reduce_prob, (long long)block);
   const FitDesc P = load_uniform(probs, prob);
   const int r = threadIdx.x & (kReduceRows - 1), side = threadIdx.x / kReduceRows;
-  const int row = (int)(block - P.reduce_offset) * kReduceRows + r;
+  const int row = (block - (int)P.reduce_offset) * kReduceRows + r;
   const int nparam = P.W * 5;
   // the row's Adam state, loaded while the partials are summed (a kernel this short is
   // bound by its chain of memory round trips)
@@ -1319,7 +1319,7 @@ hipError_t launch_fit_iteration(const FitLaunch& L, const FitAdam& adam, int mod
     if ((e = hipStreamWaitEvent(st, L.join, 0)) != hipSuccess) return e;
   }
   return in_launches(L.reduce_blocks, kReduceThreads, [&](long long first, dim3 grid) {
-    hipLaunchKernelGGL(reduce_adam_kernel, grid, dim3(kReduceThreads), 0, st, L.probs, L.reduce_prob, first, adam, mode,
+    hipLaunchKernelGGL(reduce_adam_kernel, grid, dim3(kReduceThreads), 0, st, L.probs, L.reduce_prob, (int)first, adam, mode,
                        grad_out, loss_out);
   });
 }
